@@ -149,6 +149,18 @@ __host__ __device__ inline uint32_t xcd_remap(uint32_t b, uint32_t total, uint32
     return (b % xcds) * per + b / xcds;
 }
 
+// As xcd_remap, in windows of xcds x chunk consecutive indices: each XCD
+// takes runs of `chunk` neighbours, and what is in flight over the whole chip
+// stays one stretch of consecutive indices.
+__host__ __device__ inline uint32_t xcd_chunk_remap(uint32_t b, uint32_t total, uint32_t xcds,
+                                                    uint32_t chunk) {
+    const uint32_t window = xcds * chunk;
+    const uint32_t first = b / window * window;
+    if (xcds <= 1 || total - first < window) return b;  // ragged tail keeps its order
+    const uint32_t r = b - first;
+    return first + (r % xcds) * chunk + r / xcds;
+}
+
 // Division of a dividend below 2^31 by a divisor fixed at launch: q =
 // (n * mul) >> shift with mul = ceil(2^shift / d), shift = 31 + ceil(log2 d).
 // The rounding error of mul stays below 1/d of the quotient's unit for every

@@ -17,11 +17,14 @@
 // Work decomposition.  One lane owns one column; the 64 lanes of the
 // compute wave own 64 consecutive i at fixed j (variants 1 and 2), or 64
 // consecutive columns in i-fastest order that may run on into the next row
-// (variants 3 and 4, vadv_column.h), so a level's field access is one or
+// (variants 3 to 5, vadv_column.h), so a level's field access is one or
 // two contiguous row segments.  The compute wave keeps
 // stage / wcon of the previous level in registers, loads the next PF levels
 // while it computes the current ones, stores (c', d') of levels 0..nz-2 and
 // runs the backward substitution from that storage in the same kernel.
+//
+// The default is variant 5 (vadv_regs.h): one wave per group, the highest
+// levels' (c', d') in registers, the rest in LDS.
 //
 // Storage of (c', d'): variant 1 keeps it in LDS ((nz-1) x 64 x 16 bytes
 // for FP64 arithmetic, so nz <= 160 fits one workgroup); variant 2 keeps it
@@ -38,6 +41,7 @@
 // blocks the compute wave), and after the forward sweep it does the same
 // for the pos lines of the backward substitution.
 #include <algorithm>
+#include <iterator>
 
 #include "vadv_column.h"
 #include "vadv_regs.h"
@@ -375,60 +379,87 @@ __global__ __launch_bounds__(64 * kWsWaves) void vadv_ws_kernel(Components comps
     }
 }
 
-// Variant 5: one wave per 64-column group, (c', d') of the lowest levels in
-// registers and of the rest in LDS (vadv_regs.h); consecutive groups on one
-// XCD.
-template <typename C>
-constexpr int hybrid_nr() { return sizeof(C) == 8 ? 40 : 80; }
-// levels of loads in flight: 8 levels of six loads stay below the 63
-// outstanding vector-memory instructions a wave can count (20 levels measured
-// 8 % slower at 256 x 256 x 80 with float32 storage)
-template <typename T>
-constexpr int hybrid_pf() { return 8; }
+// Variant 5: one wave per 64-column group and component, (c', d') of the
+// highest NR levels in registers and of the rest in LDS (vadv_regs.h).  An
+// item is one component of a group, components innermost: the solves that
+// read the same wcon run side by side, and all of a small domain's at once.
+// A grid of every resident wave walks the items in rounds of consecutive
+// ones, or (SPREAD) every item is a workgroup of its own; either way
+// neighbouring items run on one XCD, whose L2 fetches the cache lines at
+// their edges once.
+constexpr uint32_t kItemsPerXcd = 16;  // 4, 32, 64 and 128 measured 0-4 % slower
 
-template <typename T, typename C, bool NT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
-void vadv_hybrid_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
+template <typename T, typename C, int BUILD, bool NT, bool SPREAD>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(RegBuilds<T, C>::of[BUILD].waves_per_simd)))
+void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
     extern __shared__ unsigned char lds_raw[];
-    constexpr int AUX = NT ? 2 : 0;
     CD<C> *lds = reinterpret_cast<CD<C> *>(lds_raw) + (threadIdx.x & 63);
-    // rounds of gridDim.x consecutive groups, consecutive groups of a round on
-    // one XCD; a grid of every resident wave walks the rounds
-    const int64_t slot = xcd_remap(blockIdx.x, gridDim.x, a.xcds);
-    for (int64_t g = slot; g < a.ngroups; g += gridDim.x) {
-        for (int c = 0; c < a.ncomp; ++c) {
-            const Component &cp = comps.c[c];
-            const Rsrc R{make_rsrc(cp.stage, a.span_bytes), make_rsrc(cp.pos, a.span_bytes),
-                         make_rsrc(cp.tens, a.span_bytes), make_rsrc(cp.tensstage, a.span_bytes),
-                         make_rsrc(wcon, a.span_bytes)};
-            HybridColumn<T, C, hybrid_nr<C>(), hybrid_pf<T>(), AUX>::solve(R, cp.wshift, a, g, lds);
-        }
+    const uint32_t ncomp = uint32_t(a.ncomp), items = uint32_t(a.ngroups) * ncomp;
+    const uint32_t slot = SPREAD ? xcd_chunk_remap(blockIdx.x, gridDim.x, a.xcds, kItemsPerXcd)
+                                 : xcd_remap(blockIdx.x, gridDim.x, a.xcds);
+    for (uint32_t n = slot; n < items; n += gridDim.x) {
+        const uint32_t g = n / ncomp;
+        const Component &cp = comps.c[n - g * ncomp];
+        const Rsrc R{own_rsrc(cp.stage, a.span_bytes), own_rsrc(cp.pos, a.span_bytes),
+                     own_rsrc(cp.tens, a.span_bytes), own_rsrc(cp.tensstage, a.span_bytes),
+                     own_rsrc(wcon, a.span_bytes)};
+        RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0>::solve(R, cp.wshift, a, g,
+                                                                                  lds);
     }
 }
 
-template <typename T, typename C>
-size_t hybrid_lds_bytes(int64_t nz) {
-    return size_t(hybrid_lds_rows(nz, hybrid_nr<C>(), hybrid_pf<T>())) * 64 * sizeof(CD<C>);
-}
+// The build that holds most waves of nz levels on a CU, and how many.
+struct RegShape {
+    int build = 0, per_cu = 0;
+    size_t lds_bytes = 0;
+};
 
 template <typename T, typename C>
-hipError_t launch_hybrid(bool nt, uint64_t groups, size_t lds_bytes, const Components &comps,
-                         const T *wcon, const PipeArgs &pa, Context *ctx) {
+RegShape reg_shape(int64_t nz, size_t lds) {
+    RegShape best;
+    if (nz > reg_max_levels<C>()) return best;
+    int build = 0;
+    for (const RegLevels &levels : RegBuilds<T, C>::of) {
+        const int64_t rows = reg_lds_rows(nz, levels.nr);
+        const size_t bytes = size_t(std::max<int64_t>(rows, 0)) * 64 * sizeof(CD<C>);
+        if (rows >= 1 && bytes <= lds) {
+            const int per_cu = int(std::min<size_t>(4 * levels.waves_per_simd, lds / bytes));
+            if (per_cu > best.per_cu) best = RegShape{build, per_cu, bytes};
+        }
+        ++build;
+    }
+    return best;
+}
+
+template <typename T, typename C, int BUILD, bool NT>
+hipError_t launch_reg_k(const RegShape &shape, uint64_t items, const Components &comps,
+                        const T *wcon, const PipeArgs &pa, Context *ctx) {
+    // float32 fields: one workgroup per item.  The last of a few rounds of
+    // resident waves would be part empty, which costs a wave bound by its own
+    // instructions (512x512x160: 230 -> 216 us, 512x512x80: 113 -> 109 us);
+    // FP64 fields are bound by memory and read it more evenly in rounds
+    // (512x512x80: 202 -> 189 us, 400x400x137: 212 -> 198 us).
+    constexpr bool SPREAD = sizeof(T) == 4;
+    const uint64_t resident = uint64_t(shape.per_cu) * uint64_t(ctx->compute_units);
+    const uint64_t grid = SPREAD ? items : std::min(items, resident);
     PipeArgs args = pa;
-    // one wave per SIMD (its registers), as many per CU as the LDS allows
-    const uint64_t per_cu = lds_bytes ? std::min<uint64_t>(4, ctx->lds_per_block / lds_bytes) : 4;
-    const uint64_t grid = std::min<uint64_t>(groups, std::max<uint64_t>(1, per_cu) * ctx->compute_units);
     args.xcds = grid >= uint64_t(ctx->xcds) ? uint32_t(ctx->xcds) : 1u;
-    const void *fn = nt ? reinterpret_cast<const void *>(&vadv_hybrid_kernel<T, C, true>)
-                        : reinterpret_cast<const void *>(&vadv_hybrid_kernel<T, C, false>);
-    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds_bytes));
-    if (nt)
-        enqueue_kernel((vadv_hybrid_kernel<T, C, true>), dim3(unsigned(grid)), dim3(64),
-                       lds_bytes, ctx->stream, comps, wcon, args);
-    else
-        enqueue_kernel((vadv_hybrid_kernel<T, C, false>), dim3(unsigned(grid)), dim3(64),
-                       lds_bytes, ctx->stream, comps, wcon, args);
+    const void *fn = reinterpret_cast<const void *>(&vadv_reg_kernel<T, C, BUILD, NT, SPREAD>);
+    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(shape.lds_bytes));
+    enqueue_kernel((vadv_reg_kernel<T, C, BUILD, NT, SPREAD>), dim3(unsigned(grid)), dim3(64),
+                   shape.lds_bytes, ctx->stream, comps, wcon, args);
     return hipGetLastError();
+}
+
+template <typename T, typename C, int BUILD = 0>
+hipError_t launch_reg(const RegShape &shape, bool nt, uint64_t items, const Components &comps,
+                      const T *wcon, const PipeArgs &pa, Context *ctx) {
+    if constexpr (BUILD + 1 < int(std::size(RegBuilds<T, C>::of)))
+        if (shape.build != BUILD)
+            return launch_reg<T, C, BUILD + 1>(shape, nt, items, comps, wcon, pa, ctx);
+    return nt ? launch_reg_k<T, C, BUILD, true>(shape, items, comps, wcon, pa, ctx)
+              : launch_reg_k<T, C, BUILD, false>(shape, items, comps, wcon, pa, ctx);
 }
 
 int ensure_scratch(Context *ctx, void **scratch, size_t *have, size_t bytes) {
@@ -567,6 +598,21 @@ hipError_t launch_ws(int block, bool nt, bool fast, int per_cu_limit, uint64_t b
                                        ctx);
 }
 
+// Whether variant 5 loads stage, tens and tensstage (each read once) with the
+// non-temporal hint, which leaves L2 and the Infinity Cache to pos, read a
+// second time by the backward sweep, and to wcon, shared with the neighbour
+// columns (hints on those two as well measured up to 20 % slower than none).
+// FP64 fields: always (512x512x160 437 -> 400 us, 256x256x80 54 -> 47 us).
+// Float32 fields: where rows are whole 128-byte lines, or one component is
+// larger than the Infinity Cache (512x512x160 239 -> 217 us, 400x400x137
+// 129 -> 118 us): elsewhere neighbouring groups share a line that the hint
+// drops too early (301x283x60 30.6 -> 32.5 us, 500x500x40 all components
+// 150 -> 171 us).
+inline bool stream_hint(size_t itemsize, int64_t nx, int ncomp, uint64_t field_bytes) {
+    if (itemsize == 8 || nx % 32 == 0) return true;
+    return ncomp == 1 && 5 * field_bytes > (uint64_t(256) << 20);
+}
+
 // The checked fields and geometry of one call (sb_vadv, sb_vadv_noalloc).
 template <typename T>
 struct VadvCall {
@@ -634,56 +680,29 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
                               (g->nz - 1 + g->hk) * g->sk;
     const bool buffer_ok = g->si > 0 && g->sj > 0 && g->sk > 0 &&
                            uint64_t(last_elem + 1) * sizeof(T) < (uint64_t(1) << 32);
-    const size_t ws_lds = ws_lds_bytes<C>(g->nz);
-    const bool ws_fits = ws_lds <= ctx->lds_per_block;
-    // default: the warp-specialised solver where every workgroup gets at
-    // least two groups and the columns are tall enough: nz >= 96 for FP64
-    // storage (the single-wave pipeline is then held to one group per CU by
-    // LDS), nz >= 48 for float32 storage (measured on MI355X against the
-    // pipeline: 512x512x160 FP64 1.18x, float32 storage 1.9x; 256x256x80
-    // FP64 0.96x, float32 storage 1.20x; float32 storage 512x512x64 1.24x,
-    // 512x512x56 1.21x, 320x320x56 1.19x, 384x384x48 1.09x, 512x512x48
-    // 1.07x, 512x512x40 0.84x)
-    const int ws_min_nz = sizeof(T) == 8 ? 96 : 48;
-    const bool ws_default = ws_fits && buffer_ok &&
-                            uint64_t(last_elem + 1 + g->sk) * sizeof(T) < kWsDropOffset &&
-                            g->nz >= ws_min_nz && groups >= 2 * int64_t(ctx->compute_units);
-    // variant 5 (one wave per group, no pipeline fill or drain) where every
-    // group is in flight at once: at most one wave per SIMD (its registers)
-    // and as many per CU as its LDS allows (measured on MI355X, 256x256x80:
-    // float32 storage 34.6 against 39.6 us, FP64 53.5 against 54.7 us;
-    // with more groups than that, as at 384x384x80, it ran 8-20 % slower)
-    const size_t v5_lds = hybrid_lds_bytes<T, C>(g->nz);
-    const int64_t v5_per_cu =
-        v5_lds ? std::min<int64_t>(4, int64_t(ctx->lds_per_block / v5_lds)) : 4;
-    const bool v5_default = buffer_ok && g->nz <= 96 && v5_per_cu > 0 &&
-                            uint64_t(last_elem + 1 + g->sk) * sizeof(T) < kRegDropOffset &&
-                            groups <= v5_per_cu * int64_t(ctx->compute_units);
-    // beyond the LDS of variants 1, 3 and 4 (nz > 160 with FP64 arithmetic)
-    // variant 5 still holds the column while its LDS part fits (nz <= 201),
-    // ahead of the global scratch (512x512x160 FP64: 765 against 863 us)
-    const bool v5_fits = buffer_ok && v5_lds <= ctx->lds_per_block &&
-                         uint64_t(last_elem + 1 + g->sk) * sizeof(T) < kRegDropOffset;
-    if (variant == 0)
-        variant = v5_default ? 5
-                  : ws_default ? 4
-                  : lds_fits   ? (buffer_ok ? 3 : 1)
-                  : v5_fits    ? 5
-                               : 2;
+    // default: one wave per group with register levels (variant 5) wherever
+    // its columns fit (measured on MI355X against the fastest of the others,
+    // in us: 32x32x80 FP64 14.7 / 16.4, 128x128x80 16.6 / 18.4, 512x512x160
+    // 387 / 421, 512x512x12 36 / 36; float32 storage 512x512x160 216 / 262,
+    // 200x200x137 29 / 55, 301x283x60 all components 68 / 115); fields of
+    // 4 GiB and up or with negative strides take variant 1, taller columns
+    // the global scratch
+    const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block);
+    const uint64_t items = uint64_t(groups) * uint64_t(a.ncomp);
+    if (variant == 0) variant = buffer_ok && reg.per_cu > 0 ? 5 : lds_fits ? 1 : 2;
     SB_REQUIRE(variant >= 1 && variant <= 5, "vadv variant %d not available", variant);
     if (variant == 5) {
-        const size_t hlds = hybrid_lds_bytes<T, C>(g->nz);
-        SB_REQUIRE(hlds <= ctx->lds_per_block,
-                   "nz = %lld needs %zu bytes of LDS per column group, device allows %zu",
-                   (long long)g->nz, hlds, ctx->lds_per_block);
-        SB_REQUIRE(buffer_ok && uint64_t(last_elem + 1 + g->sk) * sizeof(T) < kRegDropOffset,
-                   "vadv variant 5 needs positive strides and fields below 4 GiB");
-        SB_REQUIRE(uint64_t(groups) < (uint64_t(1) << 31), "domain too large for one launch");
+        SB_REQUIRE(reg.per_cu > 0, "vadv variant 5 keeps at most %lld levels in registers and LDS, got nz = %lld",
+                   (long long)reg_max_levels<C>(), (long long)g->nz);
+        SB_REQUIRE(buffer_ok, "vadv variant 5 needs positive strides and fields below 4 GiB");
+        SB_REQUIRE(items < (uint64_t(1) << 31), "domain too large for one launch");
         PipeArgs pa{a.nx, a.ny, a.nz, a.si, a.sj, a.sk, a.ncomp, groups,
                     uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds)};
-        const bool nt = l && l->bz > 0 && (l->bz & 1);
+        const int hint = l ? l->bz : 0;
+        const bool nt = hint ? hint > 0 && (hint & 1)
+                             : stream_hint(sizeof(T), a.nx, a.ncomp, uint64_t(last_elem) * sizeof(T));
         return timed_launch(l, seconds, [&]() -> hipError_t {
-            return launch_hybrid<T, C>(nt, uint64_t(groups), hlds, comps, wcon, pa, ctx);
+            return launch_reg<T, C>(reg, nt, items, comps, wcon, pa, ctx);
         });
     }
     SB_REQUIRE(variant == 2 || variant == 4 || lds_fits,

@@ -1,28 +1,25 @@
 // Variant 5 of the vertical-advection solver: one wave per column group,
-// (c', d') of the lowest levels in registers and of the rest in LDS.
+// (c', d') of the highest levels in registers and of the rest in LDS.
 //
-// Why.  The warp-specialised solver keeps all of (c', d') in LDS and
-// pipelines four role waves over a sequence of column groups; with few groups
-// per workgroup (256 x 256 x 80 gives two per workgroup at two workgroups per
-// CU) its pipeline fill and drain are a third of its steps.  Here one wave
-// solves one 64-column group from its first level to its last and back.  The
-// lowest NR levels of (c', d') live in registers (4 NR 32-bit registers with
-// FP64 arithmetic), the levels above in LDS, so a short column takes a
-// fraction of the LDS a whole column would: at nz = 80 and NR = 40 a wave
-// needs 40 KB, four waves (one per SIMD) share a CU, and every group of a
-// 256 x 256 x 80 domain is in flight at once with no fill or drain.
-//
-// Register indices must be compile-time constants, so the register levels
-// are the lowest ones: the forward sweep runs levels 0 .. NR-1 fully unrolled
-// and then the levels above in blocks of PF through LDS (row k - NR); the
-// backward sweep takes the LDS levels from the top down and then the
-// register levels, again unrolled.  nz is a run-time value: levels at or
-// past nz - 1 run the same instructions on clamped inputs (loads re-read
-// level nz-1; stores go to an out-of-range offset the hardware drops), and
-// the forward state entering level nz - 1 is captured by selects, so no load
-// or store sits under a branch and the compiler can keep the prefetch rings
-// in flight.  The arithmetic is the one documented in vadv.hip, operation by
-// operation (bit-identical to the other variants).
+// Why.  A wave that solves one 64-column group alone has no pipeline to fill
+// or drain and needs no barrier, so a CU can hold as many groups as its
+// registers and LDS have room for: (c', d') of one level are 1 KB of a group
+// with FP64 arithmetic, a CU has 512 KB of registers beside its 160 KB of
+// LDS, and at nz = 80 with NR = 40 register levels four waves (one per SIMD)
+// share a CU.  What bounds such a wave is its own instruction stream: the
+// forward recurrence is one serial chain per column, alone on its SIMD.  So
+// the loop is arranged for few instructions and a short chain:
+//   - the register levels are the highest ones, nz-1-NR .. nz-2, so their
+//     unrolled code always ends at the last level, and the levels below run
+//     in blocks of PF levels after one partial block; no level needs a
+//     select, a clamp or a dropped store;
+//   - what a level does not take from the chain (b, c, d of the row) is
+//     computed one level ahead, beside the division of the current level;
+//   - the terms that repeat from level to level are taken over: a(k) =
+//     -c(k-1), and the two products of corr(k) are -P(k-1) and P(k) with
+//     P(k) = c(k) (stage(k+1) - stage(k)); negation and scaling by a power of
+//     two commute with rounding, so the bits are those of vadv.hip's order;
+//   - the reciprocal of the recurrence is column_recip below.
 #pragma once
 
 #include "vadv_column.h"
@@ -30,184 +27,315 @@
 namespace sb {
 namespace {
 
-constexpr uint32_t kRegDropOffset = 0xFFFFFF00u;  // past any field (< 4 GiB - 256 B)
+// 1 / x, correctly rounded, for the recurrence.  FP64: hardware estimate, two
+// Newton steps and the residual correction of Markstein's scheme, which is
+// the division's own sequence without the operand scaling that only
+// exponents near the ends of the range need; where any lane has such an x
+// (also 0, infinity, NaN: extreme()), the wave divides instead.  The test is
+// two integer instructions beside the chain and a branch that is not taken.
+template <typename C>
+struct Recip {
+    __device__ __forceinline__ static C estimate(C x) { return C(1) / x; }
+    __device__ __forceinline__ static bool extreme(C) { return false; }
+};
+template <>
+struct Recip<double> {
+    __device__ __forceinline__ static double estimate(double x) {
+        double r = __builtin_amdgcn_rcp(x);
+        r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+        r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+        return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    }
+    // |x| outside [2^-500, 2^501)
+    __device__ __forceinline__ static bool extreme(double x) {
+        const uint32_t hi = uint32_t(__builtin_bit_cast(uint64_t, x) >> 32);
+        return (hi << 1) - (523u << 21) >= (1001u << 21);
+    }
+};
 
-// LDS rows (levels NR .. nz-2, rounded up to whole blocks of PF) of one wave.
-__host__ __device__ constexpr int64_t hybrid_lds_rows(int64_t nz, int nr, int pf) {
-    return nz - 1 > nr ? (nz - 1 - nr + pf - 1) / pf * pf : 0;
+// Empty asm that takes and returns its operands: what they are computed from
+// is computed before this point (the compiler would sink a level's
+// right-hand side, which nothing needs before the backward sweep, below
+// hundreds of others and keep every input alive until then).
+template <typename V>
+__device__ __forceinline__ void settle(V &v) {
+    __asm__ volatile("" : "+v"(v));
 }
 
-template <typename T, typename C, int NR, int PF, int AUX>
-struct HybridColumn {
-    static_assert(NR % PF == 0 && NR >= PF, "register levels: whole prefetch blocks");
-    // The forward sweep keeps pos of the lowest NK levels in registers (all
-    // NR register levels with float32 fields; 16 with FP64 fields, which
-    // fill the wave's 512 registers without scratch, where 8, 12 and 20
-    // spilled), so the backward sweep reads pos from memory for the levels
-    // above only.
-    static constexpr int NK = sizeof(T) == 4 ? NR : 16;
+// Levels of loads in flight: 8 levels of six loads stay below the 63
+// outstanding vector-memory instructions a wave can count.
+constexpr int kRegPf = 8;
 
-    // forward state entering a level: stage(k-1), stage(k), wcon and its
-    // neighbour at k, c'(k-1), d'(k-1)
-    struct State {
-        C st_m, st_c, w_c, wn_c, c_prev, d_prev;
+// A field's buffer resource in four scalar registers of its own: resources
+// that share their size and flag words are otherwise put together anew, three
+// scalar moves before most loads.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t own_rsrc(const void *p, uint32_t bytes) {
+    int flags = kRsrcWord3;
+    __asm__ volatile("" : "+s"(bytes), "+s"(flags));
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), short(0), int(bytes), flags);
+}
+
+// Highest columns the variant takes: 201 levels with FP64 arithmetic, 401
+// with float32.
+template <typename C>
+constexpr int64_t reg_max_levels() { return sizeof(C) == 8 ? 201 : 401; }
+
+// Register levels the kernels are built for, and the waves a SIMD holds of
+// each: its registers are 512, and a level takes four (two with float32
+// arithmetic) beside some 80 (FP64 fields) or 55 (float32 fields) of the
+// prefetch ring and the recurrence.
+struct RegLevels {
+    int nr, waves_per_simd;
+};
+template <typename T, typename C>
+struct RegBuilds;
+template <>
+struct RegBuilds<double, double> {
+    static constexpr RegLevels of[] = {{0, 3}, {24, 2}, {40, 2}, {64, 1}, {96, 1}};
+};
+template <>
+struct RegBuilds<float, double> {
+    static constexpr RegLevels of[] = {{0, 4}, {24, 3}, {48, 2}, {80, 1}, {112, 1}};
+};
+template <>
+struct RegBuilds<float, float> {
+    static constexpr RegLevels of[] = {{0, 4}, {40, 3}, {80, 2}};
+};
+
+// LDS rows of one wave: levels 0 .. nz-2-NR.
+__host__ __device__ constexpr int64_t reg_lds_rows(int64_t nz, int nr) { return nz - 1 - nr; }
+
+template <typename T, typename C, int NR, int PF, int AUX>
+struct RegColumn {
+    static_assert(NR == 0 || (NR % PF == 0 && NR >= 2 * PF), "register levels: whole prefetch blocks");
+
+    // Row k of the system, apart from the recurrence, and what row k+1 takes
+    // over from it.
+    struct Row {
+        C b, c, d;  // diagonal, upper off-diagonal and right-hand side
+        C cp;       // c(k-1) = -a(k)
+        C p, st;    // P(k) and stage(k+1)
     };
 
-    __device__ __forceinline__ static State hold(bool at_last, const State &s, const State &h) {
-        return State{at_last ? s.st_m : h.st_m,   at_last ? s.st_c : h.st_c,
-                     at_last ? s.w_c : h.w_c,     at_last ? s.wn_c : h.wn_c,
-                     at_last ? s.c_prev : h.c_prev, at_last ? s.d_prev : h.d_prev};
+    __device__ __forceinline__ static Row row(const Level<T> &r, const Row &q) {
+        const C dtr = C(3.0 / 20.0);
+        const C st_n = C(r.st);
+        const C c = C(0.125) * (C(r.wn) + C(r.w));
+        const C p = c * (st_n - q.st);
+        const C d = ((dtr * C(r.pos) + C(r.tens)) + C(r.ts)) + (-q.p - p);
+        return Row{(dtr + q.c) - c, c, d, q.c, p, st_n};
     }
 
-    // level in [1, nz-2]: c'(k), d'(k) from the level record and the state
-    __device__ __forceinline__ static void middle(const Level<T> &r, State &s, C &c_out, C &d_out) {
-        const C dtr = C(3.0 / 20.0), bet_m = C(0.5), bet_p = C(0.5);
-        const C gav = C(-0.25) * (s.wn_c + s.w_c);
-        const C w_n = C(r.w), wn_n = C(r.wn), st_n = C(r.st);
-        const C gcv = C(0.25) * (wn_n + w_n);
-        const C as = gav * bet_m;
-        const C cs = gcv * bet_m;
-        const C acol = gav * bet_p;
-        C c = gcv * bet_p;
-        const C b = (dtr - acol) - c;
-        const C corr = -as * (s.st_m - s.st_c) - cs * (st_n - s.st_c);
-        C d = ((dtr * C(r.pos) + C(r.tens)) + C(r.ts)) + corr;
-        const C divided = C(1.0) / (b - s.c_prev * acol);
-        c = c * divided;
-        d = (d - s.d_prev * acol) * divided;
-        c_out = c;
-        d_out = d;
-        s = State{s.st_c, st_n, w_n, wn_n, c, d};
+    // c'(k), d'(k) from row k and c'(k-1), d'(k-1); `next` is row k+1, formed
+    // from the ring record `r` beside the division
+    __device__ __forceinline__ static void recur(const Row &q, C &cc, C &dd, const Level<T> &r,
+                                                 Row &next) {
+        const C den = q.b + cc * q.cp;
+        C rr = Recip<C>::estimate(den);
+        C dn = q.d + dd * q.cp;
+        next = row(r, q);
+        settle(rr);
+        settle(dn);
+        settle(next.b);
+        settle(next.d);
+        settle(next.p);
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(Recip<C>::extreme(den)) != 0, 0))
+            rr = C(1) / den;
+        cc = q.c * rr;
+        dd = dn * rr;
+    }
+    __device__ __forceinline__ static void recur(const Row &q, C &cc, C &dd) {
+        const C rr = C(1) / (q.b + cc * q.cp);
+        const C dn = q.d + dd * q.cp;
+        cc = q.c * rr;
+        dd = dn * rr;
     }
 
-    // `lds` is this wave's lane column: row r at lds[64 r].
+    // `lds` is this wave's lane column: level k < nz-1-NR at lds[64 k].
+    // Needs nz >= NR + 2.
     __device__ __forceinline__ static void solve(const Rsrc &R, int64_t wshift, const PipeArgs &a,
                                                  int64_t g, CD<C> *lds) {
-        const int nz = int(a.nz);
-        const int kl = nz - 1;
+        const C dtr = C(3.0 / 20.0);
+        const int nz = int(a.nz), kl = nz - 1;
+        const int low = nz - 2 - NR;            // levels 1 .. low live in LDS beside level 0
+        const int part = low % PF;              // of them in the partial block
         const uint32_t skb = uint32_t(a.sk * int64_t(sizeof(T)));
         const GroupOff F = group_offsets<T>(a, g, wshift);
-        const C dtr = C(3.0 / 20.0), bet_m = C(0.5), bet_p = C(0.5);
-        const uint32_t last = F.row + uint32_t(kl) * skb;  // offset of level nz-1
-        auto off = [&](int k) { return F.row + uint32_t(min(max(k, 0), kl)) * skb; };
-
-        // level record k: pos, tens, tensstage at k; stage, wcon and its
-        // neighbour at k + 1 (clamped to nz - 1)
-        auto load = [&](int k, Level<T> &r) {
-            const uint32_t so = off(k), sn = off(k + 1);
+        auto at = [&](int k) { return F.row + uint32_t(k) * skb; };
+        // pos, tens, tensstage at byte offset `so`; stage, wcon and its
+        // neighbour one level above
+        auto load = [&](uint32_t so, Level<T> &r) {
+            const uint32_t sn = so + skb;
             r.pos = bload<T, 0>(R.pos, F.lane, so);
             r.tens = bload<T, AUX>(R.tens, F.lane, so);
             r.ts = bload<T, AUX>(R.ts, F.lane, so);
             r.st = bload<T, AUX>(R.stage, F.lane, sn);
-            r.w = bload<T, AUX>(R.w, F.lane, sn);
-            r.wn = bload<T, AUX>(R.w, F.lane_wn, sn);
+            r.w = bload<T, 0>(R.w, F.lane, sn);
+            r.wn = bload<T, 0>(R.w, F.lane_wn, sn);
+        };
+        // a level's offset, kept running: formed anew at each level, so that
+        // no level's offset stays live from the forward to the backward sweep
+        auto step_up = [&](uint32_t &so) {
+            so += skb;
+            __asm__ volatile("" : "+s"(so));
+        };
+        auto step_down = [&](uint32_t &so) {
+            so -= skb;
+            __asm__ volatile("" : "+s"(so));
         };
 
-        // the last level's own inputs, issued first
-        const T last_pos = bload<T, 0>(R.pos, F.lane, last);
-        const T last_tens = bload<T, AUX>(R.tens, F.lane, last);
-        const T last_ts = bload<T, AUX>(R.ts, F.lane, last);
-        const T st0 = bload<T, AUX>(R.stage, F.lane, F.row);
-        Level<T> ring[PF];
+        // ---- first loads: level 0, then the ring ------------------------------
+        Level<T> first, ring[PF];
+        const T st0 = bload<T, AUX>(R.stage, F.lane, at(0));
+        load(at(0), first);
+        // slot p starts as level 1 + p of the partial block; slots past it take
+        // their level of the first whole block at once
+        const int top = max(kl - 1, 0);
 #pragma unroll
-        for (int p = 0; p < PF; ++p) load(p, ring[p]);
+        for (int p = 0; p < PF; ++p) load(at(min(1 + p + (p < part ? 0 : part), top)), ring[p]);
+        T last_pos, last_tens, last_ts;
+        auto load_last = [&] {
+            last_pos = bload<T, 0>(R.pos, F.lane, at(kl));
+            last_tens = bload<T, AUX>(R.tens, F.lane, at(kl));
+            last_ts = bload<T, AUX>(R.ts, F.lane, at(kl));
+        };
+        if constexpr (NR == 0) load_last();
 
-        C cc[NR], dd[NR];
-        T pk[NK];  // pos of the lowest NK levels
-        State s{}, h{};
-        // ---- level 0 ---------------------------------------------------------
+        // ---- level 0 ----------------------------------------------------------
+        C cc, dd;
+        Row q;
         {
-            const Level<T> r = ring[0];
-            pk[0] = r.pos;
-            load(PF, ring[0]);
-            const C gcv = C(0.25) * (C(r.wn) + C(r.w));
-            const C cs = gcv * bet_m;
-            const C c = gcv * bet_p;
+            const C st_n = C(first.st);
+            const C c = C(0.125) * (C(first.wn) + C(first.w));
+            const C p = c * (st_n - C(st0));
+            const C d = ((dtr * C(first.pos) + C(first.tens)) + C(first.ts)) - p;
             const C b = dtr - c;
-            const C corr = -cs * (C(r.st) - C(st0));
-            const C d = ((dtr * C(r.pos) + C(r.tens)) + C(r.ts)) + corr;
-            cc[0] = c / b;
-            dd[0] = d / b;
-            s = State{C(st0), C(r.st), C(r.w), C(r.wn), cc[0], dd[0]};
+            cc = c / b;
+            dd = d / b;
+            lds[0] = CD<C>{cc, dd};
+            q = Row{b, c, d, C(0), p, st_n};
         }
-        // ---- levels 1 .. NR-1: registers ---------------------------------------
+        // ---- partial block: levels 1 .. part ----------------------------------
 #pragma unroll
-        for (int k = 1; k < NR; ++k) {
-            h = hold(k == kl, s, h);
-            const Level<T> r = ring[k % PF];
-            if (k < NK) pk[k] = r.pos;
-            load(k + PF, ring[k % PF]);
-            middle(r, s, cc[k], dd[k]);
+        for (int p = 0; p < PF - 1; ++p) {
+            if (p < part) {
+                q = row(ring[p], q);
+                recur(q, cc, dd);
+                lds[int64_t(1 + p) * 64] = CD<C>{cc, dd};
+            }
         }
-        // ---- levels NR .. nz-2: LDS row k - NR, in blocks of PF -----------------
-        const int rows = int(hybrid_lds_rows(nz, NR, PF));
-        for (int kb = NR; kb < NR + rows; kb += PF) {
+        if (part) {
+#pragma unroll
+            for (int p = 0; p < PF - 1; ++p)
+                if (p < part) load(at(min(1 + p + part, top)), ring[p]);
+        }
+        // ---- whole blocks in LDS: levels 1 + part .. low -----------------------
+        Row done = q;  // the last row that has entered the chain
+        q = row(ring[0], q);
+        int k = 1 + part;
+        uint32_t so = at(k + PF - 1);  // offset of the last level loaded
+        for (; k <= low; k += PF) {
+            CD<C> *out = lds + int64_t(k) * 64;
 #pragma unroll
             for (int p = 0; p < PF; ++p) {
-                const int k = kb + p;
-                h = hold(k == kl, s, h);
-                const Level<T> r = ring[p];
-                load(k + PF, ring[p]);
-                C c, d;
-                middle(r, s, c, d);
-                lds[int64_t(k - NR) * 64] = CD<C>{c, d};
+                Row n;
+                recur(q, cc, dd, ring[(p + 1) % PF], n);
+                step_up(so);
+                load(NR >= PF ? so : min(so, at(top)), ring[p]);
+                out[p * 64] = CD<C>{cc, dd};
+                done = q;
+                q = n;
             }
         }
-        h = hold(NR + rows == kl, s, h);  // nz - 1 = NR + rows exactly
-
-        // ---- level nz-1 from the held state ------------------------------------
-        C x;
-        {
-            const C gav = C(-0.25) * (h.wn_c + h.w_c);
-            const C as = gav * bet_m;
-            const C acol = gav * bet_p;
-            const C b = dtr - acol;
-            const C corr = -as * (h.st_m - h.st_c);
-            const C d = ((dtr * C(last_pos) + C(last_tens)) + C(last_ts)) + corr;
-            x = (d - h.d_prev * acol) / (b - h.c_prev * acol);
-        }
-        bstore<T>(R.ts, F.lane, last, T(dtr * (x - C(last_pos))));
-
-        // ---- backward: LDS levels from the top, then the register levels ------
-        // slot p of the pos ring holds the level of in-block position p
-        T pr[PF];
-        // a level below NK is kept in pk, so its load is dropped (an
-        // out-of-range offset reads nothing and returns 0)
-        auto pos_load = [&](int k) {
-            const bool kept = k < NK;
-            return bload<T, 0>(R.pos, kept ? kRegDropOffset : F.lane, kept ? 0u : off(k));
-        };
+        // ---- register levels: low + 1 .. nz-2 ----------------------------------
+        C rc[NR > 0 ? NR : 1], rd[NR > 0 ? NR : 1];
+        T pr[PF];  // pos of the levels below, for the backward sweep
 #pragma unroll
-        for (int p = 0; p < PF; ++p) pr[p] = pos_load(NR + rows - PF + p);
-        for (int kb = NR + rows - PF; kb >= NR; kb -= PF) {
+        for (int i = 0; i < NR; ++i) {
+            if (i + 1 < NR) {
+                Row n;
+                recur(q, cc, dd, ring[(i + 1) % PF], n);
+                done = q;
+                q = n;
+            } else {
+                recur(q, cc, dd);
+                done = q;
+            }
+            settle(cc);
+            settle(dd);
+            rc[i] = cc;
+            rd[i] = dd;
+            if (i + PF < NR) {
+                step_up(so);
+                load(so, ring[i % PF]);
+            } else if (i + PF == NR) {
+                load_last();
+            }
+        }
+        // ---- level nz-1 ---------------------------------------------------------
+        uint32_t sp = at(kl - 1 - PF);  // offset of the last pos level loaded, plus one
+        if constexpr (NR >= PF) {
 #pragma unroll
             for (int p = PF - 1; p >= 0; --p) {
-                const int k = kb + p;
-                const T pos = pr[p];
-                pr[p] = pos_load(k - PF);
-                const bool live = k < kl;
-                const CD<C> cd = lds[int64_t(k - NR) * 64];
-                const C xn = cd.d - cd.c * x;
-                x = live ? xn : x;
-                bstore<T>(R.ts, live ? F.lane : kRegDropOffset, live ? off(k) : 0u,
-                          T(dtr * (x - C(pos))));
+                pr[p] = bload<T, 0>(R.pos, F.lane, sp);
+                step_down(sp);
             }
         }
+        C x;
+        {
+            const C b = dtr + done.c;
+            const C d = ((dtr * C(last_pos) + C(last_tens)) + C(last_ts)) - done.p;
+            x = (d + dd * done.c) / (b + cc * done.c);
+        }
+        uint32_t st = at(kl);
+        bstore<T>(R.ts, F.lane, st, T(dtr * (x - C(last_pos))));
+
+        // ---- backward: register levels ------------------------------------------
 #pragma unroll
-        for (int k = NR - 1; k >= 0; --k) {
-            const int p = k % PF;
+        for (int i = NR - 1; i >= 0; --i) {
             T pos;
-            if (k < NK) {
-                pos = pk[k];
+            if (i + PF >= NR) {
+                pos = ring[i % PF].pos;  // still there from the forward sweep
             } else {
-                pos = pr[p];
-                pr[p] = pos_load(k - PF);
+                pos = pr[i % PF];
+                pr[i % PF] = bload<T, 0>(R.pos, F.lane, i >= PF ? sp : at(max(low + 1 + i - PF, 0)));
+                if (i >= PF) step_down(sp);
             }
-            const bool live = k < kl;
-            const C xn = dd[k] - cc[k] * x;
-            x = live ? xn : x;
-            bstore<T>(R.ts, live ? F.lane : kRegDropOffset, live ? off(k) : 0u,
-                      T(dtr * (x - C(pos))));
+            step_down(st);
+            x = rd[i] - rc[i] * x;
+            bstore<T>(R.ts, F.lane, st, T(dtr * (x - C(pos))));
+        }
+        // ---- backward: whole blocks in LDS --------------------------------------
+        T pp[PF];  // pos of the partial block's levels and of level 0
+#pragma unroll
+        for (int p = 0; p < PF; ++p) pp[p] = bload<T, 0>(R.pos, F.lane, at(min(p, part)));
+        if constexpr (NR == 0) {
+#pragma unroll
+            for (int p = 0; p < PF; ++p)
+                pr[p] = bload<T, 0>(R.pos, F.lane, at(max(low - PF + 1 + p, 0)));
+        }
+        for (k = low - PF + 1; k > part; k -= PF) {
+            const CD<C> *in = lds + int64_t(k) * 64;
+            CD<C> cd[PF];
+#pragma unroll
+            for (int p = PF - 1; p >= 0; --p) cd[p] = in[p * 64];
+#pragma unroll
+            for (int p = PF - 1; p >= 0; --p) {
+                const T pos = pr[p];
+                pr[p] = bload<T, 0>(R.pos, F.lane, at(max(k + p - PF, 0)));
+                step_down(st);
+                x = cd[p].d - cd[p].c * x;
+                bstore<T>(R.ts, F.lane, st, T(dtr * (x - C(pos))));
+            }
+        }
+        // ---- backward: levels part .. 0 ------------------------------------------
+#pragma unroll
+        for (int p = PF - 1; p >= 0; --p) {
+            if (p <= part) {
+                const CD<C> cd = lds[int64_t(p) * 64];
+                x = cd.d - cd.c * x;
+                bstore<T>(R.ts, F.lane, at(p), T(dtr * (x - C(pp[p]))));
+            }
         }
     }
 };

@@ -406,6 +406,38 @@ def test_vadv_one_wave_register_columns_several_rounds(gpu, prec, domain):
     assert np.array_equal(got[inner(domain, halo)], expected)
 
 
+# nz at the edges of the register builds (0, 24, 40, 48, 64, 80, 96 and 112
+# levels, and two levels beside them) and of their blocks of 8 levels, with
+# every component an item of its own
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("nz", [9, 10, 11, 25, 26, 27, 35, 43, 50, 51, 66, 67, 83, 99, 114, 115,
+                                137])
+def test_vadv_register_builds(gpu, prec, nz):
+    domain, halo = (45, 7, nz), (1, 1, 0)
+    fields = make_fields(domain, halo, _dtype(prec), count=16, seed=nz)
+    got = _run_vadv(gpu, fields, [3, 7, 11], domain, halo, _prec(gpu, prec), True, 0)
+    expected = _vadv_expected(fields, domain, halo, prec, ("u", "v", "w"))
+    for g, e in zip(got, expected):
+        assert np.array_equal(g[inner(domain, halo)], e)
+
+
+# pivots at zero and past both ends of the exponent range that the recurrence's
+# reciprocal covers without a division: the register solver gives what the
+# solver that divides at every level gives, infinities and NaN included
+@pytest.mark.parametrize("scale", [2.0**-1070, 2.0**-600, 2.0**499, 2.0**502, 2.0**600, 1e308])
+@pytest.mark.parametrize("nz", [12, 60])
+def test_vadv_register_columns_extreme_pivots(gpu, scale, nz):
+    domain, halo = (70, 3, nz), (1, 0, 0)
+    fields = make_fields(domain, halo, np.float64, count=8, seed=2)
+    wcon = fields[4]
+    rng = np.random.default_rng(4)
+    wcon[...] = rng.choice([0.0, scale, -scale, 0.6, 1.2, -0.6, np.inf, np.nan, 0.3], wcon.shape,
+                           p=[.2, .2, .1, .15, .1, .1, .01, .01, .13])
+    got = [_run_vadv(gpu, [f.copy() for f in fields], [3], domain, halo, gpu.SB_F64, False,
+                     variant)[0][inner(domain, halo)] for variant in (5, 1)]
+    assert np.array_equal(got[0], got[1], equal_nan=True)
+
+
 def test_vadv_one_wave_rejects_columns_beyond_lds(gpu):
     from stencil_benchmarks_amd.benchmark import ExecutionError
 
