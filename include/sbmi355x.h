@@ -264,8 +264,10 @@ int sb_stream_check(int prec, const void *x, size_t n, double expected,
  * positive strides, every field below 4 GiB, nz small enough that a 64-column
  * Thomas buffer fits in LDS (nz <= 160 with FP64 arithmetic).
  * Launch options: hdiff_launch->by / ->bz / ->unroll = tile height / planes
- * per item / non-temporal flags (as sb_hdiff); vadv_launch->variant = 4
- * (default: warp-specialised solver, items of ->by column groups, 0 = 16,
+ * per item / non-temporal flags (as sb_hdiff); vadv_launch all zero = the
+ * register-column solver of sb_vadv's variant 5, one launch per register
+ * build the columns need; ->variant = 4 (also 0 with any option of it:
+ * warp-specialised solver, items of ->by column groups, 0 = 16,
  * drawn from per-XCD device work queues in order of decreasing cost, ->unroll
  * = levels per barrier step 4 or 8, 0 = 4, ->bx = waves per workgroup 4 or
  * 5, 0 = 4, the fifth loading wcon for the others) or 3
@@ -282,10 +284,10 @@ typedef struct sb_subdomain {
 } sb_subdomain;
 
 /* One timestep for `count` subdomains: a counter reset, one persistent hdiff
- * launch (tiles from per-XCD device work queues) and one or two persistent
- * vadv launches (warp-specialised: column-group items from per-XCD device
- * work queues, one launch per LDS class; variant 3: items from one device
- * counter).  Does not flip the parities; the caller does. */
+ * launch (tiles from per-XCD device work queues) and the vadv launches (by
+ * default one to five, a workgroup per column group; warp-specialised: one or
+ * two persistent ones, column-group items from per-XCD device work queues,
+ * one launch per LDS class; variant 3: items from one device counter).  Does not flip the parities; the caller does. */
 int sb_batch_step(int prec, const sb_subdomain *subs, int count, const sb_launch *hdiff_launch,
                   const sb_launch *vadv_launch, double *seconds);
 /* A fixed set of subdomains advanced `steps` steps per run: device tables

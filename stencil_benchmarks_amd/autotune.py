@@ -6,17 +6,18 @@ tools/multirun.py); here the sweep is a tuner that times candidate launch
 options on the device and keeps the fastest per device and workload:
 
 * batched steps (`tune_batch`): hdiff tile height, k-planes per item and
-  cache hints, then the vadv solver (warp-specialised with 8/16/32 column
-  groups per item, 4 or 8 levels per barrier step and 4 or 5 waves, or the
-  single-wave pipeline at prefetch depth 4/8),
+  cache hints, then the vadv solver (register columns, warp-specialised with
+  8/16/32 column groups per item, 4 or 8 levels per barrier step and 4 or 5
+  waves, or the single-wave pipeline at prefetch depth 4/8),
   chosen by coordinate descent (hdiff with the default vadv, then vadv with
   the chosen hdiff), each candidate timed over whole steps on scratch
   subdomains of the workload's geometry (user fields are never advanced);
 * plain horizontal diffusion (`tune_hdiff`): tile height x k-planes x cache
   hints over one domain;
 * plain vertical advection (`tune_vadv`): the warp-specialised solver at 4 or
-  8 levels per barrier step or the single-wave pipeline at prefetch depth
-  4/8/16, each with plain or non-temporal streamed loads, over one domain.
+  8 levels per barrier step, the single-wave pipeline at prefetch depth
+  4/8/16 or register columns, each with plain or non-temporal streamed loads,
+  over one domain.
 
 Every candidate computes the same arithmetic (the tests check that results
 are bit-identical across launch options), so tuning changes speed only.
@@ -45,10 +46,11 @@ BATCH_HDIFF_SPACE = (
     {"by": 16, "bz": 2}, {"by": 16, "bz": 2, "unroll": 4}, {"by": 32, "bz": 2},
     {"by": 16, "bz": 1}, {"by": 8, "bz": 1},
 )
-# vadv options of the batched step (variant 4: ->by column groups per item,
+# vadv options of the batched step (none: register columns; variant 4: ->by column groups per item,
 # ->unroll levels per barrier step, ->bx waves per workgroup; variant 3:
 # ->unroll prefetch depth)
 BATCH_VADV_SPACE = (
+    {},
     {"variant": 4, "by": 16}, {"variant": 4, "by": 8}, {"variant": 4, "by": 32},
     {"variant": 4, "by": 16, "unroll": 8}, {"variant": 4, "by": 8, "unroll": 8},
     {"variant": 4, "by": 32, "unroll": 8},
@@ -68,7 +70,8 @@ PLAIN_HDIFF_SPACE = tuple({"variant": 1, "by": by, "bz": bz, "unroll": u}
 PLAIN_VADV_SPACE = tuple({"variant": v, "unroll": u, "bz": bz}
                          for v, depths in ((4, (4, 8)), (3, (4, 8, 16)))
                          for u in depths for bz in (1, -1)) + (
-    {"variant": 5, "unroll": 0, "bz": -1}, {"variant": 5, "unroll": 0, "bz": 1},
+    {"variant": 5, "unroll": 0, "bz": 0}, {"variant": 5, "unroll": 0, "bz": -1},
+    {"variant": 5, "unroll": 0, "bz": 1},
     {"variant": 2, "unroll": 8, "bz": 1})
 
 

@@ -24,7 +24,7 @@
 //     halo rows and row-edge cache lines once; with one queue for the chip
 //     they ran on any XCD (measured on MI355X, 96-subdomain batch: reads
 //     1.38x / 1.63x the algorithmic bytes in FP64 / float32 storage);
-//   vadv items:  (subdomain, residue r): the 64-column groups r, r + m,
+//   vadv items of variant 4:  (subdomain, residue r): the 64-column groups r, r + m,
 //     r + 2m, ... of one subdomain, where m (the subdomain's item count) is
 //     at most the number of resident workgroups, solved by the
 //     warp-specialised column solver of the plain kernel (vadv_ws.h; the
@@ -48,6 +48,14 @@
 // the start of every sequence (no memset nodes, so the sequence can be
 // captured in a hipGraph and replayed).  Every workgroup exits once the
 // counters pass their item counts.
+//
+// By default vadv runs the register-column solver (vadv_regs.h) instead, one
+// workgroup per column group and one launch per register build that the
+// columns need (vadv_reg_batch_kernel).  Measured on MI355X against the
+// warp-specialised launches, whole steps with the hdiff launch: 32 subdomains
+// of 32..512 squared x 40..160, float32 storage 2.63 -> 2.07 ms, FP64 4.39 ->
+// 3.84 ms; 6 subdomains of 32..200 squared x 40..120 399 -> 84 us, FP64 471 ->
+// 90 us.
 #include <algorithm>
 #include <cstring>
 #include <memory>
@@ -58,6 +66,7 @@
 
 #include "hdiff_tile.h"
 #include "vadv_column.h"
+#include "vadv_regs.h"
 #include "vadv_ws.h"
 
 namespace sb {
@@ -85,6 +94,10 @@ constexpr int kCountersPerStep = (kPipeCounter + 1) * kCounterStride;
 // batch, 8 and 64 slower).
 constexpr int kWsGroupsPerItem = 16;
 
+// The register-column solver among the vadv variants (it has no options, so a
+// launch names it by giving none)
+constexpr int kRegVariant = 5;
+
 // One scheduled item of the warp-specialised vadv: subdomain rank, residue.
 struct VItem {
     int32_t rank, residue;
@@ -102,6 +115,9 @@ struct SubDev {
     int32_t tiles_i, tiles_j;
     uint32_t span_bytes;
     int32_t vstride;  // vadv items of this subdomain = group stride
+    int64_t row;      // lanes of a row of columns (register-column vadv)
+    int32_t aligned;  // groups are whole aligned chunks (vadv_regs.h)
+    int32_t reserved;
     // division by tiles_i * tiles_j and by tiles_i (hdiff item decode)
     UDiv hdiv_tiles, hdiv_tiles_i;
 };
@@ -232,7 +248,7 @@ void vadv_batch_kernel(const SubDev *__restrict__ subs, const int64_t *__restric
         const int64_t m = d.vstride;
         const int64_t g0 = item - prefix[s];
         const int64_t n = (groups - g0 + m - 1) / m;  // groups g0, g0 + m, ...
-        const PipeArgs a{d.nx, d.ny, d.nz, d.si, d.sj, d.sk, 1, groups, d.span_bytes, 0};
+        const PipeArgs a{d.nx, d.ny, d.nz, d.si, d.sj, d.sk, 1, groups, d.span_bytes, 0, d.nx};
         const Rsrc R{make_rsrc(d.out, d.span_bytes), make_rsrc(d.pos, d.span_bytes),
                      make_rsrc(d.tens, d.span_bytes), make_rsrc(d.ts, d.span_bytes),
                      make_rsrc(d.wcon, d.span_bytes)};
@@ -288,13 +304,46 @@ __global__ __launch_bounds__(64 * NW) void vadv_ws_batch_kernel(
             const int64_t m = d.vstride;
             const int64_t res = int64_t(__builtin_amdgcn_readfirstlane(it.residue));
             const PipeArgs a{d.nx, d.ny, d.nz, d.si, d.sj, d.sk, 1, groups, d.span_bytes,
-                             uint32_t(queues)};
+                             uint32_t(queues), d.nx};
             const WsFields f{d.out, d.pos, d.tens, d.ts, d.wcon, d.span_bytes};
             // u component: wcon neighbour at i+1
             WsSolver<T, C, 0, FAST, MB, NW>::run(f, d.si, a, WsSeq{res, m, (groups - res + m - 1) / m},
                                                  lane0, lane0 + ws_rows(d.nz, MB) * 64);
         }
     }
+}
+
+// Default vadv of a step: the column solver of the plain kernel's variant 5
+// (vadv_regs.h) over the 64-column groups of the subdomains of one class
+// (those of one register build), one wave and one workgroup per group.  A
+// workgroup finds its subdomain by a search of the class's prefix sums and
+// leaves the balance to the dispatcher, so the step needs no queue and no
+// cost model, and neighbouring groups run on one XCD.
+template <typename T, typename C, int BUILD, bool NT>
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(RegBuilds<T, C>::of[BUILD].waves_per_simd)))
+void vadv_reg_batch_kernel(const SubDev *__restrict__ subs, const int32_t *__restrict__ ranks,
+                           const int32_t *__restrict__ prefix, int count, uint32_t xcds) {
+    extern __shared__ unsigned char lds_raw[];
+    CD<C> *lds = reinterpret_cast<CD<C> *>(lds_raw) + (threadIdx.x & 63);
+    const int32_t item =
+        int32_t(xcd_chunk_remap(blockIdx.x, gridDim.x, xcds, kRegItemsPerXcd));
+    int lo = 0, hi = count;  // largest c with prefix[c] <= item
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (prefix[mid] <= item)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    const SubDev d = subs[ranks[lo]];
+    const PipeArgs a{d.nx, d.ny, d.nz, d.si, d.sj, d.sk, 1, 0, d.span_bytes, 0, d.row};
+    const Rsrc R{own_rsrc(d.out, d.span_bytes), own_rsrc(d.pos, d.span_bytes),
+                 own_rsrc(d.tens, d.span_bytes), own_rsrc(d.ts, d.span_bytes),
+                 own_rsrc(d.wcon, d.span_bytes)};
+    // u component: wcon neighbour at i+1
+    RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0>::solve(
+        R, d.si, a, item - prefix[lo], lds);
 }
 
 // ---- host side ---------------------------------------------------------------
@@ -321,6 +370,17 @@ struct Plan {
         std::vector<VItem> host_list;
     } ws[2];
     std::vector<int8_t> host_vclass;  // LDS class of each subdomain (by rank)
+    // register-column vadv (the default): one launch per class
+    struct RegClass {
+        int build = 0;
+        size_t lds_bytes = 0;           // of its tallest column
+        int64_t aligned_groups = 0;     // of subdomains whose groups are aligned chunks
+        std::vector<int32_t> host;      // ranks, then prefix sums of their groups
+        int32_t *dev = nullptr;
+        int count() const { return int(host.size() / 2); }
+        int32_t items() const { return host.back(); }
+    };
+    std::vector<RegClass> reg;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     // host copies
@@ -342,11 +402,16 @@ int hdiff_kc(const sb_launch *l, int) {
     return (l && l->bz) ? l->bz : 8;
 }
 int hdiff_flags(const sb_launch *l) { return l && l->unroll ? (l->unroll & 3) : 2; }
-// vadv launch options: variant 4 (default) warp-specialised solver, 3 the
+// vadv solvers: without options the register-column solver, variant 4 the
+// warp-specialised solver, 3 the
 // single-wave pipeline (unroll = prefetch depth 4 or 8, bz > 0 non-temporal
 // streamed loads); for variant 4, bz bit 2 selects the fast reciprocal
 // (float32 storage with FP64 arithmetic only)
-int vadv_variant(const sb_launch *l) { return (l && l->variant) ? l->variant : 4; }
+int vadv_variant(const sb_launch *l) {
+    if (l && l->variant) return l->variant;
+    // options of the warp-specialised solver without a variant select it
+    return l && (l->bx || l->by || l->bz || l->unroll) ? 4 : kRegVariant;
+}
 // groups per item of the warp-specialised solver (launch->by, 0 = default)
 int vadv_ws_per_item(const sb_launch *l) { return (l && l->by > 0) ? l->by : kWsGroupsPerItem; }
 // levels per barrier step of the warp-specialised solver (launch->unroll:
@@ -393,7 +458,7 @@ size_t vadv_lds_bytes(int max_nz) {
 
 // LDS per workgroup of the batched vadv (`block`: levels per step of variant 4)
 size_t plan_vadv_lds(int prec, int max_nz, int variant, int block) {
-    if (variant == 4)
+    if (variant != 3)
         return prec == SB_F32 ? ws_lds_bytes<float>(max_nz, block)
                               : ws_lds_bytes<double>(max_nz, block);
     return prec == SB_F32 ? vadv_lds_bytes<float>(max_nz) : vadv_lds_bytes<double>(max_nz);
@@ -455,6 +520,47 @@ void schedule_ws(Plan &p, int cls, int workers, int queues) {
     }
 }
 
+RegShape batch_reg_shape(int prec, int64_t nz, const Context *ctx) {
+    if (prec == SB_F64) return reg_shape<double, double>(nz, ctx->lds_per_block);
+    if (prec == SB_F32) return reg_shape<float, float>(nz, ctx->lds_per_block);
+    return reg_shape<float, double>(nz, ctx->lds_per_block);
+}
+
+// Classes of the register-column vadv, tallest columns first, the subdomains
+// of each in order of decreasing height (the last workgroups to start are the
+// short ones).
+void build_reg_classes(Plan &p, const Context *ctx) {
+    p.reg.clear();
+    const std::vector<SubDev> &subs = p.host_subs[0];
+    std::vector<int32_t> ranks(subs.size());
+    std::iota(ranks.begin(), ranks.end(), 0);
+    std::stable_sort(ranks.begin(), ranks.end(),
+                     [&](int32_t a, int32_t b) { return subs[a].nz > subs[b].nz; });
+    std::vector<int32_t> prefix;
+    auto close = [&] {
+        if (p.reg.empty()) return;
+        std::vector<int32_t> &host = p.reg.back().host;
+        host.push_back(0);  // as many prefix sums as ranks, and the total
+        host.insert(host.end(), prefix.begin(), prefix.end());
+        prefix.clear();
+    };
+    for (int32_t r : ranks) {
+        const RegShape shape = batch_reg_shape(p.prec, subs[r].nz, ctx);
+        if (p.reg.empty() || p.reg.back().build != shape.build) {
+            close();
+            p.reg.emplace_back();
+            p.reg.back().build = shape.build;
+        }
+        Plan::RegClass &c = p.reg.back();
+        c.lds_bytes = std::max(c.lds_bytes, shape.lds_bytes);
+        c.host.push_back(r);
+        const int32_t groups = int32_t(vadv_groups(subs[r].row, subs[r].ny));
+        prefix.push_back((prefix.empty() ? 0 : prefix.back()) + groups);
+        if (subs[r].aligned) c.aligned_groups += groups;
+    }
+    close();
+}
+
 // Build descriptors and prefix sums (largest subdomains first).
 void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch *hl, Plan &p,
                   const Context *ctx) {
@@ -471,6 +577,7 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
     for (int i = 0; i < count; ++i) p.max_nz = std::max<int>(p.max_nz, int(subs[i].geom.nz));
     const int64_t workers = vadv_workers(p, ctx);
     const bool ws = vadv_variant(&p.vl) == 4;
+    p.reg.clear();
     const int64_t per_item = ws ? vadv_ws_per_item(&p.vl) : kMinGroupsPerItem;
     // warp-specialised solver: columns whose slot buffer fits twice in a
     // CU's LDS (class 0) run in their own launch at two workgroups per CU,
@@ -528,6 +635,12 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
             d.hdiv_tiles_i = make_udiv(uint32_t(d.tiles_i));
             d.span_bytes = uint32_t(uint64_t(last + 1) * esize);
             d.vstride = int32_t(vitems);
+            const ColumnRow row =
+                padded_row(g.nx, g.si, g.sj, esize,
+                           std::initializer_list<const void *>{s.u[0], s.u[1], s.upos, s.utens,
+                                                               s.utensstage, s.wcon});
+            d.row = row.lanes;
+            d.aligned = row.aligned;
             p.host_subs[flip][r] = d;
         }
         const int64_t hitems = tiles_i * ((g.ny + ty - 1) / ty) * ((g.nz + kc - 1) / kc);
@@ -538,6 +651,26 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
         for (int c = 0; c < 2; ++c)
             if (p.ws[c].max_nz)
                 schedule_ws(p, c, p.ws[c].per_cu * ctx->compute_units, vadv_queues(ctx));
+    if (vadv_variant(&p.vl) == kRegVariant) build_reg_classes(p, ctx);
+}
+
+// The vadv launch of one class.
+template <typename T, typename C, int BUILD = 0>
+hipError_t enqueue_reg_class(const Plan::RegClass &c, const SubDev *subs, Context *ctx) {
+    if constexpr (BUILD + 1 < int(std::size(RegBuilds<T, C>::of)))
+        if (c.build != BUILD) return enqueue_reg_class<T, C, BUILD + 1>(c, subs, ctx);
+    // non-temporal loads as in the plain kernel (stream_hint in vadv.hip), for
+    // float32 fields where most groups are aligned chunks
+    const bool stream = sizeof(T) == 8 || 2 * c.aligned_groups > int64_t(c.items());
+    const auto kernel = stream ? vadv_reg_batch_kernel<T, C, BUILD, true>
+                               : vadv_reg_batch_kernel<T, C, BUILD, false>;
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, int(c.lds_bytes));
+    const uint32_t items = uint32_t(c.items());
+    const uint32_t xcds = items >= uint32_t(ctx->xcds) ? uint32_t(ctx->xcds) : 1u;
+    hipLaunchKernelGGL(kernel, dim3(items), dim3(64), c.lds_bytes, ctx->stream, subs, c.dev,
+                       c.dev + c.count(), c.count(), xcds);
+    return hipGetLastError();
 }
 
 // Enqueue one step (both kernels) on ctx->stream.
@@ -568,6 +701,13 @@ hipError_t enqueue_step(const Plan &p, int flip, unsigned long long *counters, C
 #undef SB_HB
     if (return_h != hipSuccess) return return_h;
     // vadv
+    if (vadv_variant(&p.vl) == kRegVariant) {
+        for (const Plan::RegClass &c : p.reg) {
+            const hipError_t e = enqueue_reg_class<T, C>(c, subs, ctx);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     const unsigned vgrid = vadv_workers(p, ctx);
     if (vadv_variant(&p.vl) == 4) {
         // one launch per LDS class, taller columns first
@@ -646,6 +786,7 @@ int upload_tables(Plan &p, Context *ctx) {
     for (const Plan::WsClass &c : p.ws)
         ws_bytes += ((sizeof(int32_t) * c.host_off.size() + 7) & ~size_t(7)) +
                     sizeof(VItem) * c.host_list.size();
+    for (const Plan::RegClass &c : p.reg) ws_bytes += sizeof(int32_t) * c.host.size();
     const size_t need = sched + ws_bytes + 256;
     if (p.dev_bytes < need) {
         // steps enqueued earlier may still read the old tables
@@ -696,6 +837,11 @@ int upload_tables(Plan &p, Context *ctx) {
         if (list_bytes) std::memcpy(host + at, c.host_list.data(), list_bytes);
         at += list_bytes;
     }
+    for (Plan::RegClass &c : p.reg) {
+        c.dev = reinterpret_cast<int32_t *>(base + at);
+        std::memcpy(host + at, c.host.data(), sizeof(int32_t) * c.host.size());
+        at += sizeof(int32_t) * c.host.size();
+    }
     // one copy, ordered on the stream before the steps that read the tables
     // (and after the previous steps, which read the same device tables)
     SB_HIP(hipMemcpyAsync(p.dev, host, at, hipMemcpyHostToDevice, ctx->stream));
@@ -710,7 +856,8 @@ int sync_stream(Context *ctx) {
 
 int check_lds(const Plan &p, Context *ctx) {
     const int variant = vadv_variant(&p.vl);
-    SB_REQUIRE(variant == 3 || variant == 4, "batched vadv variant %d not available", variant);
+    SB_REQUIRE(p.vl.variant == 0 || variant == 3 || variant == 4,
+               "batched vadv variant %d not available", variant);
     SB_REQUIRE(!vadv_fast(&p.vl) || (variant == 4 && p.prec == SB_F32_F64),
                "the fast reciprocal needs variant 4 and float32 storage with FP64 arithmetic");
     SB_REQUIRE(variant != 4 || vadv_ws_block_ok(&p.vl),

@@ -41,7 +41,6 @@
 // blocks the compute wave), and after the forward sweep it does the same
 // for the pos lines of the backward substitution.
 #include <algorithm>
-#include <iterator>
 
 #include "vadv_column.h"
 #include "vadv_regs.h"
@@ -387,8 +386,6 @@ __global__ __launch_bounds__(64 * kWsWaves) void vadv_ws_kernel(Components comps
 // ones, or (SPREAD) every item is a workgroup of its own; either way
 // neighbouring items run on one XCD, whose L2 fetches the cache lines at
 // their edges once.
-constexpr uint32_t kItemsPerXcd = 16;  // 4, 32, 64 and 128 measured 0-4 % slower
-
 template <typename T, typename C, int BUILD, bool NT, bool SPREAD>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(RegBuilds<T, C>::of[BUILD].waves_per_simd)))
@@ -396,7 +393,7 @@ void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
     extern __shared__ unsigned char lds_raw[];
     CD<C> *lds = reinterpret_cast<CD<C> *>(lds_raw) + (threadIdx.x & 63);
     const uint32_t ncomp = uint32_t(a.ncomp), items = uint32_t(a.ngroups) * ncomp;
-    const uint32_t slot = SPREAD ? xcd_chunk_remap(blockIdx.x, gridDim.x, a.xcds, kItemsPerXcd)
+    const uint32_t slot = SPREAD ? xcd_chunk_remap(blockIdx.x, gridDim.x, a.xcds, kRegItemsPerXcd)
                                  : xcd_remap(blockIdx.x, gridDim.x, a.xcds);
     for (uint32_t n = slot; n < items; n += gridDim.x) {
         const uint32_t g = n / ncomp;
@@ -407,29 +404,6 @@ void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
         RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0>::solve(R, cp.wshift, a, g,
                                                                                   lds);
     }
-}
-
-// The build that holds most waves of nz levels on a CU, and how many.
-struct RegShape {
-    int build = 0, per_cu = 0;
-    size_t lds_bytes = 0;
-};
-
-template <typename T, typename C>
-RegShape reg_shape(int64_t nz, size_t lds) {
-    RegShape best;
-    if (nz > reg_max_levels<C>()) return best;
-    int build = 0;
-    for (const RegLevels &levels : RegBuilds<T, C>::of) {
-        const int64_t rows = reg_lds_rows(nz, levels.nr);
-        const size_t bytes = size_t(std::max<int64_t>(rows, 0)) * 64 * sizeof(CD<C>);
-        if (rows >= 1 && bytes <= lds) {
-            const int per_cu = int(std::min<size_t>(4 * levels.waves_per_simd, lds / bytes));
-            if (per_cu > best.per_cu) best = RegShape{build, per_cu, bytes};
-        }
-        ++build;
-    }
-    return best;
 }
 
 template <typename T, typename C, int BUILD, bool NT>
@@ -603,15 +577,24 @@ hipError_t launch_ws(int block, bool nt, bool fast, int per_cu_limit, uint64_t b
 // second time by the backward sweep, and to wcon, shared with the neighbour
 // columns (hints on those two as well measured up to 20 % slower than none).
 // FP64 fields: always (512x512x160 437 -> 400 us, 256x256x80 54 -> 47 us).
-// Float32 fields: where rows are whole 128-byte lines, or one component is
-// larger than the Infinity Cache (512x512x160 239 -> 217 us, 400x400x137
-// 129 -> 118 us): elsewhere neighbouring groups share a line that the hint
-// drops too early (301x283x60 30.6 -> 32.5 us, 500x500x40 all components
-// 150 -> 171 us).
-inline bool stream_hint(size_t itemsize, int64_t nx, int ncomp, uint64_t field_bytes) {
-    if (itemsize == 8 || nx % 32 == 0) return true;
+// Float32 fields: where groups are whole chunks of aligned rows, or one
+// component is larger than the Infinity Cache (512x512x160 239 -> 217 us,
+// 313x327x100 59 -> 49 us): elsewhere neighbouring groups share a line that
+// the hint drops too early (301x283x60 without row padding 30.6 -> 32.5 us,
+// 500x500x40 all components 150 -> 171 us).
+inline bool stream_hint(size_t itemsize, bool aligned, int ncomp, uint64_t field_bytes) {
+    if (itemsize == 8 || aligned) return true;
     return ncomp == 1 && 5 * field_bytes > (uint64_t(256) << 20);
 }
+
+// The fields that a call reads and writes, in argument order.
+struct FieldList {
+    void *const *f;
+    int n;
+    void *const *begin() const { return f; }
+    void *const *end() const { return f + n; }
+};
+inline FieldList fields_of(void *const *f, int ncomp) { return {f, 4 * ncomp + 1}; }
 
 // The checked fields and geometry of one call (sb_vadv, sb_vadv_noalloc).
 template <typename T>
@@ -688,7 +671,9 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
     // 4 GiB and up or with negative strides take variant 1, taller columns
     // the global scratch
     const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block);
-    const uint64_t items = uint64_t(groups) * uint64_t(a.ncomp);
+    const ColumnRow row = padded_row(g->nx, g->si, g->sj, sizeof(T), fields_of(f, a.ncomp));
+    const int64_t reg_groups = vadv_groups(row.lanes, g->ny);
+    const uint64_t items = uint64_t(reg_groups) * uint64_t(a.ncomp);
     if (variant == 0) variant = buffer_ok && reg.per_cu > 0 ? 5 : lds_fits ? 1 : 2;
     SB_REQUIRE(variant >= 1 && variant <= 5, "vadv variant %d not available", variant);
     if (variant == 5) {
@@ -696,11 +681,11 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
                    (long long)reg_max_levels<C>(), (long long)g->nz);
         SB_REQUIRE(buffer_ok, "vadv variant 5 needs positive strides and fields below 4 GiB");
         SB_REQUIRE(items < (uint64_t(1) << 31), "domain too large for one launch");
-        PipeArgs pa{a.nx, a.ny, a.nz, a.si, a.sj, a.sk, a.ncomp, groups,
-                    uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds)};
+        PipeArgs pa{a.nx, a.ny, a.nz, a.si, a.sj, a.sk, a.ncomp, reg_groups,
+                    uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds), row.lanes};
         const int hint = l ? l->bz : 0;
         const bool nt = hint ? hint > 0 && (hint & 1)
-                             : stream_hint(sizeof(T), a.nx, a.ncomp, uint64_t(last_elem) * sizeof(T));
+                             : stream_hint(sizeof(T), row.aligned, a.ncomp, uint64_t(last_elem) * sizeof(T));
         return timed_launch(l, seconds, [&]() -> hipError_t {
             return launch_reg<T, C>(reg, nt, items, comps, wcon, pa, ctx);
         });
@@ -749,7 +734,7 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
         SB_REQUIRE(buffer_ok && uint64_t(last_elem + 1 + g->sk) * sizeof(T) < kWsDropOffset,
                    "warp-specialised vadv needs positive strides and fields below 4 GiB");
         PipeArgs pa{a.nx, a.ny, a.nz, a.si, a.sj, a.sk, a.ncomp, groups,
-                    uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds)};
+                    uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds), a.nx};
         const int per_cu_limit = l ? l->bx : 0;
         return timed_launch(l, seconds, [&]() -> hipError_t {
             return launch_ws<T, C>(ws_block, flags & 1, fast_div, per_cu_limit, uint64_t(groups),
@@ -765,7 +750,7 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
         SB_REQUIRE(g->si > 0 && g->sj > 0 && g->sk > 0 && span < (uint64_t(1) << 32),
                    "pipelined vadv needs positive strides and fields below 4 GiB");
         PipeArgs pa{a.nx, a.ny, a.nz, a.si, a.sj, a.sk, a.ncomp, groups, uint32_t(span),
-                    uint32_t(ctx->xcds)};
+                    uint32_t(ctx->xcds), a.nx};
         // persistent grid: launch->bx workgroups per CU (0: as many as LDS allows)
         const int fit = int(size_t(ctx->lds_per_block) / (lds_bytes + kStaticLds));
         const int per_cu = (l && l->bx > 0) ? min(l->bx, max(fit, 1)) : max(fit, 1);

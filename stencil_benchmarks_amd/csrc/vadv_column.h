@@ -69,6 +69,7 @@ struct PipeArgs {
     int64_t ngroups;  // column groups: ceil(nx * ny / 64)
     uint32_t span_bytes;  // addressable bytes from each field's interior origin
     uint32_t xcds;        // XCDs of the device: consecutive groups share one XCD's L2
+    int64_t row;          // lanes a row of columns takes: nx, or more (padded_row)
 };
 
 // Buffer-resource addressing: every field is one descriptor based at its
@@ -122,25 +123,25 @@ struct GroupOff {
     uint32_t lane, lane_wn, row;
 };
 
-// Number of column groups of an nx x ny domain.
-__host__ __device__ constexpr int64_t vadv_groups(int64_t nx, int64_t ny) {
-    return (nx * ny + 63) / 64;
+// Number of column groups of ny rows of `row` lanes (row = nx: no padding).
+__host__ __device__ constexpr int64_t vadv_groups(int64_t row, int64_t ny) {
+    return (row * ny + 63) / 64;
 }
 
-// Group g holds columns 64 g .. 64 g + 63 of the domain's nx * ny columns in
-// i-fastest order: a group runs on into the next row where nx is not a
-// multiple of 64, so only the domain's last group can have idle lanes.
-// Idle lanes duplicate the last column: same inputs, same outputs, so their
-// (identical) stores are harmless.  Column indices fit 32 bits (every field
-// is below 4 GiB).
+// Group g holds lanes 64 g .. 64 g + 63 of the domain's a.row * ny lanes in
+// i-fastest order: a group runs on into the next row where a row is not a
+// multiple of 64 lanes.  Lanes past nx of their row, and past the last row,
+// duplicate the last column before them: same inputs, same outputs, so their
+// (identical) stores are harmless.  Lane indices fit 32 bits (every field is
+// below 4 GiB).
 template <typename T>
 __device__ __forceinline__ GroupOff group_offsets(const PipeArgs &a, int64_t g, int64_t wshift) {
-    const uint32_t nx = uint32_t(a.nx), cols = uint32_t(a.nx * a.ny);
+    const uint32_t row = uint32_t(a.row), cols = uint32_t(a.row * a.ny);
     const uint32_t first = min(uint32_t(g) * 64u, cols - 1);
-    const uint32_t j0 = first / nx;  // uniform: the group's first row
+    const uint32_t j0 = first / row;  // uniform: the group's first row
     uint32_t col = first + (threadIdx.x & 63);
     col = col < cols ? col : cols - 1;
-    const uint32_t j = col / nx, i = col - j * nx;
+    const uint32_t j = col / row, i = min(col - j * row, uint32_t(a.nx) - 1u);
     const int64_t e = int64_t(i) * a.si + int64_t(j - j0) * a.sj;
     GroupOff o;
     o.lane = uint32_t(e * int64_t(sizeof(T)));

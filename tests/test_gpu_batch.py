@@ -94,6 +94,35 @@ def test_batch_steps_match_oracle(gpu, prec, variant, unroll, domains):
     _check(subs, hosts, dtype)
 
 
+# the default vadv: columns of every register build in one batch (a launch per
+# build), rows with and without lane padding
+@pytest.mark.parametrize("prec", ["f64", "f32_f64", "f32"])
+def test_batch_register_classes(gpu, prec):
+    from stencil_benchmarks_amd import batch
+
+    dtype = np.float64 if prec == "f64" else np.float32
+    domains = [(3, 70, 160), (70, 37, 9), (33, 20, 30), (61, 16, 60), (130, 5, 100), (40, 9, 137),
+               (100, 3, 43), (65, 4, 82)]
+    subs, hosts = _make_batch(dtype, seed=6, domains=domains)
+    compute = np.float32 if prec == "f32" else np.float64
+    for _ in range(2):
+        batch.step(subs, compute=compute)
+    if prec == "f32":  # against the warp-specialised solver: float32 arithmetic has no oracle step
+        from stencil_benchmarks_amd import native
+        twins, _ = _make_batch(dtype, seed=6, domains=domains)
+        for _ in range(2):
+            batch.step(twins, compute=compute, vadv_options=native.launch_options(variant=4))
+        for sub, twin in zip(subs, twins):
+            sl = inner(sub.domain, sub.halo)
+            assert np.array_equal(sub.state()[sl], twin.state()[sl])
+            assert np.array_equal(sub.download("utensstage")[sl], twin.download("utensstage")[sl])
+        return
+    for _ in range(2):
+        for sub, hf in zip(subs, hosts):
+            oracle_step(hf, sub.domain, sub.halo, dtype)
+    _check(subs, hosts, dtype)
+
+
 def test_batch_plan_graph_replays_match_eager(gpu):
     from stencil_benchmarks_amd import batch
 

@@ -421,6 +421,26 @@ def test_vadv_register_builds(gpu, prec, nz):
         assert np.array_equal(g[inner(domain, halo)], e)
 
 
+# rows padded to whole 128- or 64-byte chunks of lanes (vadv_regs.h): the
+# lanes past a row's end repeat its last column; 64-byte aligned fields with
+# odd and even multiples of 64 bytes as row pitch, one of unaligned rows
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("domain,alignment", [((100, 7, 26), 64), ((60, 11, 27), 128),
+                                              ((61, 3, 12), 64), ((127, 4, 50), 512),
+                                              ((119, 5, 42), 64), ((119, 5, 42), 8)])
+def test_vadv_padded_rows(gpu, prec, domain, alignment):
+    halo = (3, 3, 3)
+    fields = make_fields(domain, halo, _dtype(prec), count=16, seed=sum(domain),
+                         alignment=alignment)
+    got = _run_vadv(gpu, fields, [3, 7, 11], domain, halo, _prec(gpu, prec), True, 0)
+    expected = _vadv_expected(fields, domain, halo, prec, ("u", "v", "w"))
+    for w, (g, e) in zip((3, 7, 11), zip(got, expected)):
+        assert np.array_equal(g[inner(domain, halo)], e)
+        outside = np.ones(g.shape, bool)
+        outside[inner(domain, halo)] = False
+        assert np.array_equal(g[outside], fields[w][outside])
+
+
 # pivots at zero and past both ends of the exponent range that the recurrence's
 # reciprocal covers without a division: the register solver gives what the
 # solver that divides at every level gives, infinities and NaN included
