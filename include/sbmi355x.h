@@ -162,11 +162,11 @@ int sb_laplacian(int prec, int along_x, int along_y, int along_z,
  * Replaces kernel(double*, inp, coeff, out) of the hdiff variants
  * (stencils/cuda_hip/horizontal_diffusion.py:50-128 and
  * templates/horizontal_diffusion_*.j2); semantics of base.py:276-311.
- * Requires hi, hj >= 2.  Variants: 0 default (2 for SB_F64 domains of
- * whole 64 x 8 tiles and float32 domains of whole 64 x 16 tiles when no
- * tile option is given, else 1 where positive i
- * and j strides and a k-plane below 4 GiB let the tile use 32-bit plane
- * offsets, else 3), 1 LDS-staged tile
+ * Requires hi, hj >= 2.  Variants: 0 default (the kernel of 2, also on
+ * partial tiles and any alignment, where si = 1, 0 < sj with a row pitch
+ * below 16 MiB, a k-plane is below 4 GiB and no tile option is given; else 1
+ * where positive i and j strides and a k-plane below 4 GiB let the tile use
+ * 32-bit plane offsets, else 3), 1 LDS-staged tile
  * (launch->by = tile rows 8/16/32, ->bz = k-planes per workgroup 1..16, 0
  * measured default; ->unroll 0 = default (non-temporal coeff loads), else
  * 4 | flags with bit 0 non-temporal out stores, bit 1 non-temporal coeff

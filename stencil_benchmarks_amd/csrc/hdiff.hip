@@ -7,7 +7,7 @@
 //   fly(i,j) = lap(i,j+1) - lap(i,j), set to 0 if fly * (in(i,j+1) - in(i,j)) > 0
 //   out      = in - coeff * (((flx(i,j) - flx(i-1,j)) + fly(i,j)) - fly(i,j-1))
 //
-// Variant 1 (LDS tile, default).  A workgroup of 64 x (TY/RPT) threads owns
+// Variant 1 (LDS tile).  A workgroup of 64 x (TY/RPT) threads owns
 // a 64 x TY output tile of one k-plane.  It stages the (64+4) x (TY+4) input
 // tile (2-point halo on every side) in LDS with coalesced loads, each
 // thread then walks RPT consecutive rows of one column: it computes the
@@ -18,18 +18,21 @@
 // HBM; each output point costs one inp read (plus the halo share), one
 // coeff read and one out write.
 //
-// Variant 2 (LDS-DMA tile; default wherever it applies).  The same arithmetic (HdiffTile::plane) on a
-// 64 x TY tile of one k-plane per workgroup, its (64+4) x (TY+4) input tile
-// staged straight into LDS by global-to-LDS loads: the tile is one
-// contiguous LDS array, so wave instruction n stages units 64n .. 64n+63
-// of it and no VGPR holds the staged data.  A unit is a 16-byte chunk (two
-// adjacent doubles of a row) for FP64 fields and one 4-byte element for
-// float32 fields.  With 64 x 8 FP64 tiles and 2 rows per thread a workgroup
-// needs 54 VGPRs and 11.4 KB of LDS, so eight share a CU and overlap one
-// another's staging and arithmetic.  It takes whole tiles only (nx a
-// multiple of 64, ny of TY) and unit i stride, and for FP64 fields even row
-// and plane strides and a 16-byte aligned interior origin; other domains
-// take variant 1.
+// Variant 2 (LDS-DMA tile; default wherever it applies).  The same arithmetic
+// (HdiffTile::plane) on a 64 x TY tile of one k-plane per workgroup, its
+// (64+4) x (TY+4) input tile staged straight into LDS by global-to-LDS loads:
+// no VGPR holds the staged data (HdiffDma, hdiff_tile.h).  With 64 x 8 FP64
+// tiles and 2 rows per thread a workgroup needs few registers and 11.4 KB of
+// LDS, so eight share a CU and overlap one another's staging and arithmetic.
+// The kernel is bound by memory in FP64 and FP32; float32 storage with FP64
+// arithmetic was bound by its instructions (a scalar unit serves the four
+// SIMDs of a CU, and a wave issued 177 scalar beside 210 vector
+// instructions; 111 and 165 now).  Unit i stride and a row pitch below 16 MiB
+// (hdiff_dma_unit); a domain's last tiles may be partial.  When the variant is
+// asked for by number it takes whole tiles only.  Measured on MI355X against
+// variant 1, launches back to back: 512x512x160 FP64 172 / 189 us, float32
+// storage 94 / 112 us, 397x411x137 96 / 110 and 53 / 70 us, 128x128x80 6.9 /
+// 9.5 and 5.1 / 11.6 us.
 //
 // Variant 3 (on the fly).  One thread per point reading its 13 inputs
 // through the caches; the schedule of the reference's OnTheFly body
@@ -83,90 +86,50 @@ __global__ __launch_bounds__(64 * (TY / RPT)) void hdiff_lds_kernel(
               s_lap);
 }
 
-// Variant 2 kernel (see the file comment).  The staged tile is one
-// contiguous LDS array counted from point (i0-2, j0-2), LW elements a row;
-// lane l of wave instruction n stages unit 64n + l of it.  A unit is a
-// 16-byte chunk (two adjacent doubles of a row) for 8-byte fields, whose
-// tile corner is then 16-byte aligned, and a 4-byte word (one element) for
-// float32 fields, which need no alignment beyond the element's.  The coeff
-// loads are non-temporal (not re-read), the stores plain.
-template <typename T, typename C, int TY, int RPT>
+// Variant 2 kernel: one 64 x TY tile of one k-plane per workgroup
+// (HdiffDma, hdiff_tile.h).
+template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT>
 __global__ __launch_bounds__(64 * (TY / RPT)) void hdiff_dma_kernel(
     const T *__restrict__ inp, const T *__restrict__ coeff, T *__restrict__ out, HdiffArgs a,
     TileGrid tg) {
-    using Tile = HdiffTile<T, C, TY, RPT, 2>;
-    constexpr int LW = Tile::LW, LH = Tile::LH, NW = Tile::NW;
-    constexpr int UNIT = sizeof(T) == 8 ? 16 : 4;   // bytes a lane stages per instruction
-    constexpr int PER = UNIT / int(sizeof(T));      // elements per unit: 2 or 1
-    constexpr int UNITS = LH * LW / PER;            // units of the staged tile
-    constexpr int STEPS = (UNITS + 63) / 64;        // wave instructions that stage it
-    static_assert(LW % PER == 0, "a unit must not straddle two rows");
-    __shared__ __attribute__((aligned(16))) T s_tile[STEPS * 64 * PER];
-    __shared__ C s_lap[Tile::LAP_ELEMS];
+    using Dma = HdiffDma<T, C, TY, RPT, UNIT, HINT>;
+    __shared__ __attribute__((aligned(16))) T s_tile[Dma::TILE_ELEMS];
+    __shared__ C s_lap[Dma::Tile::LAP_ELEMS];
     uint32_t ti, tj, k;
     tile_of(blockIdx.x, tg, ti, tj, k);
-    const int64_t i0 = int64_t(ti) * Tile::TX;
-    const int64_t j0 = int64_t(tj) * TY;
-    // the wave index read as wave-uniform: the branches on it and the row
-    // offsets derived from it are scalar
-    const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int tid = ty * Tile::TX + tx;
-    using GB = __attribute__((address_space(1))) const char *;
-    using GP = __attribute__((address_space(1))) const void *;
-    using LP = __attribute__((address_space(3))) void *;
-    const GB corner =
-        (GB)(inp) + ((int64_t(k) * a.sk + (j0 - 2) * a.sj + (i0 - 2)) * int64_t(sizeof(T)));
-    // row pitch below 2^24 bytes (checked on the host): a staged unit's byte
-    // offset from the tile corner is one 24-bit multiply and an add
-    const uint32_t pitch = uint32_t(a.sj) * uint32_t(sizeof(T));
-#pragma unroll
-    for (int n = 0; n < STEPS; ++n) {
-        if (n % NW != ty) continue;  // instruction n belongs to wave n % NW
-        const int c = n * 64 + tx;
-        if (c < UNITS) {
-            const uint32_t row = uint32_t(c) / (LW / PER);
-            const uint32_t unit = uint32_t(c) - __umul24(row, uint32_t(LW / PER));
-            const GP src = (GP)(corner + (__umul24(row, pitch) + unit * uint32_t(UNIT)));
-            if constexpr (UNIT == 16)
-                __builtin_amdgcn_global_load_lds(src, (LP)(s_tile + n * 64 * PER), 16, 0, 0);
-            else
-                __builtin_amdgcn_global_load_lds(src, (LP)(s_tile + n * 64 * PER), 4, 0, 0);
-        }
-    }
-    using GT = __attribute__((address_space(1))) const T *;
-    const int64_t point = int64_t(k) * a.sk + (j0 + ty * RPT) * a.sj + i0 + tx;
-    C cf[RPT];
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) cf[q] = C(__builtin_nontemporal_load((GT)(coeff) + point + q * a.sj));
-    __syncthreads();  // every wave's staging has landed
-    C res[RPT];
-    Tile::plane(s_tile, s_lap, cf, res, tx, ty, tid);
-    using GO = __attribute__((address_space(1))) T *;
-#pragma unroll
-    for (int q = 0; q < RPT; ++q) *((GO)(out) + point + q * a.sj) = T(res[q]);
+    Dma::run(as_global(inp), as_global(coeff), as_global(out), int32_t(a.nx), int32_t(a.ny),
+             int32_t(a.sj), a.sk, int32_t(ti * 64), int32_t(tj * TY), int32_t(k), s_tile, s_lap);
 }
 
-// Whether the variant-2 kernel with TY-row tiles takes this domain: whole
-// tiles, unit i stride, a positive row pitch below 16 MiB, and for 8-byte fields
-// (16-byte units) even row and plane strides and a 16-byte aligned interior
-// origin.
+// Whether variant 2 with TY-row tiles takes this domain when it is asked for:
+// whole tiles, unit i stride, a positive row pitch below 16 MiB, and for
+// 8-byte fields (16-byte units) even row and plane strides and a 16-byte
+// aligned interior origin.
 bool hdiff_dma_fits(const sb_geom *g, const void *inp, int ty, size_t itemsize) {
-    const bool tiles = g->si == 1 && g->nx % 64 == 0 && g->ny % ty == 0 && g->sj > 0 &&
-                       g->sj * int64_t(itemsize) < (int64_t(1) << 24);
-    if (itemsize != 8) return tiles;
-    return tiles && g->sj % 2 == 0 && g->sk % 2 == 0 && reinterpret_cast<uintptr_t>(inp) % 16 == 0;
+    const int unit = hdiff_dma_unit(*g, inp, itemsize);
+    return g->nx % 64 == 0 && g->ny % ty == 0 && unit >= (itemsize == 8 ? 16 : 4);
 }
 
-template <typename T, typename C, int TY, int RPT>
+// Workgroups of variant 2.
+uint64_t hdiff_dma_blocks(const HdiffArgs &a, int ty) {
+    return uint64_t((a.nx + 63) / 64) * uint64_t((a.ny + ty - 1) / ty) * uint64_t(a.nz);
+}
+
+template <typename T, typename C, int TY, int RPT, int UNIT>
 hipError_t launch_dma(const T *inp, const T *coeff, T *out, HdiffArgs a, Context *ctx) {
-    a.tiles_i = int32_t(a.nx / 64);
-    a.tiles_j = int32_t(a.ny / TY);
-    const uint64_t blocks = uint64_t(a.tiles_i) * uint64_t(a.tiles_j) * uint64_t(a.nz);
+    a.tiles_i = int32_t((a.nx + 63) / 64);
+    a.tiles_j = int32_t((a.ny + TY - 1) / TY);
+    const uint64_t blocks = hdiff_dma_blocks(a, TY);
     if (blocks >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
     const TileGrid tg = make_tile_grid(uint32_t(blocks), uint32_t(a.tiles_i), uint32_t(a.tiles_j),
                                        ctx->xcds);
-    enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT>), dim3(unsigned(blocks)), dim3(64, TY / RPT), 0,
-                   ctx->stream, inp, coeff, out, a, tg);
+    const dim3 grid{unsigned(blocks)}, threads{64u, unsigned(TY / RPT)};
+    if (hdiff_dma_hint(double(a.nx) * double(a.ny) * double(a.nz), sizeof(T)))
+        enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, true>), grid, threads, 0, ctx->stream,
+                       inp, coeff, out, a, tg);
+    else
+        enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, false>), grid, threads, 0,
+                       ctx->stream, inp, coeff, out, a, tg);
     return hipGetLastError();
 }
 
@@ -262,20 +225,17 @@ int launch_hdiff(const void *inp_v, const void *coeff_v, void *out_v, const sb_g
     // tile options (rows, planes, cache hints) select the register-staged tile
     const bool tile_options = l && (l->by || l->bz || l->unroll);
     int variant = l ? l->variant : 0;
+    const int unit = hdiff_dma_unit(*g, inp, sizeof(T));  // bytes that variant 2 stages at a time
     if (variant == 0) {
-        // the LDS-DMA tile where it applies (measured on MI355X at 512 x 512
-        // x 160 against variant 1's defaults: FP64 156.5-157.3 us against
-        // 168.7 us, FP32 80.7 us against 93.0-93.4 us, float32 storage with
-        // FP64 arithmetic 86.0 us against 97.5-99.2 us)
-        if (!tile_options && hdiff_dma_fits(g, inp, dma_rows, sizeof(T)))
+        // the LDS-DMA tile where it applies (figures: file comment)
+        if (!tile_options && unit && hdiff_dma_blocks(a, dma_rows) < (uint64_t(1) << 31))
             variant = 2;
         else
             variant = tile_fits ? 1 : 3;
-    }
-    if (variant == 2) {
-        const int ty2 = (l && l->by) ? l->by : dma_rows;
+    } else if (variant == 2) {
+        const int ty2 = l->by ? l->by : dma_rows;
         SB_REQUIRE(ty2 == 8 || ty2 == 16, "LDS-DMA hdiff tile height %d not in {8, 16}", ty2);
-        SB_REQUIRE(!l || (l->bz <= 1 && l->unroll == 0),
+        SB_REQUIRE(l->bz <= 1 && l->unroll == 0,
                    "the LDS-DMA hdiff tile takes one k-plane per workgroup and no cache-hint options");
         SB_REQUIRE(hdiff_dma_fits(g, inp, ty2, sizeof(T)),
                    "the LDS-DMA hdiff tile needs nx a multiple of 64, ny a multiple of %d, unit i "
@@ -283,9 +243,15 @@ int launch_hdiff(const void *inp_v, const void *coeff_v, void *out_v, const sb_g
                    "strides "
                    "and a 16-byte aligned interior origin",
                    ty2);
+    }
+    if (variant == 2) {
+        const int ty2 = (l && l->by) ? l->by : dma_rows;
         return timed_launch(l, seconds, [&]() -> hipError_t {
-            return ty2 == 8 ? launch_dma<T, C, 8, 2>(inp, coeff, out, a, ctx)
-                            : launch_dma<T, C, 16, 4>(inp, coeff, out, a, ctx);
+            if (unit == 16)
+                return ty2 == 8 ? launch_dma<T, C, 8, 2, 16>(inp, coeff, out, a, ctx)
+                                : launch_dma<T, C, 16, 4, 16>(inp, coeff, out, a, ctx);
+            return ty2 == 8 ? launch_dma<T, C, 8, 2, 4>(inp, coeff, out, a, ctx)
+                            : launch_dma<T, C, 16, 4, 4>(inp, coeff, out, a, ctx);
         });
     }
     SB_REQUIRE(variant != 1 || tile_fits,

@@ -96,8 +96,8 @@ struct HdiffTile {
     static constexpr int LAP_ELEMS = TY * PW;
 
     // Laplacian, limited fluxes and update of the calling thread's RPT output
-    // points (column tx, rows ty*RPT ..) from one staged plane `sin` (LW
-    // elements of type S per row, rows -2 .. TY+1, columns -2 .. TX+1; each
+    // points (column tx, rows ty*RPT ..) from one staged plane `sin` (SW
+    // elements of type S per row, rows -2 .. TY+1, columns from -LEFT on; each
     // read widened to the arithmetic type C, so a plane staged in the storage
     // type gives the same results as one staged in C).  Each thread
     // computes its column's Laplacian for rows -1..RPT in registers and
@@ -108,33 +108,41 @@ struct HdiffTile {
     // which keeps its own copy: calling this from there changes the register
     // allocation of the float32-storage kernel (126 -> 130 VGPRs, one wave
     // per SIMD fewer, 100 -> 110 us at 512x512x160).
-    template <typename S>
+    template <int SW = LW, int LEFT = 2, typename S>
     __device__ static void plane(const S *sin, C *s_lap, const C (&cf)[RPT], C (&res)[RPT], int tx,
                                  int ty, int tid) {
-        const int col = tx + 2;         // staged column of this thread
+        // 4 c - sum: 4 c of a float32 value is exact in FP64, so the fused form
+        // rounds once, as the two operations do
+        auto laplacian = [](C c, C sum) {
+            if constexpr (sizeof(S) == 4 && sizeof(C) == 8)
+                return __builtin_fma(C(4), c, -sum);
+            else
+                return C(4) * c - sum;
+        };
+        const int col = tx + LEFT;      // staged column of this thread
         const int row0 = ty * RPT + 2;  // staged row of its first output
         C ic[RPT + 4], il[RPT + 2], ir[RPT + 2], lap[RPT + 2];
     #pragma unroll
-        for (int q = 0; q < RPT + 4; ++q) ic[q] = C(sin[(row0 - 2 + q) * LW + col]);
+        for (int q = 0; q < RPT + 4; ++q) ic[q] = C(sin[(row0 - 2 + q) * SW + col]);
     #pragma unroll
         for (int q = 0; q < RPT + 2; ++q) {
-            il[q] = C(sin[(row0 - 1 + q) * LW + col - 1]);
-            ir[q] = C(sin[(row0 - 1 + q) * LW + col + 1]);
+            il[q] = C(sin[(row0 - 1 + q) * SW + col - 1]);
+            ir[q] = C(sin[(row0 - 1 + q) * SW + col + 1]);
         }
     #pragma unroll
         for (int q = 0; q < RPT + 2; ++q)
-            lap[q] = C(4) * ic[q + 1] - (((ir[q] + il[q]) + ic[q + 2]) + ic[q]);
+            lap[q] = laplacian(ic[q + 1], ((ir[q] + il[q]) + ic[q + 2]) + ic[q]);
     #pragma unroll
         for (int q = 0; q < RPT; ++q) s_lap[(ty * RPT + q) * PW + tx + 1] = lap[q + 1];
         if (tid < 2 * TY) {
             // Laplacian of the tile's halo columns -1 and TX.
             const int side = tid / TY, r = tid - side * TY;
-            const int c = side ? TX + 2 : 1;
+            const int c = side ? TX + LEFT : LEFT - 1;
             const int rr = r + 2;
-            const C v = C(4) * C(sin[rr * LW + c]) -
-                        (((C(sin[rr * LW + c + 1]) + C(sin[rr * LW + c - 1])) +
-                          C(sin[(rr + 1) * LW + c])) +
-                         C(sin[(rr - 1) * LW + c]));
+            const C v = laplacian(C(sin[rr * SW + c]),
+                                  ((C(sin[rr * SW + c + 1]) + C(sin[rr * SW + c - 1])) +
+                                   C(sin[(rr + 1) * SW + c])) +
+                                      C(sin[(rr - 1) * SW + c]));
             s_lap[r * PW + (side ? TX + 1 : 0)] = v;
         }
         __syncthreads();
@@ -286,6 +294,150 @@ struct HdiffTile {
         }
     }
 };
+
+// LDS-DMA tile worker, shared by the plain kernel's variant 2 (hdiff.hip) and
+// the batched kernel (batch.hip): the calling workgroup (64 x TY/RPT threads)
+// computes the 64 x TY output tile at (i0, j0) of plane k.  The staged tile
+// is one contiguous LDS array counted from point (i0-LEFT, j0-2), LW elements
+// a row; lane l of wave instruction n stages unit 64n + l of it.  A unit is a
+// 16-byte chunk of a row (two doubles from column i0-2 on, four floats from
+// column i0-4 on) for fields whose tile corners are 16-byte aligned, else a
+// 4-byte word, which needs no alignment beyond the element's.  Float32 fields
+// gain most from the wide units: FP64 arithmetic bounds the kernel by its
+// instructions, and 64x16 tiles take 6 staging instructions instead of 22.
+// The stores are non-temporal (512x512x160 FP64 179 -> 172 us, float32
+// storage 95 -> 91 us; a vadv launch that reads the result next loses nothing
+// by it), and with HINT the coeff loads (dma_hint below).
+//
+// A tile that reaches past the domain's last row or column (EDGE, a uniform
+// branch) clamps its unit addresses to the last halo row and to the unit that
+// holds column nx + 1, as the register-staged tile does: what is staged there
+// only feeds outputs that are not stored.  A 16-byte unit may read up to two
+// columns more than the halo of 2 on either side; hdiff_dma_unit says where
+// the field holds them.
+template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT>
+struct HdiffDma {
+    using Tile = HdiffTile<T, C, TY, RPT, 2>;
+    static constexpr int LEFT = UNIT == 16 ? 16 / int(sizeof(T)) : 2;
+    static constexpr int LW = Tile::TX + 2 * LEFT, LH = Tile::LH, NW = Tile::NW;
+    static constexpr int WORDS = int(sizeof(T)) * LW / UNIT;  // units of a staged row
+    static constexpr int UNITS = LH * WORDS;
+    static constexpr int STEPS = (UNITS + 63) / 64;  // wave instructions that stage the tile
+    static constexpr int TILE_ELEMS = STEPS * 64 * UNIT / int(sizeof(T));
+    static_assert(int(sizeof(T)) * LW % UNIT == 0, "a unit must not straddle two rows");
+
+    // `corner` points at the tile's first staged element; wave ty of the NW
+    // issues instructions ty, ty + NW, ...
+    template <bool EDGE>
+    __device__ __forceinline__ static void stage(global_ptr<const T> corner, T *s_tile,
+                                                 uint32_t last_row, uint32_t last_unit,
+                                                 uint32_t pitch, int tx, int ty) {
+        __builtin_assume(tx >= 0 && tx < 64 && ty >= 0 && ty < NW);
+        using GP = __attribute__((address_space(1))) const void *;
+        using LP = __attribute__((address_space(3))) void *;
+    #pragma unroll
+        for (int m = 0; m < (STEPS + NW - 1) / NW; ++m) {
+            const int n = ty + NW * m;
+            const int c = n * 64 + tx;
+            if ((m + 1) * NW * 64 <= UNITS || c < UNITS) {
+                uint32_t row = uint32_t(c) / WORDS;
+                uint32_t unit = uint32_t(c) - __umul24(row, uint32_t(WORDS));
+                if constexpr (EDGE) {
+                    row = min(row, last_row);
+                    unit = min(unit, last_unit);
+                }
+                const GP src = (GP)at(corner, __umul24(row, pitch) + unit * uint32_t(UNIT));
+                LP dst = (LP)((char *)s_tile + n * 64 * UNIT);
+                if constexpr (UNIT == 16)
+                    __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
+                else
+                    __builtin_amdgcn_global_load_lds(src, dst, 4, 0, 0);
+            }
+        }
+    }
+
+    // A pointer kept in scalar registers, apart from the offset arithmetic
+    // around it: the accesses then take the scalar-base form, one vector
+    // register of offset each.
+    template <typename P>
+    __device__ __forceinline__ static P scalar(P p) {
+        uint64_t v = (uint64_t)p;
+        __asm__("" : "+s"(v));
+        return (P)v;
+    }
+
+    // Offsets within a plane are 32-bit (hdiff_dma_unit), on a plane's uniform
+    // base.
+    __device__ static void run(global_ptr<const T> inp, global_ptr<const T> coeff,
+                               global_ptr<T> out, int32_t nx, int32_t ny, int32_t sj, int64_t sk,
+                               int32_t i0, int32_t j0, int32_t k, T *s_tile, C *s_lap) {
+        // the wave index read as wave-uniform: the branches on it and the row
+        // offsets derived from it are scalar
+        const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
+        const int tid = ty * Tile::TX + tx;
+        const bool edge = i0 + Tile::TX > nx || j0 + TY > ny;
+        // row pitch below 2^24 bytes (checked on the host): a staged unit's byte
+        // offset from the tile corner is one 24-bit multiply and an add
+        const uint32_t pitch = uint32_t(sj) * uint32_t(sizeof(T));
+        const int64_t plane = k * sk;
+        const global_ptr<const T> corner = scalar(inp + plane + ((j0 - 2) * sj + (i0 - LEFT)));
+        if (edge) {
+            const uint32_t last_row = uint32_t(ny + 3 - j0);
+            const uint32_t last_unit =
+                uint32_t(nx + 1 + LEFT - i0) * uint32_t(sizeof(T)) / uint32_t(UNIT) +
+                (UNIT < int(sizeof(T)) ? 1u : 0u);
+            stage<true>(corner, s_tile, last_row, last_unit, pitch, tx, ty);
+        } else {
+            stage<false>(corner, s_tile, 0, 0, pitch, tx, ty);
+        }
+        const int row0 = j0 + ty * RPT;  // this wave's first output row
+        const global_ptr<const T> cf_k = scalar(coeff + plane + i0);
+        const global_ptr<T> out_k = scalar(out + plane + i0);
+        // lanes past the domain re-read its last column, rows its last row
+        const uint32_t lane = uint32_t(min(tx, nx - 1 - i0)) * uint32_t(sizeof(T));
+        C cf[RPT];
+    #pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            cf[q] = C(ld_nt<HINT>(at(cf_k, uint32_t(min(row0 + q, ny - 1)) * pitch + lane)));
+        __syncthreads();  // every wave's staging has landed
+        C res[RPT];
+        Tile::template plane<LW, LEFT>(s_tile, s_lap, cf, res, tx, ty, tid);
+        if (tx < nx - i0) {
+    #pragma unroll
+            for (int q = 0; q < RPT; ++q)
+                if (row0 + q < ny) st_nt<true>(at(out_k, uint32_t(row0 + q) * pitch + lane), T(res[q]));
+        }
+    }
+};
+
+// Whether coeff is loaded non-temporally: not where inp, coeff and out of a
+// launch together are small enough to stay in the Infinity Cache until they
+// are used again (200x200x80 FP64, 77 MB: 16.1 us with the hint, 13.7 without;
+// 400x400x100 float32 storage, 192 MB: 36.8 / 41.1 us).
+inline bool hdiff_dma_hint(double points, size_t itemsize) {
+    return 3 * points * double(itemsize) > 96.0 * (1 << 20);
+}
+
+// Bytes of the unit that the LDS-DMA tile stages this field by, or 0 where it
+// does not take it: unit i stride, a positive row pitch below 16 MiB and a
+// plane below 4 GiB (2^31 elements); 16
+// where the tile corners are 16-byte aligned (row and plane strides of whole
+// chunks and an aligned interior origin) and the field holds the columns
+// beyond the halo of 2 that come with the chunks: column nx + 2 with odd nx
+// (8-byte fields, a halo of 3), or columns -4 .. nx + 3 (4-byte fields; past
+// a row's own halo they are in the neighbouring rows or planes).
+inline int hdiff_dma_unit(const sb_geom &g, const void *inp, size_t itemsize) {
+    if (g.si != 1 || g.sj <= 0 || g.sj * int64_t(itemsize) >= (int64_t(1) << 24)) return 0;
+    if (!hdiff_tile_fits(g.nx, g.ny, g.si, g.sj, itemsize) ||
+        (g.ny + 3) * g.sj + g.nx + 4 >= (int64_t(1) << 31))
+        return 0;
+    const int64_t chunk = 16 / int64_t(itemsize);
+    const bool aligned = g.sj % chunk == 0 && g.sk % chunk == 0 &&
+                         reinterpret_cast<uintptr_t>(inp) % 16 == 0;
+    const bool holds = itemsize == 8 ? g.nx % 2 == 0 || g.hi >= 3
+                                     : g.hi >= 4 || g.hj >= 3 || g.hk >= 1;
+    return aligned && holds ? 16 : 4;
+}
 
 }  // namespace
 }  // namespace sb

@@ -164,19 +164,19 @@ __host__ __device__ inline uint32_t xcd_chunk_remap(uint32_t b, uint32_t total, 
 // Division of a dividend below 2^31 by a divisor fixed at launch: q =
 // (n * mul) >> shift with mul = ceil(2^shift / d), shift = 31 + ceil(log2 d).
 // The rounding error of mul stays below 1/d of the quotient's unit for every
-// such n, so q = floor(n / d) exactly.  Wave-uniform dividends then take a
+// such n, so q = floor(n / d) exactly; mul stays below 2^32, since 2^shift / d
+// < 2^32.  Wave-uniform dividends then take a
 // few scalar instructions instead of the VALU reciprocal sequence of a
 // division by a run-time divisor.
 struct UDiv {
-    uint64_t mul;
-    uint32_t shift, d;
+    uint32_t mul, shift, d;
 };
 
 inline UDiv make_udiv(uint32_t d) {
     uint32_t l = 0;
     while ((uint64_t(1) << l) < d) ++l;
     const uint32_t shift = 31 + l;
-    return UDiv{((uint64_t(1) << shift) + d - 1) / d, shift, d};
+    return UDiv{uint32_t(((uint64_t(1) << shift) + d - 1) / d), shift, d};
 }
 
 __host__ __device__ inline uint32_t udiv(uint32_t n, const UDiv &u) {

@@ -276,6 +276,25 @@ def test_hdiff_lds_dma_tile(gpu, prec, tile, domain, halo, alignment):
     _check_halo(got, domain, halo)
 
 
+# the default tile on domains of partial tiles: columns and rows around the
+# tile's edges, staged by 16-byte chunks (aligned rows, halos that hold the
+# chunks' extra columns) and by words (odd strides, narrow halos)
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("domain", [(1, 1, 1), (2, 7, 2), (63, 8, 3), (65, 9, 2), (66, 15, 2),
+                                    (127, 16, 1), (129, 17, 4), (200, 33, 3)])
+@pytest.mark.parametrize("halo,alignment", [((2, 2, 0), 64), ((2, 3, 0), 16), ((3, 3, 3), 64),
+                                            ((3, 2, 1), 8), ((4, 2, 0), 128), ((3, 3, 3), 0)])
+def test_hdiff_partial_tiles(gpu, prec, domain, halo, alignment):
+    dtype = _dtype(prec)
+    inp, coeff = make_fields(domain, halo, dtype, (2, 1, 0), alignment, count=2,
+                             seed=sum(domain) + alignment)
+    out = _with_sentinel(make_fields(domain, halo, dtype, (2, 1, 0), alignment)[0])
+    got, = _run(gpu, "sb_hdiff", [inp, coeff, out], [2], domain, halo, _prec(gpu, prec))
+    expected = _expected(lambda a, b: oracle.hdiff(a, b, domain, halo), [inp, coeff], prec)
+    assert np.array_equal(got[inner(domain, halo)], expected)
+    _check_halo(got, domain, halo)
+
+
 @pytest.mark.parametrize("domain,prec,tile,match", [((70, 16, 2), "f64", 0, "multiple of 64"),
                                                     ((64, 12, 2), "f64", 0, "multiple of 8"),
                                                     ((70, 16, 2), "f32_f64", 0, "multiple of 64"),
