@@ -263,8 +263,10 @@ int sb_stream_check(int prec, const void *x, size_t n, double expected,
  * values; they are never written.  Requirements: hi, hj >= 2, nz >= 2,
  * positive strides, every field below 4 GiB, nz small enough that a 64-column
  * Thomas buffer fits in LDS (nz <= 160 with FP64 arithmetic).
- * Launch options: hdiff_launch->by / ->bz / ->unroll = tile height / planes
- * per item / non-temporal flags (as sb_hdiff); vadv_launch all zero = the
+ * Launch options: hdiff_launch all zero = the LDS-DMA tile of sb_hdiff, one
+ * workgroup per tile and plane (where it takes every subdomain); ->by / ->bz /
+ * ->unroll = tile height / planes per item / non-temporal flags of the
+ * register-staged tile, drawn from work queues; vadv_launch all zero = the
  * register-column solver of sb_vadv's variant 5, one launch per register
  * build the columns need; ->variant = 4 (also 0 with any option of it:
  * warp-specialised solver, items of ->by column groups, 0 = 16,
@@ -283,8 +285,9 @@ typedef struct sb_subdomain {
     int32_t reserved;
 } sb_subdomain;
 
-/* One timestep for `count` subdomains: a counter reset, one persistent hdiff
- * launch (tiles from per-XCD device work queues) and the vadv launches (by
+/* One timestep for `count` subdomains: one hdiff launch (with hdiff options a
+ * persistent one, tiles from per-XCD device work queues; a counter reset
+ * precedes launches that use queues) and the vadv launches (by
  * default one to five, a workgroup per column group; warp-specialised: one or
  * two persistent ones, column-group items from per-XCD device work queues,
  * one launch per LDS class; variant 3: items from one device counter).  Does not flip the parities; the caller does. */

@@ -5,8 +5,8 @@ The reference sweeps block sizes by hand (its collection scripts run fixed
 tools/multirun.py); here the sweep is a tuner that times candidate launch
 options on the device and keeps the fastest per device and workload:
 
-* batched steps (`tune_batch`): hdiff tile height, k-planes per item and
-  cache hints, then the vadv solver (register columns, warp-specialised with
+* batched steps (`tune_batch`): the LDS-DMA hdiff or the register-staged one
+  with its tile height, k-planes per item and cache hints, then the vadv solver (register columns, warp-specialised with
   8/16/32 column groups per item, 4 or 8 levels per barrier step and 4 or 5
   waves, or the single-wave pipeline at prefetch depth 4/8),
   chosen by coordinate descent (hdiff with the default vadv, then vadv with
@@ -38,10 +38,12 @@ import numpy as np
 
 from . import native
 
-# hdiff options of the batched step (launch->by tile rows, ->bz k-planes per
+# hdiff options of the batched step (none: the LDS-DMA tile, a workgroup per
+# tile and plane; else the register-staged tile: launch->by tile rows, ->bz k-planes per
 # item, ->unroll 4 = plain coeff loads instead of non-temporal ones): the
 # combinations the batched kernel is built for
 BATCH_HDIFF_SPACE = (
+    {},
     {"by": 16, "bz": 8}, {"by": 16, "bz": 8, "unroll": 4}, {"by": 16, "bz": 4},
     {"by": 16, "bz": 2}, {"by": 16, "bz": 2, "unroll": 4}, {"by": 32, "bz": 2},
     {"by": 16, "bz": 1}, {"by": 8, "bz": 1},

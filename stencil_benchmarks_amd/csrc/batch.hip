@@ -49,7 +49,10 @@
 // captured in a hipGraph and replayed).  Every workgroup exits once the
 // counters pass their item counts.
 //
-// By default vadv runs the register-column solver (vadv_regs.h) instead, one
+// By default hdiff runs the plain kernel's LDS-DMA tile instead, one workgroup
+// per tile and plane (hdiff_dma_batch_kernel; 32 subdomains of 32..512 squared
+// x 40..160, float32 storage 772 -> 600 us per step), and
+// vadv runs the register-column solver (vadv_regs.h), one
 // workgroup per column group and one launch per register build that the
 // columns need (vadv_reg_batch_kernel).  Measured on MI355X against the
 // warp-specialised launches, whole steps with the hdiff launch: 32 subdomains
@@ -229,6 +232,35 @@ __global__ __launch_bounds__(64 * (TY / RPT)) void hdiff_batch_kernel(
     }
 }
 
+// Default hdiff of a step: the plain kernel's LDS-DMA tile (HdiffDma,
+// hdiff_tile.h) over the tiles and planes of all subdomains, one workgroup
+// each and no queue: the tiles cost the same, so the dispatcher balances
+// them, and consecutive ones run on one XCD.  first[s] is the first item of
+// subdomain s and start[i] the subdomain that item 2^kStartShift i belongs to,
+// so a workgroup finds its own in a few scalar loads.
+constexpr int kStartShift = 6;
+
+template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT>
+__global__ __launch_bounds__(64 * (TY / RPT)) void hdiff_dma_batch_kernel(
+    const SubDev *__restrict__ subs, const int32_t *__restrict__ first,
+    const int32_t *__restrict__ start, TileGrid tg) {
+    using Dma = HdiffDma<T, C, TY, RPT, UNIT, HINT>;
+    __shared__ __attribute__((aligned(16))) T s_tile[Dma::TILE_ELEMS];
+    __shared__ C s_lap[Dma::Tile::LAP_ELEMS];
+    const int32_t item = int32_t(remapped(blockIdx.x, tg));
+    int s = start[item >> kStartShift];
+    while (first[s + 1] <= item) ++s;
+    const SubDev &d = subs[s];
+    const uint32_t local = uint32_t(item - first[s]);
+    const uint32_t k = udiv(local, d.hdiv_tiles);
+    const uint32_t t = local - k * d.hdiv_tiles.d;
+    const uint32_t tj = udiv(t, d.hdiv_tiles_i);
+    const uint32_t ti = t - tj * d.hdiv_tiles_i.d;
+    Dma::run(as_global(static_cast<const T *>(d.inp)), as_global(static_cast<const T *>(d.coeff)),
+             as_global(static_cast<T *>(d.out)), int32_t(d.nx), int32_t(d.ny), int32_t(d.sj), d.sk,
+             int32_t(ti * 64), int32_t(tj * TY), int32_t(k), s_tile, s_lap);
+}
+
 template <typename T, typename C, int PF, bool NT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
 void vadv_batch_kernel(const SubDev *__restrict__ subs, const int64_t *__restrict__ prefix,
@@ -370,6 +402,13 @@ struct Plan {
         std::vector<VItem> host_list;
     } ws[2];
     std::vector<int8_t> host_vclass;  // LDS class of each subdomain (by rank)
+    // LDS-DMA hdiff (the default): bytes of its staging unit (0: the queues
+    // of register-staged tiles), first item of each subdomain and the total,
+    // then the subdomain of every 2^kStartShift-th item
+    int dma_unit = 0;
+    bool dma_hint = false;
+    std::vector<int32_t> host_dma;
+    int32_t *dma = nullptr;
     // register-column vadv (the default): one launch per class
     struct RegClass {
         int build = 0;
@@ -395,6 +434,10 @@ struct Plan {
     int stage_next = 0;
 };
 
+// hdiff options select the register-staged tile
+bool hdiff_options(const sb_launch *l) { return l && (l->by || l->bz || l->unroll); }
+// rows of the LDS-DMA tile: the plain kernel's defaults
+int dma_rows(int prec) { return prec == SB_F64 ? 8 : 16; }
 int hdiff_ty(const sb_launch *l) { return (l && l->by) ? l->by : 16; }
 int hdiff_kc(const sb_launch *l, int) {
     // 8 planes per item measured best for every precision on the 96-subdomain
@@ -565,7 +608,23 @@ void build_reg_classes(Plan &p, const Context *ctx) {
 void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch *hl, Plan &p,
                   const Context *ctx) {
     const size_t esize = prec == SB_F64 ? 8 : 4;
-    const int ty = hdiff_ty(hl), kc = hdiff_kc(hl, prec);
+    // the LDS-DMA hdiff where it takes every subdomain, by the narrowest
+    // staging unit that one of them needs
+    double points = 0.0;
+    uint64_t dma_items = 0;
+    p.dma_unit = hdiff_options(hl) ? 0 : 16;
+    for (int i = 0; i < count; ++i) {
+        const sb_geom &g = subs[i].geom;
+        for (const void *u : subs[i].u) p.dma_unit = std::min(p.dma_unit, hdiff_dma_unit(g, u, esize));
+        points += double(g.nx) * double(g.ny) * double(g.nz);
+        dma_items += uint64_t((g.nx + 63) / 64) *
+                     uint64_t((g.ny + dma_rows(prec) - 1) / dma_rows(prec)) * uint64_t(g.nz);
+    }
+    if (dma_items >= (uint64_t(1) << 31)) p.dma_unit = 0;
+    p.dma_hint = hdiff_dma_hint(points, esize);
+    p.host_dma.clear();
+    const int ty = p.dma_unit ? dma_rows(prec) : hdiff_ty(hl);
+    const int kc = p.dma_unit ? 1 : hdiff_kc(hl, prec);
     std::vector<int> order(count);
     std::iota(order.begin(), order.end(), 0);
     auto cost = [&](int i) {
@@ -652,6 +711,34 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
             if (p.ws[c].max_nz)
                 schedule_ws(p, c, p.ws[c].per_cu * ctx->compute_units, vadv_queues(ctx));
     if (vadv_variant(&p.vl) == kRegVariant) build_reg_classes(p, ctx);
+    if (p.dma_unit) {
+        p.host_dma.assign(p.host_hprefix.begin(), p.host_hprefix.end());
+        int32_t s = 0;
+        for (int64_t item = 0; item < p.host_hprefix[count]; item += int64_t(1) << kStartShift) {
+            while (p.host_hprefix[s + 1] <= item) ++s;
+            p.host_dma.push_back(s);
+        }
+    }
+}
+
+// The hdiff launch of the LDS-DMA tile.
+template <typename T, typename C, int UNIT, bool HINT>
+hipError_t enqueue_dma_k(const Plan &p, const SubDev *subs, Context *ctx) {
+    constexpr int TY = sizeof(T) == 8 ? 8 : 16, RPT = TY / 4;
+    const uint32_t items = uint32_t(p.host_dma[size_t(p.count)]);
+    const TileGrid tg = make_tile_grid(items, 1, 1, ctx->xcds);
+    hipLaunchKernelGGL((hdiff_dma_batch_kernel<T, C, TY, RPT, UNIT, HINT>), dim3(items), dim3(64, 4),
+                       0, ctx->stream, subs, p.dma, p.dma + p.count + 1, tg);
+    return hipGetLastError();
+}
+
+template <typename T, typename C>
+hipError_t enqueue_dma(const Plan &p, const SubDev *subs, Context *ctx) {
+    if (p.dma_unit == 16)
+        return p.dma_hint ? enqueue_dma_k<T, C, 16, true>(p, subs, ctx)
+                          : enqueue_dma_k<T, C, 16, false>(p, subs, ctx);
+    return p.dma_hint ? enqueue_dma_k<T, C, 4, true>(p, subs, ctx)
+                      : enqueue_dma_k<T, C, 4, false>(p, subs, ctx);
 }
 
 // The vadv launch of one class.
@@ -696,7 +783,8 @@ hipError_t enqueue_step(const Plan &p, int flip, unsigned long long *counters, C
     if (ty == TY_ && kc == KC_ && fl == FL_)                                                \
         return_h = launch_h(hdiff_batch_kernel<T, C, TY_, RPT_, KC_, FL_>, 64 * (TY_ / RPT_));
     hipError_t return_h = hipErrorInvalidValue;
-    SB_HB(16, 4, 2, 2) else SB_HB(16, 4, 2, 0) else SB_HB(16, 4, 8, 2) else SB_HB(16, 4, 8, 0)
+    if (p.dma_unit) return_h = enqueue_dma<T, C>(p, subs, ctx);
+    else SB_HB(16, 4, 2, 2) else SB_HB(16, 4, 2, 0) else SB_HB(16, 4, 8, 2) else SB_HB(16, 4, 8, 0)
         else SB_HB(8, 2, 1, 2) else SB_HB(32, 8, 2, 2) else SB_HB(16, 4, 4, 2) else SB_HB(16, 4, 1, 2)
 #undef SB_HB
     if (return_h != hipSuccess) return return_h;
@@ -762,10 +850,13 @@ hipError_t enqueue_step(const Plan &p, int flip, unsigned long long *counters, C
 
 template <typename T, typename C>
 hipError_t enqueue_sequence(const Plan &p, Context *ctx) {
-    const int ncounters = kCountersPerStep * p.steps;
-    hipLaunchKernelGGL(reset_counters, dim3((ncounters + 255) / 256), dim3(256), 0, ctx->stream,
-                       p.counters, ncounters);
-    hipError_t e = hipGetLastError();
+    hipError_t e = hipSuccess;
+    if (!p.dma_unit || vadv_variant(&p.vl) != kRegVariant) {  // there are queues
+        const int ncounters = kCountersPerStep * p.steps;
+        hipLaunchKernelGGL(reset_counters, dim3((ncounters + 255) / 256), dim3(256), 0, ctx->stream,
+                           p.counters, ncounters);
+        e = hipGetLastError();
+    }
     for (int s = 0; s < p.steps && e == hipSuccess; ++s)
         e = enqueue_step<T, C>(p, s & 1, p.counters + size_t(kCountersPerStep) * s, ctx);
     return e;
@@ -787,6 +878,7 @@ int upload_tables(Plan &p, Context *ctx) {
         ws_bytes += ((sizeof(int32_t) * c.host_off.size() + 7) & ~size_t(7)) +
                     sizeof(VItem) * c.host_list.size();
     for (const Plan::RegClass &c : p.reg) ws_bytes += sizeof(int32_t) * c.host.size();
+    ws_bytes += sizeof(int32_t) * p.host_dma.size();
     const size_t need = sched + ws_bytes + 256;
     if (p.dev_bytes < need) {
         // steps enqueued earlier may still read the old tables
@@ -842,6 +934,10 @@ int upload_tables(Plan &p, Context *ctx) {
         std::memcpy(host + at, c.host.data(), sizeof(int32_t) * c.host.size());
         at += sizeof(int32_t) * c.host.size();
     }
+    p.dma = reinterpret_cast<int32_t *>(base + at);
+    if (!p.host_dma.empty())
+        std::memcpy(host + at, p.host_dma.data(), sizeof(int32_t) * p.host_dma.size());
+    at += sizeof(int32_t) * p.host_dma.size();
     // one copy, ordered on the stream before the steps that read the tables
     // (and after the previous steps, which read the same device tables)
     SB_HIP(hipMemcpyAsync(p.dev, host, at, hipMemcpyHostToDevice, ctx->stream));

@@ -208,10 +208,15 @@ inline TileGrid make_tile_grid(uint32_t blocks, uint32_t tiles_i, uint32_t tiles
     return g;
 }
 
+// Logical index of workgroup b (the grid's XCD remap).
+__host__ __device__ inline uint32_t remapped(uint32_t b, const TileGrid &g) {
+    return b < g.full ? (b & g.xcd_mask) * g.per + (b >> g.xcd_shift) : b;
+}
+
 // Tile (ti, tj) and plane k of workgroup b of such a grid.
 __host__ __device__ inline void tile_of(uint32_t b, const TileGrid &g, uint32_t &ti, uint32_t &tj,
                                uint32_t &k) {
-    if (b < g.full) b = (b & g.xcd_mask) * g.per + (b >> g.xcd_shift);
+    b = remapped(b, g);
     k = udiv(b, g.tiles);
     const uint32_t t = b - k * g.tiles.d;
     tj = udiv(t, g.tiles_i);
