@@ -5,13 +5,14 @@ The reference sweeps block sizes by hand (its collection scripts run fixed
 tools/multirun.py); here the sweep is a tuner that times candidate launch
 options on the device and keeps the fastest per device and workload:
 
-* batched steps (`tune_batch`): the LDS-DMA hdiff or the register-staged one
-  with its tile height, k-planes per item and cache hints, then the vadv solver (register columns, warp-specialised with
-  8/16/32 column groups per item, 4 or 8 levels per barrier step and 4 or 5
-  waves, or the single-wave pipeline at prefetch depth 4/8),
-  chosen by coordinate descent (hdiff with the default vadv, then vadv with
-  the chosen hdiff), each candidate timed over whole steps on scratch
-  subdomains of the workload's geometry (user fields are never advanced);
+* batched steps (`tune_batch`): hdiff tile height, k-planes per item and
+  cache hints, then the vadv solver (warp-specialised with 8/16/32 column
+  groups per item, 4 or 8 levels per barrier step and 4 or 5 waves, or the
+  single-wave pipeline at prefetch depth 4/8),
+  chosen by coordinate descent (hdiff with the first vadv, then vadv with
+  the chosen hdiff), then compared with no options at all, each candidate
+  timed over whole steps on scratch subdomains of the workload's geometry
+  (user fields are never advanced);
 * plain horizontal diffusion (`tune_hdiff`): tile height x k-planes x cache
   hints over one domain;
 * plain vertical advection (`tune_vadv`): the warp-specialised solver at 4 or
@@ -38,21 +39,18 @@ import numpy as np
 
 from . import native
 
-# hdiff options of the batched step (none: the LDS-DMA tile, a workgroup per
-# tile and plane; else the register-staged tile: launch->by tile rows, ->bz k-planes per
+# hdiff options of the batched step's register-staged tile (launch->by tile rows, ->bz k-planes per
 # item, ->unroll 4 = plain coeff loads instead of non-temporal ones): the
 # combinations the batched kernel is built for
 BATCH_HDIFF_SPACE = (
-    {},
     {"by": 16, "bz": 8}, {"by": 16, "bz": 8, "unroll": 4}, {"by": 16, "bz": 4},
     {"by": 16, "bz": 2}, {"by": 16, "bz": 2, "unroll": 4}, {"by": 32, "bz": 2},
     {"by": 16, "bz": 1}, {"by": 8, "bz": 1},
 )
-# vadv options of the batched step (none: register columns; variant 4: ->by column groups per item,
+# vadv options of the batched step (variant 4: ->by column groups per item,
 # ->unroll levels per barrier step, ->bx waves per workgroup; variant 3:
 # ->unroll prefetch depth)
 BATCH_VADV_SPACE = (
-    {},
     {"variant": 4, "by": 16}, {"variant": 4, "by": 8}, {"variant": 4, "by": 32},
     {"variant": 4, "by": 16, "unroll": 8}, {"variant": 4, "by": 8, "unroll": 8},
     {"variant": 4, "by": 32, "unroll": 8},
@@ -161,14 +159,16 @@ class TuneResult:
     seconds: float
     from_cache: bool
     trials: list = field(default_factory=list)
+    # no options were faster than the best of the spaces, `hdiff` and `vadv`
+    defaults: bool = False
 
     @property
     def hdiff_options(self):
-        return launch_from(self.hdiff)
+        return launch_from({} if self.defaults else self.hdiff)
 
     @property
     def vadv_options(self):
-        return launch_from(self.vadv)
+        return launch_from({} if self.defaults else self.vadv)
 
 
 def tune_batch(specs, storage, compute=None, cache=None, repeats=3, force=False, warmup=4):
@@ -185,7 +185,8 @@ def tune_batch(specs, storage, compute=None, cache=None, repeats=3, force=False,
     cache = cache if cache is not None else TuneCache()
     hit = None if force else cache.get(key)
     if hit:
-        return TuneResult(key, hit["hdiff"], hit["vadv"], hit["seconds"], True)
+        return TuneResult(key, hit["hdiff"], hit["vadv"], hit["seconds"], True,
+                          defaults=hit.get("defaults", False))
     scratch = [batch.Subdomain(s.domain, s.halo, storage, seed=index)
                for index, s in enumerate(specs)]
     try:
@@ -203,11 +204,17 @@ def tune_batch(specs, storage, compute=None, cache=None, repeats=3, force=False,
 
         h, v, seconds, trials = descend(BATCH_HDIFF_SPACE, BATCH_VADV_SPACE, measure,
                                         BATCH_VADV_SPACE[0])
+        # the kernels without options, the LDS-DMA tile and the register
+        # columns, have no entry in the spaces
+        trials.append(({}, {}, measure({}, {})))
+        defaults = trials[-1][2] <= seconds
+        seconds = min(seconds, trials[-1][2])
     finally:
         for sub in scratch:
             sub.free()
-    cache.put(key, {"hdiff": h, "vadv": v, "seconds": seconds, "trials": len(trials)})
-    return TuneResult(key, h, v, seconds, False, trials)
+    cache.put(key, {"hdiff": h, "vadv": v, "seconds": seconds, "trials": len(trials),
+                    "defaults": defaults})
+    return TuneResult(key, h, v, seconds, False, trials, defaults)
 
 
 def tune_hdiff(domain, storage, compute=None, halo=(3, 3, 3), cache=None, repeats=3,
