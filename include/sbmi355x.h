@@ -133,18 +133,20 @@ int sb_flush_caches(void);
  * Computations of the generated basic kernels
  * (stencils/cuda_hip/basic.py:101-132, templates/basic_1d.j2, basic_3d.j2),
  * interior points only, with the arithmetic order of the verification
- * oracles (stencils/base.py:180-254).  Launch options (averages and
- * Laplacian): ->variant 0 default, 1 row kernel (->by = rows per workgroup
- * 4/8/16), 2 marching kernel (a thread walks ->bz = 8/16/32/64 rows of the
+ * oracles (stencils/base.py:180-254).  Launch options: ->variant 0 default,
+ * 1 row kernel (->by = rows per workgroup 4/8/16), 2 marching kernel
+ * (averages and Laplacian: a thread walks ->bz = 8/16/32/64 rows of the
  * second-smallest-stride axis keeping three rows in registers; needs
  * 16-byte vector access along the unit-stride axis and no term along the
  * largest-stride axis), 3 (sb_laplacian only: SB_F64 with terms along x and
- * y only, si == 1, 0 < sj with a row pitch below 16 MiB, nx a multiple of 64 and ny of
- * ->by) LDS-DMA tile: a
- * 64 x ->by tile (8/16/32 rows, 0 = 16 where ny allows, else 8) of one
- * k-plane per workgroup, staged by global-to-LDS loads.  The default is 3
- * where it applies and no ->by/->bz is given, else marches where a term lies
- * along the second axis. */
+ * y only, si == 1, 0 < sj with a row pitch below 16 MiB, nx a multiple of 64
+ * and ny of ->by) LDS-DMA tile: a 64 x ->by tile (8/16/32 rows, 0 = 16 where
+ * ny allows, else 8) of one k-plane per workgroup, staged by global-to-LDS
+ * loads.  The default without ->by/->bz is 3 where it applies to fields of more
+ * than 256 MB together, else the packed kernel (rows packed over the lanes,
+ * any alignment, non-temporal stores) where one axis has unit stride and, for
+ * sb_laplacian, strides grow from x to z; otherwise it marches where a term
+ * lies along the second axis and takes the row kernel where none does. */
 int sb_copy(int prec, const void *inp, void *out, const sb_geom *g,
             const sb_launch *l, double *seconds);
 /* out = (inp[x + e_axis] + inp[x]) / 2 (base.py:191-205). */

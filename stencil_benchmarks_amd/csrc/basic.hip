@@ -2,7 +2,11 @@
 // Laplacian.
 //
 // The host permutes the three logical axes so that kernel axis 0 is the one
-// with unit stride.  Each thread computes V consecutive points along it:
+// with unit stride.  Four kernels: the packed kernel, default wherever it fits;
+// the row kernel, for any strides; the marching kernel; and an LDS tile for
+// the FP64 Laplacian along i and j.
+//
+// Row kernel: each thread computes V consecutive points along axis 0:
 // the centre and the off-axis neighbours are V-wide aligned vector loads
 // (one dwordx4 for V*sizeof(T) == 16), the two along-axis neighbours that
 // fall outside the vector are scalar loads, the rest are register shuffles.
@@ -272,7 +276,150 @@ __global__ __launch_bounds__(BLOCK) void march_kernel(const T *__restrict__ inp,
     }
 }
 
-// Laplacian along i and j in FP64 (variant 3, default where it applies): a
+// Packed kernel: the lanes of a plane are its vectors of 16 bytes in order,
+// rows packed one after the other, so no lane idles whatever the row length.
+// A row's last vector ends at the row's last point and overlaps the one before
+// (both store the same values).  Vectors need no alignment beyond the
+// element's: global loads and stores of 16 bytes take any 4-byte aligned
+// address.  AXES says along which (permuted) axes the stencil reads
+// neighbours; along axis 0 that is two more loads of one element beside each
+// vector, along the others RPT points of a lane share what they load.  Those
+// lie along axis 2 where the stencil reads neighbours there, else along axis 1.
+// Stores are non-temporal: the output is not read back, and left in the caches
+// it pushes out input rows that neighbouring runs still need.
+//
+// HBM bounds it: 333x517x79 with float32 and a term along every axis takes
+// 21 us (the bytes of one read and one write at 6.1 TB/s: 18 us) where the row
+// kernel took 62; the copy of 401x400x137 without padding 28 us (floor 29) and
+// 62; 1024x1024x80 in FP64 the copy 218 us (floor 220) and 226-256, the Laplacian
+// along all axes 325 us and 479-509.  What is left is input fetched twice along axis 2.
+struct PackedArgs {
+    int32_t n0, n1, n2;
+    uint32_t pitch;      // bytes of a row
+    int64_t plane;       // bytes of a plane
+    int32_t lanes;       // of a plane, or of a run of planes
+    UDiv vectors;        // by the vectors of a row
+    UDiv blocks;         // by the workgroups of a plane, or of a run of planes
+    TileGrid grid;       // XCD remap
+};
+
+template <typename T, int V>
+using PackedVec = T __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+
+template <typename T, typename C, int OP, int AXES, int V, int RPT>
+__global__ __launch_bounds__(BLOCK) void packed_kernel(const T *__restrict__ inp,
+                                                       T *__restrict__ out, PackedArgs a) {
+    using VT = PackedVec<T, V>;
+    using GP = __attribute__((address_space(1))) const char *;
+    using GO = __attribute__((address_space(1))) char *;
+    constexpr bool A0 = (AXES & 1) != 0, A1 = (AXES & 2) != 0, A2 = (AXES & 4) != 0;
+    constexpr bool MINUS = OP == OP_AVG2 || OP == OP_LAP;  // reads the lower neighbours too
+    const uint32_t b = remapped(blockIdx.x, a.grid);
+    const int32_t outer = int32_t(udiv(b, a.blocks));  // plane, or run of planes
+    const uint32_t block = b - uint32_t(outer) * a.blocks.d;
+    const int32_t lane = int32_t(block) * BLOCK + int32_t(threadIdx.x);
+    if (lane >= a.lanes) return;
+    const uint32_t line = udiv(uint32_t(lane), a.vectors);  // row, or run of rows
+    const int32_t i = min((lane - int32_t(line * a.vectors.d)) * V, a.n0 - V);
+    const int32_t j0 = A2 ? int32_t(line) : int32_t(line) * RPT;
+    const int32_t k0 = A2 ? outer * RPT : outer;
+    const uint32_t col = uint32_t(i + 1) * uint32_t(sizeof(T));
+    // offsets count from point (-1, -1) of a plane, so none is negative
+    const int64_t corner = -int64_t(a.pitch) - int64_t(sizeof(T));
+    // plane k0 + q and row j0 + q of the run.  Past the run's last point lies
+    // its upper neighbour, which is all that runs beyond the domain may read
+    auto plane = [&](int32_t q, int32_t end) {
+        return (GP)inp + (corner + int64_t(min(k0 + q, end)) * a.plane);
+    };
+    auto row = [&](int32_t q) {
+        return uint32_t(min(j0 + q, a.n1 - (A1 && !A2 ? 0 : 1)) + 1) * a.pitch + col;
+    };
+    const uint32_t last_row = uint32_t(a.n1) * a.pitch + col;
+    auto vec = [](GP base, uint32_t off) {
+        return *(__attribute__((address_space(1))) const VT *)(base + off);
+    };
+    auto one = [](GP base, uint32_t off) {
+        return *(__attribute__((address_space(1))) const T *)(base + off);
+    };
+    GP base[RPT];
+    uint32_t off[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        base[q] = plane(A2 ? q : 0, a.n2 - (A2 ? 0 : 1));
+        off[q] = row(A2 ? 0 : q);
+    }
+    // the run's points, the points before and after it, and beside a run along
+    // axis 2 the neighbours along axis 1
+    VT cv[RPT]{}, before{}, after{}, lo[RPT]{}, hi[RPT]{};
+    T left[RPT]{}, right[RPT]{};
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) cv[q] = vec(base[q], off[q]);
+    if constexpr (A2) {
+        if constexpr (MINUS) before = vec(plane(-1, a.n2), off[0]);
+        after = vec(plane(RPT, a.n2), off[0]);
+        if constexpr (A1) {
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const GP own = plane(q, a.n2 - 1);
+                hi[q] = vec(own, off[q] + a.pitch);
+                if constexpr (MINUS) lo[q] = vec(own, off[q] - a.pitch);
+            }
+        }
+    } else if constexpr (A1) {
+        if constexpr (MINUS) before = vec(base[0], row(-1));
+        after = vec(base[0], row(RPT));
+    }
+    if constexpr (A0) {
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            const GP own = A2 ? plane(q, a.n2 - 1) : base[q];
+            const uint32_t at = A1 && !A2 ? min(off[q], last_row) : off[q];
+            right[q] = one(own, at + uint32_t(V * sizeof(T)));
+            if constexpr (MINUS) left[q] = one(own, at - uint32_t(sizeof(T)));
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        VT res;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const C c = C(cv[q][e]);
+            // upper and lower neighbour along axis 0, along the run and, beside
+            // a run along axis 2, along axis 1
+            C p0 = C(0), m0 = C(0), pr = C(0), mr = C(0), p1 = C(0), m1 = C(0);
+            if constexpr (A0) {
+                p0 = e + 1 < V ? C(cv[q][e + 1 < V ? e + 1 : e]) : C(right[q]);
+                if constexpr (MINUS) m0 = e > 0 ? C(cv[q][e > 0 ? e - 1 : e]) : C(left[q]);
+            }
+            if constexpr (A1 || A2) {
+                pr = q + 1 < RPT ? C(cv[q + 1 < RPT ? q + 1 : q][e]) : C(after[e]);
+                if constexpr (MINUS) mr = q > 0 ? C(cv[q > 0 ? q - 1 : q][e]) : C(before[e]);
+            }
+            if constexpr (A1 && A2) {
+                p1 = C(hi[q][e]);
+                if constexpr (MINUS) m1 = C(lo[q][e]);
+            }
+            C value;
+            if constexpr (OP == OP_COPY) {
+                value = c;
+            } else if constexpr (OP == OP_LAP) {
+                value = C(0);
+                if constexpr (A0) value += (C(2) * c - p0) - m0;
+                if constexpr (A1 && A2) value += (C(2) * c - p1) - m1;
+                if constexpr (A1 || A2) value += (C(2) * c - pr) - mr;
+            } else {
+                value = ((A0 ? p0 : pr) + (OP == OP_AVG1 ? c : A0 ? m0 : mr)) / C(2);
+            }
+            res[e] = T(value);
+        }
+        if (A2 ? k0 + q < a.n2 : j0 + q < a.n1) {
+            const GO to = (GO)out + (corner + int64_t(k0 + (A2 ? q : 0)) * a.plane);
+            __builtin_nontemporal_store(res, (__attribute__((address_space(1))) VT *)(to + off[q]));
+        }
+    }
+}
+
+// Laplacian along i and j in FP64 (variant 3, default for large fields): a
 // 64 x TY tile of one k-plane per workgroup, its (64+2) x (TY+2) input tile
 // staged straight into LDS by 4-byte global-to-LDS loads (one contiguous LDS
 // array; wave instruction n stages dwords 64n .. 64n+63 of it, so the tile's
@@ -350,6 +497,76 @@ hipError_t launch_lap_dma(const double *inp, double *out, const sb_geom *g, Cont
     return hipGetLastError();
 }
 
+// Points of a run.  Along axis 1, four; without neighbours along axes 1 and 2,
+// none to share.  Along axis 2 a run's lanes also wait for more planes at once,
+// measured at 333x517x79 to 1024x1024x80:
+//   one-sided average   2 (FP64, us): 41 and 250; 4: 43 and 251; 8: 45 and 251
+//   only along axis 2   8: 44 and 247; 4: 43 and 290; 2: 48 and 313
+//   all axes            8 points of a lane, so two vectors of float32 (21 and
+//                       182; four: 24 and 186) and four of FP64 (56 and 332;
+//                       two: 56 and 364)
+template <int OP, int AXES, int V>
+constexpr int packed_run() {
+    if (AXES & 4) return OP == OP_AVG1 ? 2 : (AXES & 2) ? (V == 4 ? 2 : 4) : 8;
+    return (AXES & 2) ? 4 : 1;
+}
+
+template <typename T, typename C, int OP, int AXES, int V>
+hipError_t launch_packed(const T *inp, T *out, const BasicArgs &b, Context *ctx) {
+    constexpr bool A2 = (AXES & 4) != 0;
+    constexpr int RPT = packed_run<OP, AXES, V>();
+    PackedArgs a{};
+    a.n0 = int32_t(b.n[0]);
+    a.n1 = int32_t(b.n[1]);
+    a.n2 = int32_t(b.n[2]);
+    a.pitch = uint32_t(b.s[1] * int64_t(sizeof(T)));
+    a.plane = b.s[2] * int64_t(sizeof(T));
+    const uint32_t vectors = uint32_t((b.n[0] + V - 1) / V);
+    const uint32_t lines = uint32_t(A2 ? b.n[1] : (b.n[1] + RPT - 1) / RPT);
+    const uint32_t outers = uint32_t(A2 ? (b.n[2] + RPT - 1) / RPT : b.n[2]);
+    a.vectors = make_udiv(vectors);
+    a.lanes = int32_t(vectors * lines);
+    const uint32_t blocks = uint32_t((a.lanes + BLOCK - 1) / BLOCK);
+    a.blocks = make_udiv(blocks);
+    const uint64_t total = uint64_t(blocks) * uint64_t(outers);
+    if (total >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
+    a.grid = make_tile_grid(uint32_t(total), 1, 1, ctx->xcds);
+    enqueue_kernel((packed_kernel<T, C, OP, AXES, V, RPT>), dim3(uint32_t(total)), dim3(BLOCK), 0,
+                   ctx->stream, inp, out, a);
+    return hipGetLastError();
+}
+
+template <typename T, typename C, int OP, int AXES = 7>
+hipError_t launch_packed_axes(int axes, bool wide, const T *inp, T *out, const BasicArgs &b,
+                              Context *ctx) {
+    if constexpr (AXES > 0)
+        if (axes != AXES)
+            return launch_packed_axes<T, C, OP, AXES - 1>(axes, wide, inp, out, b, ctx);
+    constexpr bool used = OP == OP_COPY ? AXES == 0
+                          : OP == OP_LAP ? AXES > 0 : AXES == 1 || AXES == 2 || AXES == 4;
+    if constexpr (used)
+        return wide ? launch_packed<T, C, OP, AXES, int(16 / sizeof(T))>(inp, out, b, ctx)
+                    : launch_packed<T, C, OP, AXES, 1>(inp, out, b, ctx);
+    else
+        return hipErrorInvalidValue;
+}
+
+// Whether the packed kernel takes this call, its default: unit stride along
+// axis 0, rows upwards, offsets of a plane and its neighbour rows below 4 GiB,
+// indexes of lanes and workgroups below 2^31, and for the Laplacian, whose
+// terms are summed in the order i, j, k, axes in that order of strides.  The
+// other kernels were slower at every size measured, from 32x32x80 up
+// (128x128x80 FP64 average along j: 6.5 us against 5.0).
+bool packed_fits(const BasicArgs &a, int op) {
+    const double rows = double(a.n[1]), row = double(a.n[0]);
+    return a.s[0] == 1 && a.s[1] > 0 &&
+           ((rows + 9) * double(a.s[1]) + row + 9) * 8.0 < 4294967296.0 &&
+           row * (rows + 9) < 1073741824.0 &&
+           (row * (rows + 9) / BLOCK + 1) * double(a.n[2]) < 2147483648.0 &&
+           (op == OP_COPY || op == OP_AVG1 || op == OP_AVG2 ||
+            (a.lap_mask && a.perm[0] < a.perm[1] && a.perm[1] < a.perm[2]));
+}
+
 template <int P, int OP>
 int launch_basic_prec(const void *inp_v, void *out_v, const sb_geom *g, int axis, int lap_mask,
                       const sb_launch *l, double *seconds) {
@@ -397,11 +614,12 @@ int launch_basic_prec(const void *inp_v, void *out_v, const sb_geom *g, int axis
     if (!ctx) return 1;
     a.xcds = ctx->xcds;
     // launch->variant: 0 default, 1 the row kernel, 2 the marching kernel.
-    // The marching kernel needs vector access along axis 0 and no term along
-    // axis 2; by default it runs where a term lies along axis 1, whose rows
-    // it reuses (measured on MI355X, 512x512x160 FP64: Laplacian ij 3.72 ->
-    // 4.76 TB/s); with terms along axis 0 only the row kernel is faster
-    // (more workgroups in flight, nothing to reuse).
+    // The default is the packed kernel wherever it fits and no row option asks
+    // for one of the others.  The marching kernel needs vector access along
+    // axis 0 and no term along axis 2; of the two it is the default where a
+    // term lies along axis 1, whose rows it reuses (512x512x160 FP64,
+    // Laplacian ij: 4.76 TB/s, row kernel 3.72); with terms along axis 0 only
+    // the row kernel is faster (more workgroups in flight, nothing to reuse).
     bool marchable = OP != OP_COPY && V > 1, axis1 = false;
     if constexpr (OP == OP_LAP) {
         for (int o = 0; o < 3; ++o) {
@@ -414,18 +632,23 @@ int launch_basic_prec(const void *inp_v, void *out_v, const sb_geom *g, int axis
     }
     const int variant = l ? l->variant : 0;
     SB_REQUIRE(variant >= 0 && variant <= 3, "basic stencil variant %d not in {0, 1, 2, 3}", variant);
+    const bool row_options = l && (l->by || l->bz);
     // launch->variant 3: the LDS-DMA Laplacian (FP64, terms along i and j,
     // unit i stride, whole 64 x by tiles; launch->by = tile rows 8, 16 or 32,
-    // 0 = 16 where ny allows, else 8), the default for such calls without
-    // row options.  512x512x160: 107 us with 16 rows, 110 us with 32, 125 us
-    // with 8, against 131 us for the marching kernel.
+    // 0 = 16 where ny allows, else 8), the default for such calls without row
+    // options on two fields that together exceed the 256 MB last-level cache.
+    // Per launch, 512x512x160 takes 108 us with 16 rows, 110 us with 32, 125 us
+    // with 8, 122 us on the packed kernel and 131 us on the marching kernel;
+    // 2048x2048x40 back to back 464 us, packed 479.  Smaller fields are bound
+    // by the tile's 4-byte staging instead: 512x512x40 35 us, packed 25;
+    // 256x256x80 18.6 us, packed 13.6.
     constexpr bool lap64 = OP == OP_LAP && std::is_same_v<T, double> && std::is_same_v<C, double>;
     SB_REQUIRE(variant != 3 || lap64,
                "basic stencil variant 3 (LDS-DMA tile) takes FP64 Laplacians only");
     if constexpr (lap64) {
         const int ty = (l && l->by) ? l->by : (g->ny % 16 == 0 ? 16 : 8);
-        const bool row_options = l && (l->by || l->bz);
-        if (variant == 3 || (variant == 0 && !row_options && lap_dma_fits(g, lap_mask, ty))) {
+        const bool streams = 2 * a.n[0] * a.n[1] * a.n[2] * int64_t(sizeof(T)) > (int64_t(256) << 20);
+        if (variant == 3 || (variant == 0 && !row_options && streams && lap_dma_fits(g, lap_mask, ty))) {
             SB_REQUIRE(ty == 8 || ty == 16 || ty == 32, "LDS-DMA Laplacian tile rows %d not in {8, 16, 32}",
                        ty);
             SB_REQUIRE(lap_dma_fits(g, lap_mask, ty),
@@ -438,6 +661,13 @@ int launch_basic_prec(const void *inp_v, void *out_v, const sb_geom *g, int axis
                 return launch_lap_dma<32, 8>(inp, out, g, ctx);
             });
         }
+    }
+    if (variant == 0 && !row_options && packed_fits(a, OP)) {
+        const int axes = OP == OP_LAP ? lap_mask : OP == OP_COPY ? 0 : 1 << a.axis;
+        const bool wide = a.n[0] >= int64_t(16 / sizeof(T));
+        return timed_launch(l, seconds, [&]() -> hipError_t {
+            return launch_packed_axes<T, C, OP>(axes, wide, inp, out, a, ctx);
+        });
     }
     SB_REQUIRE(variant != 2 || marchable,
                "the marching kernel needs vector access along the unit-stride axis and no "

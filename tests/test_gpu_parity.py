@@ -148,6 +148,41 @@ def test_basic_stencil_kernels(gpu, prec, domain, variant, rows):
         _check_halo(got, domain, halo)
 
 
+# rows of less, of exactly and of just over one or two 16-byte vectors; rows and
+# planes around the run lengths 2, 4 and 8; several workgroups with a ragged last one
+PACKED_DOMAINS = [(1, 5, 9), (2, 4, 8), (3, 3, 7), (4, 2, 6), (5, 1, 1), (7, 9, 17), (8, 8, 16),
+                  (9, 7, 2), (67, 21, 4), (515, 6, 11)]
+
+
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("alignment", [0, 64])
+@pytest.mark.parametrize("domain", PACKED_DOMAINS)
+def test_basic_stencils_packed(gpu, prec, alignment, domain):
+    """The default kernel on tight halos against the oracle and, bit for bit
+    over the whole field, the row kernel (variant 1)."""
+    dtype = _dtype(prec)
+    code = _prec(gpu, prec)
+    cases = [("sb_copy", (), (0, 0, 0), oracle.copy, ())]
+    for axis in range(3):
+        halo = tuple(int(axis == a) for a in range(3))
+        cases.append(("sb_onesided_average", (axis,), halo, oracle.onesided_average, (axis,)))
+        cases.append(("sb_symmetric_average", (axis,), halo, oracle.symmetric_average, (axis,)))
+    for bits in range(1, 8):
+        mask = tuple(bits >> a & 1 for a in range(3))
+        cases.append(("sb_laplacian", mask, mask, oracle.laplacian, (mask,)))
+    for entry, extra, halo, func, args in cases:
+        inp, = make_fields(domain, halo, dtype, (2, 1, 0), alignment, seed=sum(domain))
+        got = []
+        for variant in (0, 1):
+            out = _with_sentinel(make_fields(domain, halo, dtype, (2, 1, 0), alignment)[0])
+            got += _run(gpu, entry, [inp, out], [1], domain, halo, code, *extra,
+                        launch=gpu.launch_options(variant=variant))
+        expected = _expected(lambda f: func(f, *args, domain, halo), [inp], prec)
+        assert np.array_equal(got[0][inner(domain, halo)], expected), (entry, extra)
+        assert np.array_equal(got[0], got[1]), (entry, extra)
+        _check_halo(got[0], domain, halo)
+
+
 def test_marching_kernel_rejects_axis_2_terms(gpu):
     from stencil_benchmarks_amd.benchmark import ExecutionError
 
