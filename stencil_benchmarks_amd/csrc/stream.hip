@@ -200,10 +200,9 @@ constexpr size_t kMaxGridYZ = 65535;
 
 template <typename T, int OP, int V, int U>
 int launch_stream(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *l,
-                  double *seconds, int block, int per_cu, int axis) {
+                  double *seconds, int block, int per_cu, int axis, int nt) {
     const size_t nvec = n / V;
     const size_t pass = size_t(U) * block;
-    const int nt = l ? (l->variant & 3) : 0;
     Context *ctx = context();
     if (!ctx) return 1;
     size_t blocks = (nvec + pass - 1) / pass;
@@ -243,24 +242,31 @@ int launch_stream(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *l,
 
 template <typename T, int OP, int V>
 int dispatch_unroll(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *l,
-                    double *seconds, int block, int per_cu, int axis) {
-    const int unroll = (l && l->unroll) ? l->unroll : 4;
+                    double *seconds, int block, int per_cu, int axis, int nt, int unroll) {
     switch (unroll) {
-        case 1: return launch_stream<T, OP, V, 1>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
-        case 2: return launch_stream<T, OP, V, 2>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
-        case 4: return launch_stream<T, OP, V, 4>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
-        case 8: return launch_stream<T, OP, V, 8>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
+        case 1: return launch_stream<T, OP, V, 1>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt);
+        case 2: return launch_stream<T, OP, V, 2>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt);
+        case 4: return launch_stream<T, OP, V, 4>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt);
+        case 8: return launch_stream<T, OP, V, 8>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt);
         default: set_error("STREAM unroll %d not in {1, 2, 4, 8}", unroll); return 2;
     }
 }
 
 // launch->by: elements per vector (0: 16 bytes), ->bz: workgroups per CU of
 // a persistent grid (0: one pass over the arrays), ->variant bits 2-3: the
-// grid axis (0 x, 1 y, 2 z).
+// grid axis (0 x, 1 y, 2 z).  A shape that the caller leaves open altogether
+// is one 16-byte vector per thread, 1024 threads and non-temporal accesses:
+// HBM bounds it, and the streamed lines gain nothing from the caches.  2^27
+// FP64 elements: triad 563 -> 492 us (6.55 TB/s), copy 367 -> 340, against the
+// 256 threads of four vectors and plain accesses that were taken before; those
+// with the same hints take 505 and 335, one vector of 256 threads 499 and 367.
 template <typename T, int OP>
 int dispatch_vector(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *l,
                     double *seconds) {
-    const int block = (l && l->bx) ? l->bx : 256;
+    const bool open = !l || !(l->variant || l->bx || l->by || l->bz || l->unroll);
+    const int nt = open ? 3 : l->variant & 3;
+    const int unroll = open ? 1 : l->unroll ? l->unroll : 4;
+    const int block = open ? 1024 : l->bx ? l->bx : 256;
     SB_REQUIRE(block >= 64 && block <= 1024 && block % 64 == 0,
                "STREAM block size %d must be a multiple of 64 in [64, 1024]", block);
     constexpr int kWide = int(16 / sizeof(T));
@@ -273,11 +279,11 @@ int dispatch_vector(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *
         SB_REQUIRE(reinterpret_cast<uintptr_t>(p) % (size_t(vec) * sizeof(T)) == 0,
                    "STREAM arrays must be aligned to the vector size");
     switch (vec) {
-        case 1: return dispatch_unroll<T, OP, 1>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
-        case 2: return dispatch_unroll<T, OP, 2>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
+        case 1: return dispatch_unroll<T, OP, 1>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt, unroll);
+        case 2: return dispatch_unroll<T, OP, 2>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt, unroll);
         case 4:
             if constexpr (sizeof(T) == 4)
-                return dispatch_unroll<T, OP, 4>(a, b, c, n, scalar, l, seconds, block, per_cu, axis);
+                return dispatch_unroll<T, OP, 4>(a, b, c, n, scalar, l, seconds, block, per_cu, axis, nt, unroll);
             [[fallthrough]];
         default:
             set_error("STREAM vector size %d not in {1, %d} elements of %zu bytes", vec, kWide,

@@ -641,6 +641,35 @@ def test_stream_kernels(gpu, dtype, op, unroll, nt, vector, per_cu, axis):
         assert np.array_equal(g, e)
 
 
+# around one workgroup of 1024 vectors of 2 (FP64) or 4 (float32) elements
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("n", [1, 3, 2047, 2048, 2050, 4097, 100003])
+def test_stream_default_shape(gpu, dtype, n):
+    from stencil_benchmarks_amd.device import DeviceBuffer
+
+    code = gpu.SB_F64 if dtype == "float64" else gpu.SB_F32
+    host = [np.random.default_rng(q).random(n + 8).astype(dtype) for q in range(3)]
+    bufs = [DeviceBuffer(h.nbytes) for h in host]
+    s = np.dtype(dtype).type(3.0)
+    for op, written, func in (("copy", 2, lambda a, b, c: a), ("scale", 1, lambda a, b, c: s * c),
+                              ("add", 2, lambda a, b, c: a + b),
+                              ("triad", 0, lambda a, b, c: b + s * c)):
+        for b, h in zip(bufs, host):
+            gpu.call("sb_memcpy_h2d", ctypes.c_void_p(b.ptr), ctypes.c_void_p(h.ctypes.data),
+                     h.nbytes)
+        gpu.call("sb_stream_kernel", code, gpu.STREAM_OPS[op],
+                 *[ctypes.c_void_p(b.ptr) for b in bufs], n, 3.0, gpu.launch_options(), None)
+        gpu.call("sb_synchronize")
+        for q, (b, h) in enumerate(zip(bufs, host)):
+            out = np.empty_like(h)
+            gpu.call("sb_memcpy_d2h", ctypes.c_void_p(out.ctypes.data), ctypes.c_void_p(b.ptr),
+                     h.nbytes)
+            expected = h.copy()
+            if q == written:
+                expected[:n] = func(*[x[:n] for x in host])
+            assert np.array_equal(out, expected), (op, q)
+
+
 def test_stream_rejects_bad_shapes(gpu):
     from stencil_benchmarks_amd.benchmark import ExecutionError
     from stencil_benchmarks_amd.device import DeviceBuffer
