@@ -113,6 +113,10 @@ int sb_host_free(void *ptr);
 int sb_memcpy_h2d(void *dst, const void *src, size_t bytes);
 int sb_memcpy_d2h(void *dst, const void *src, size_t bytes);
 int sb_memcpy_d2d(void *dst, const void *src, size_t bytes);
+/* Asynchronously (ordered as kernels are): dst[(i ny + j) nz + k] = point
+ * (i, j, k) of the interior whose origin is `src`, in the storage type of
+ * prec; dst holds nx ny nz elements and does not overlap the interior. */
+int sb_pack_interior(int prec, const void *src, void *dst, const sb_geom *g);
 int sb_memset(void *dst, int value, size_t bytes);
 int sb_synchronize(void);
 /* Markers on the library stream (the reference times with events inside the

@@ -115,6 +115,19 @@ class Subdomain:
         """Current u (after the steps run so far)."""
         return self.download(f"u{self.parity}")
 
+    def take_interior(self, name, scratch):
+        """The interior of field `name` as a C-ordered host array, by way of
+        field `scratch`, whose contents are given up.  Packed on the device,
+        only the interior crosses the link, and no array of the field's own
+        order is turned on the host (which took most of a retirement)."""
+        out = np.empty(self.domain, self.dtype)
+        via = self.fields[scratch].base
+        native.call("sb_pack_interior", native.precision_code(self.dtype, self.dtype),
+                    ctypes.c_void_p(self.fields[name].pointer()), ctypes.c_void_p(via), self.geom)
+        native.call("sb_memcpy_d2h", ctypes.c_void_p(out.ctypes.data), ctypes.c_void_p(via),
+                    out.nbytes)
+        return out
+
     def struct(self):
         f = self.fields
         s = SubdomainStruct()

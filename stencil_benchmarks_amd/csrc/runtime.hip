@@ -1,6 +1,12 @@
 // Library lifecycle, errors, device memory and cache flushing.
+#include <sched.h>
+
+#include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "sb_internal.h"
@@ -31,6 +37,141 @@ __global__ __launch_bounds__(256) void flush_kernel(uint4 *buf, size_t n) {
         acc.w ^= v.w;
     }
     if ((acc.x & acc.y & acc.z & acc.w) == 0xFFFFFFFFu) buf[0] = acc;
+}
+
+// Device-to-host copies into pageable memory.  One thread gets 17 GB/s of the
+// link's 54 (100 MiB: 5.8 ms, into pinned memory 1.85), and 10 GB/s into memory
+// that has not been touched yet: copying out of a staging buffer and the page
+// faults of the destination take the rest.  From kStagedBytes on, workers
+// therefore take kPieceBytes at a time through a pinned buffer of their own,
+// so one worker's copy and faults run beside the others' and beside the link:
+// 100 MiB in 2.7 ms (5.8 before), untouched 3.1 (9.7).  Pieces of 1 MiB take
+// 3.4 ms, eight workers gain 0.2 ms.
+constexpr size_t kPieceBytes = size_t(2) << 20;
+constexpr int kMaxWorkers = 4;
+constexpr size_t kStagedBytes = 2 * kPieceBytes;
+
+// Pinned buffers of one device's workers, allocated at its first large copy
+// and kept (8 MiB); a copy that finds them in use takes the direct way.
+struct Staging {
+    std::mutex busy;
+    char *piece[kMaxWorkers] = {};
+    hipEvent_t done[kMaxWorkers] = {};
+};
+constexpr int kMaxDevices = 64;
+Staging g_staging[kMaxDevices];
+
+int usable_cpus() {
+    cpu_set_t set;
+    CPU_ZERO(&set);
+    return sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+}
+
+// Copies pieces drawn from `next` until none is left or a copy fails.
+void copy_pieces(int device, hipStream_t stream, char *piece, hipEvent_t done, char *dst,
+                 const char *src, size_t bytes, std::atomic<size_t> *next,
+                 std::atomic<int> *error) {
+    if (const hipError_t e = hipSetDevice(device); e != hipSuccess) error->store(int(e));
+    for (;;) {
+        const size_t at = next->fetch_add(kPieceBytes);
+        if (at >= bytes || error->load() != hipSuccess) return;
+        const size_t n = std::min(kPieceBytes, bytes - at);
+        hipError_t e = hipMemcpyAsync(piece, src + at, n, hipMemcpyDeviceToHost, stream);
+        if (e == hipSuccess) e = hipEventRecord(done, stream);
+        if (e == hipSuccess) e = hipEventSynchronize(done);
+        if (e != hipSuccess) {
+            error->store(int(e));
+            return;
+        }
+        std::memcpy(dst + at, piece, n);
+    }
+}
+
+// Whether the staged way took the copy (`status` its result).
+bool staged_download(Context *ctx, void *dst, const void *src, size_t bytes, int *status) {
+    if (bytes < kStagedBytes || ctx->device >= kMaxDevices) return false;
+    hipPointerAttribute_t where;
+    if (hipPointerGetAttributes(&where, dst) != hipSuccess)
+        (void)hipGetLastError();  // pageable memory: unknown to the runtime
+    else if (where.type != hipMemoryTypeUnregistered)
+        return false;
+    Staging &s = g_staging[ctx->device];
+    std::unique_lock<std::mutex> lock(s.busy, std::try_to_lock);
+    if (!lock.owns_lock()) return false;
+    const int want = int(std::min<size_t>({size_t(kMaxWorkers), bytes / kPieceBytes,
+                                           size_t(std::max(1, usable_cpus() / 2))}));
+    if (want < 2) return false;
+    for (int w = 0; w < want; ++w) {
+        if (!s.piece[w] && hipHostMalloc(reinterpret_cast<void **>(&s.piece[w]), kPieceBytes,
+                                         hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            s.piece[w] = nullptr;
+            return false;
+        }
+        if (!s.done[w] && hipEventCreateWithFlags(&s.done[w], hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            s.done[w] = nullptr;
+            return false;
+        }
+    }
+    std::atomic<size_t> next{0};
+    std::atomic<int> error{hipSuccess};
+    std::thread workers[kMaxWorkers];
+    for (int w = 1; w < want; ++w) {
+        try {
+            workers[w] = std::thread(copy_pieces, ctx->device, ctx->stream, s.piece[w], s.done[w],
+                                     static_cast<char *>(dst), static_cast<const char *>(src),
+                                     bytes, &next, &error);
+        } catch (const std::system_error &) {
+            break;  // no more threads: the others take its pieces
+        }
+    }
+    copy_pieces(ctx->device, ctx->stream, s.piece[0], s.done[0], static_cast<char *>(dst),
+                static_cast<const char *>(src), bytes, &next, &error);
+    for (std::thread &worker : workers)
+        if (worker.joinable()) worker.join();
+    *status = 0;
+    if (error.load() != hipSuccess) {
+        set_error("copy to the host: %s", hipGetErrorString(hipError_t(error.load())));
+        *status = 1;
+    }
+    return true;
+}
+
+// Interior of a field, any strides, packed to C order: a 32 x 32 tile of axes
+// i and k at one j per workgroup, turned in LDS so that both sides are
+// accessed along their own contiguous axis.
+template <typename T>
+__global__ __launch_bounds__(256) void pack_kernel(const T *__restrict__ src, T *__restrict__ dst,
+                                                   int64_t nx, int64_t ny, int64_t nz, int64_t si,
+                                                   int64_t sj, int64_t sk, uint32_t tiles_i,
+                                                   uint32_t tiles_k) {
+    __shared__ T tile[32][33];
+    const uint32_t plane = blockIdx.x / tiles_i;
+    const int64_t i0 = int64_t(blockIdx.x - plane * tiles_i) * 32;
+    const int64_t j = plane / tiles_k;
+    const int64_t k0 = int64_t(plane - uint32_t(j) * tiles_k) * 32;
+    const int x = threadIdx.x % 32, y = threadIdx.x / 32;
+    for (int r = y; r < 32; r += 8)
+        if (i0 + x < nx && k0 + r < nz)
+            tile[r][x] = src[(i0 + x) * si + j * sj + (k0 + r) * sk];
+    __syncthreads();
+    for (int r = y; r < 32; r += 8)
+        if (i0 + r < nx && k0 + x < nz) dst[((i0 + r) * ny + j) * nz + k0 + x] = tile[x][r];
+}
+
+template <typename T>
+int pack_interior(const void *src, void *dst, const sb_geom *g, Context *ctx) {
+    const int64_t ti = (g->nx + 31) / 32, tk = (g->nz + 31) / 32;
+    if (g->nx == 0 || g->ny == 0 || g->nz == 0) return 0;
+    SB_REQUIRE(src && dst, "NULL field pointer");
+    SB_REQUIRE(double(ti) * double(tk) * double(g->ny) < 2147483648.0,
+               "domain too large for one launch");
+    enqueue_kernel(pack_kernel<T>, dim3(unsigned(ti * tk * g->ny)), dim3(256), 0, ctx->stream,
+                   static_cast<const T *>(src), static_cast<T *>(dst), g->nx, g->ny, g->nz, g->si,
+                   g->sj, g->sk, uint32_t(ti), uint32_t(tk));
+    SB_HIP(hipGetLastError());
+    return 0;
 }
 
 int init_context(Context &c, int device) {
@@ -230,11 +371,23 @@ int sb_memcpy_h2d(void *dst, const void *src, size_t bytes) {
 }
 
 int sb_memcpy_d2h(void *dst, const void *src, size_t bytes) {
+    Context *ctx = context();
+    int status = 0;
+    if (ctx && dst && src && staged_download(ctx, dst, src, bytes, &status)) return status;
     return copy_sync(dst, src, bytes, hipMemcpyDeviceToHost);
 }
 
 int sb_memcpy_d2d(void *dst, const void *src, size_t bytes) {
     return copy_sync(dst, src, bytes, hipMemcpyDeviceToDevice);
+}
+
+int sb_pack_interior(int prec, const void *src, void *dst, const sb_geom *g) {
+    SB_REQUIRE(prec == SB_F64 || prec == SB_F32 || prec == SB_F32_F64, "invalid precision %d", prec);
+    if (check_geom(g, 0, 0, 0)) return 2;
+    Context *ctx = context();
+    if (!ctx) return 1;
+    return prec == SB_F64 ? pack_interior<double>(src, dst, g, ctx)
+                          : pack_interior<float>(src, dst, g, ctx);
 }
 
 int sb_memset(void *dst, int value, size_t bytes) {

@@ -79,6 +79,7 @@ SIGNATURES = {
     "sb_memcpy_h2d": [_P, _P, _SZ],
     "sb_memcpy_d2h": [_P, _P, _SZ],
     "sb_memcpy_d2d": [_P, _P, _SZ],
+    "sb_pack_interior": [_I, _P, _P, _GP],
     "sb_memset": [_P, _I, _SZ],
     "sb_synchronize": [],
     "sb_event_create": [ctypes.POINTER(_P)],

@@ -118,3 +118,47 @@ def test_poisson_stream_shape():
     gaps = np.diff([0.0] + [r.arrival for r in reqs])
     assert abs(gaps.mean() - 0.01) < 0.002
     assert 1 <= min(r.steps for r in reqs) and max(r.steps for r in reqs) <= 20
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("domain,layout", [((1, 1, 1), (2, 1, 0)), ((33, 31, 40), (2, 1, 0)),
+                                           ((32, 2, 65), (0, 1, 2)), ((64, 5, 33), (1, 2, 0)),
+                                           ((200, 150, 60), (2, 1, 0))])
+def test_take_interior_equals_download(gpu, dtype, domain, layout):
+    from stencil_benchmarks_amd import batch
+
+    sub = batch.Subdomain(domain, (3, 2, 1), dtype, seed=5, layout=layout)
+    for name in ("u0", "wcon"):
+        expected = sub.download(name)[inner(domain, (3, 2, 1))]
+        got = sub.take_interior(name, "u1")
+        assert got.flags.c_contiguous and got.dtype == expected.dtype
+        assert np.array_equal(got, expected)
+    sub.free()
+
+
+# around the size from which pieces of 2 MiB go through pinned buffers, and whole and
+# ragged numbers of pieces beyond all workers'
+@pytest.mark.parametrize("nbytes", [0, 1, (4 << 20) - 1, 4 << 20, (4 << 20) + 1, 20 << 20,
+                                    (41 << 20) + 13])
+def test_download_of_any_size(gpu, nbytes):
+    import ctypes
+
+    from stencil_benchmarks_amd.device import DeviceBuffer
+
+    host = np.random.default_rng(nbytes).integers(0, 256, nbytes + 64, dtype=np.uint8)
+    buffer = DeviceBuffer(host.nbytes)
+    gpu.call("sb_memcpy_h2d", ctypes.c_void_p(buffer.ptr), ctypes.c_void_p(host.ctypes.data),
+             host.nbytes)
+    out = np.full(nbytes + 64, 7, np.uint8)
+    gpu.call("sb_memcpy_d2h", ctypes.c_void_p(out.ctypes.data + 5), ctypes.c_void_p(buffer.ptr + 3),
+             nbytes)
+    assert np.array_equal(out[5:nbytes + 5], host[3:nbytes + 3])
+    assert np.all(out[:5] == 7) and np.all(out[nbytes + 5:] == 7)
+    pinned = ctypes.c_void_p()
+    gpu.call("sb_host_malloc", ctypes.byref(pinned), nbytes + 1)
+    try:
+        gpu.call("sb_memcpy_d2h", pinned, ctypes.c_void_p(buffer.ptr), nbytes)
+        copied = np.ctypeslib.as_array((ctypes.c_uint8 * (nbytes + 1)).from_address(pinned.value))
+        assert np.array_equal(copied[:nbytes], host[:nbytes])
+    finally:
+        gpu.call("sb_host_free", pinned)
