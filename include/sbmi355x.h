@@ -239,7 +239,8 @@ int sb_vadv_noalloc(int prec, int all_components, void *const *fields,
  * per CU of a persistent grid (0: a grid covering the arrays once),
  * ->unroll = vectors per thread (0: 4), ->variant bit 0 = non-temporal
  * loads, bit 1 = non-temporal stores, bits 2-3 = grid axis 0 x, 1 y, 2 z;
- * all of them 0: 1024 threads, one vector each, non-temporal accesses
+ * all of them 0: 1024 threads, one vector each, non-temporal stores, and
+ * loads of more than 512 MB
  * (block_size / vector_size / unroll_factor / streaming_* / axis of
  * stream/cuda_hip.py:41-60). */
 int sb_stream_fill(int prec, void *x, size_t n, double value);

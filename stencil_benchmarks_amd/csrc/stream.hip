@@ -255,16 +255,24 @@ int dispatch_unroll(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *
 // launch->by: elements per vector (0: 16 bytes), ->bz: workgroups per CU of
 // a persistent grid (0: one pass over the arrays), ->variant bits 2-3: the
 // grid axis (0 x, 1 y, 2 z).  A shape that the caller leaves open altogether
-// is one 16-byte vector per thread, 1024 threads and non-temporal accesses:
-// HBM bounds it, and the streamed lines gain nothing from the caches.  2^27
-// FP64 elements: triad 563 -> 492 us (6.55 TB/s), copy 367 -> 340, against the
-// 256 threads of four vectors and plain accesses that were taken before; those
-// with the same hints take 505 and 335, one vector of 256 threads 499 and 367.
+// is one 16-byte vector per thread, 1024 threads and non-temporal stores, and
+// non-temporal loads too where the kernel's arrays take more than 512 MB.
+// HBM bounds it.  2^27 FP64 elements: triad 563 -> 492 us (6.55 TB/s), copy 367
+// -> 340, against the 256 threads of four vectors and plain accesses that were
+// taken before; those with the same hints take 505 and 335, one vector of 256
+// threads 499 and 367.  Arrays that fit in the 256 MB last-level cache are
+// found there by plain loads (non-temporal ones: 60 MB triad float32 10.7 ->
+// 12.1 us, 128 MB copy 20 -> 23); stores that leave them there gain too (128 MB
+// copies in turn 24.7 -> 19.9 us).  Between the two sizes it depends on what
+// ran before: 384 MB triad again and again 55 us with plain loads and 63 with
+// non-temporal ones, three in turn 69 and 64.
 template <typename T, int OP>
 int dispatch_vector(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *l,
                     double *seconds) {
     const bool open = !l || !(l->variant || l->bx || l->by || l->bz || l->unroll);
-    const int nt = open ? 3 : l->variant & 3;
+    constexpr size_t kWords = OP == SB_STREAM_COPY || OP == SB_STREAM_SCALE ? 2 : 3;
+    const bool streams = n > (size_t(512) << 20) / (kWords * sizeof(T));
+    const int nt = !open ? l->variant & 3 : streams ? 3 : 2;
     const int unroll = open ? 1 : l->unroll ? l->unroll : 4;
     const int block = open ? 1024 : l->bx ? l->bx : 256;
     SB_REQUIRE(block >= 64 && block <= 1024 && block % 64 == 0,

@@ -641,9 +641,11 @@ def test_stream_kernels(gpu, dtype, op, unroll, nt, vector, per_cu, axis):
         assert np.array_equal(g, e)
 
 
-# around one workgroup of 1024 vectors of 2 (FP64) or 4 (float32) elements
-@pytest.mark.parametrize("dtype", ["float64", "float32"])
-@pytest.mark.parametrize("n", [1, 3, 2047, 2048, 2050, 4097, 100003])
+# around one workgroup of 1024 vectors of 2 (FP64) or 4 (float32) elements, and
+# one past the 512 MB of three float32 arrays from which loads are non-temporal
+@pytest.mark.parametrize("dtype,n", [(dtype, n) for dtype in ("float64", "float32")
+                                     for n in (1, 3, 2047, 2048, 2050, 4097, 100003)]
+                         + [("float32", (512 << 20) // 12 + 1)])
 def test_stream_default_shape(gpu, dtype, n):
     from stencil_benchmarks_amd.device import DeviceBuffer
 
