@@ -357,7 +357,6 @@ __attribute__((amdgpu_waves_per_eu(RegBuilds<T, C>::of[BUILD].waves_per_simd)))
 void vadv_reg_batch_kernel(const SubDev *__restrict__ subs, const int32_t *__restrict__ ranks,
                            const int32_t *__restrict__ prefix, int count, uint32_t xcds) {
     extern __shared__ unsigned char lds_raw[];
-    CD<C> *lds = reinterpret_cast<CD<C> *>(lds_raw) + (threadIdx.x & 63);
     const int32_t item =
         int32_t(xcd_chunk_remap(blockIdx.x, gridDim.x, xcds, kRegItemsPerXcd));
     int lo = 0, hi = count;  // largest c with prefix[c] <= item
@@ -374,8 +373,8 @@ void vadv_reg_batch_kernel(const SubDev *__restrict__ subs, const int32_t *__res
                  own_rsrc(d.tens, d.span_bytes), own_rsrc(d.ts, d.span_bytes),
                  own_rsrc(d.wcon, d.span_bytes)};
     // u component: wcon neighbour at i+1
-    RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0>::solve(
-        R, d.si, a, item - prefix[lo], lds);
+    RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0,
+              RegBuilds<T, C>::of[BUILD].pos>::solve(R, d.si, a, item - prefix[lo], lds_raw);
 }
 
 // ---- host side ---------------------------------------------------------------
@@ -564,9 +563,9 @@ void schedule_ws(Plan &p, int cls, int workers, int queues) {
 }
 
 RegShape batch_reg_shape(int prec, int64_t nz, const Context *ctx) {
-    if (prec == SB_F64) return reg_shape<double, double>(nz, ctx->lds_per_block);
-    if (prec == SB_F32) return reg_shape<float, float>(nz, ctx->lds_per_block);
-    return reg_shape<float, double>(nz, ctx->lds_per_block);
+    if (prec == SB_F64) return reg_shape<double, double>(nz, ctx->lds_per_block, 4);
+    if (prec == SB_F32) return reg_shape<float, float>(nz, ctx->lds_per_block, 4);
+    return reg_shape<float, double>(nz, ctx->lds_per_block, 4);
 }
 
 // Classes of the register-column vadv, tallest columns first, the subdomains

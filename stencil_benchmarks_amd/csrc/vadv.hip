@@ -391,7 +391,6 @@ __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(RegBuilds<T, C>::of[BUILD].waves_per_simd)))
 void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
     extern __shared__ unsigned char lds_raw[];
-    CD<C> *lds = reinterpret_cast<CD<C> *>(lds_raw) + (threadIdx.x & 63);
     const uint32_t ncomp = uint32_t(a.ncomp), items = uint32_t(a.ngroups) * ncomp;
     const uint32_t slot = SPREAD ? xcd_chunk_remap(blockIdx.x, gridDim.x, a.xcds, kRegItemsPerXcd)
                                  : xcd_remap(blockIdx.x, gridDim.x, a.xcds);
@@ -401,8 +400,8 @@ void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
         const Rsrc R{own_rsrc(cp.stage, a.span_bytes), own_rsrc(cp.pos, a.span_bytes),
                      own_rsrc(cp.tens, a.span_bytes), own_rsrc(cp.tensstage, a.span_bytes),
                      own_rsrc(wcon, a.span_bytes)};
-        RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0>::solve(R, cp.wshift, a, g,
-                                                                                  lds);
+        RegColumn<T, C, RegBuilds<T, C>::of[BUILD].nr, kRegPf, NT ? 2 : 0,
+                  RegBuilds<T, C>::of[BUILD].pos>::solve(R, cp.wshift, a, g, lds_raw);
     }
 }
 
@@ -670,10 +669,11 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
     // 200x200x137 29 / 55, 301x283x60 all components 68 / 115); fields of
     // 4 GiB and up or with negative strides take variant 1, taller columns
     // the global scratch
-    const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block);
     const ColumnRow row = padded_row(g->nx, g->si, g->sj, sizeof(T), fields_of(f, a.ncomp));
     const int64_t reg_groups = vadv_groups(row.lanes, g->ny);
     const uint64_t items = uint64_t(reg_groups) * uint64_t(a.ncomp);
+    const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block,
+                                         reg_waves_needed(items, uint64_t(ctx->compute_units)));
     if (variant == 0) variant = buffer_ok && reg.per_cu > 0 ? 5 : lds_fits ? 1 : 2;
     SB_REQUIRE(variant >= 1 && variant <= 5, "vadv variant %d not available", variant);
     if (variant == 5) {

@@ -114,52 +114,72 @@ constexpr int64_t reg_max_levels() { return sizeof(C) == 8 ? 201 : 401; }
 // Register levels the kernels are built for, and the waves a SIMD holds of
 // each: its registers are 512, and a level takes four (two with float32
 // arithmetic) beside some 80 (FP64 fields) or 55 (float32 fields) of the
-// prefetch ring and the recurrence.
+// prefetch ring and the recurrence.  With `pos` every level also keeps its
+// pos, in registers or LDS as its (c', d'), so the backward sweep loads
+// nothing: the second read of pos is a seventh of a column's traffic, and
+// the sweep's loads are a fifth of its instructions.
 struct RegLevels {
     int nr, waves_per_simd;
+    bool pos;
 };
 template <typename T, typename C>
 struct RegBuilds;
 template <>
 struct RegBuilds<double, double> {
-    static constexpr RegLevels of[] = {{0, 3}, {24, 2}, {40, 2}, {64, 1}, {96, 1}};
+    static constexpr RegLevels of[] = {{0, 3, false}, {24, 2, false}, {40, 2, false}, {64, 1, false}, {96, 1, false}, {16, 2, true}, {40, 1, true}, {64, 1, true}};
 };
 template <>
 struct RegBuilds<float, double> {
-    static constexpr RegLevels of[] = {{0, 4}, {24, 3}, {48, 2}, {80, 1}, {112, 1}};
+    static constexpr RegLevels of[] = {{0, 4, false}, {24, 3, false}, {48, 2, false}, {80, 1, false}, {112, 1, false}, {16, 3, true}, {40, 2, true}, {88, 1, true}};
 };
 template <>
 struct RegBuilds<float, float> {
-    static constexpr RegLevels of[] = {{0, 4}, {40, 3}, {80, 2}};
+    static constexpr RegLevels of[] = {{0, 4, false}, {40, 3, false}, {80, 2, false}};
 };
 
 // LDS rows of one wave: levels 0 .. nz-2-NR.
 __host__ __device__ constexpr int64_t reg_lds_rows(int64_t nz, int nr) { return nz - 1 - nr; }
 
-// The build that holds most waves of nz levels on a CU, and how many.
+// Waves per CU beyond which more of them gain less than keeping pos does: all
+// that there are, or four where they run in many rounds (in a few rounds,
+// fewer at a time can leave the last round nearly empty: 301x283x60 FP64, 1344
+// waves, 47 us with eight a CU, 52 with four).
+inline uint64_t reg_waves_needed(uint64_t items, uint64_t cus) {
+    return items >= 12 * cus ? 4 : (items + cus - 1) / cus;
+}
+
+// The build that holds most waves of nz levels on a CU, and how many; one that
+// keeps pos where it holds as many or `need`.  Measured on MI355X (us, most
+// waves / this choice): FP64 512x512x60 141 / 135, three components 409 / 386,
+// 400x400x60 three components 268 / 251, 64x64x160 25.7 / 24.5; float32 storage
+// 32x32x80 14.8 / 13.9, 128x128x80 15.7 / 14.8, 301x283x60 three components 65.5 /
+// 63, 400x400x60 three components 124 / 128; 512x512x80 FP64, as many waves either
+// way, 187 / 180.
 struct RegShape {
     int build = 0, per_cu = 0;
     size_t lds_bytes = 0;
 };
 
 template <typename T, typename C>
-RegShape reg_shape(int64_t nz, size_t lds) {
-    RegShape best;
-    if (nz > reg_max_levels<C>()) return best;
+RegShape reg_shape(int64_t nz, size_t lds, uint64_t need) {
+    RegShape most, keeps;
+    if (nz > reg_max_levels<C>()) return most;
     int build = 0;
     for (const RegLevels &levels : RegBuilds<T, C>::of) {
         const int64_t rows = reg_lds_rows(nz, levels.nr);
-        const size_t bytes = size_t(std::max<int64_t>(rows, 0)) * 64 * sizeof(CD<C>);
+        const size_t bytes = size_t(std::max<int64_t>(rows, 0)) * 64 *
+                             (sizeof(CD<C>) + (levels.pos ? sizeof(T) : 0));
         if (rows >= 1 && bytes <= lds) {
             const int per_cu = int(std::min<size_t>(4 * levels.waves_per_simd, lds / bytes));
+            RegShape &best = levels.pos ? keeps : most;
             if (per_cu > best.per_cu) best = RegShape{build, per_cu, bytes};
         }
         ++build;
     }
-    return best;
+    return uint64_t(keeps.per_cu) >= std::min(uint64_t(most.per_cu), need) ? keeps : most;
 }
 
-template <typename T, typename C, int NR, int PF, int AUX>
+template <typename T, typename C, int NR, int PF, int AUX, bool POS>
 struct RegColumn {
     static_assert(NR == 0 || (NR % PF == 0 && NR >= 2 * PF), "register levels: whole prefetch blocks");
 
@@ -205,14 +225,17 @@ struct RegColumn {
         dd = dn * rr;
     }
 
-    // `lds` is this wave's lane column: level k < nz-1-NR at lds[64 k].
-    // Needs nz >= NR + 2.
+    // `lds_raw`: this wave's LDS, level k < nz-1-NR of a lane's column at
+    // lds[64 k], with POS followed by pos of the same levels.  Needs nz >= NR + 2.
     __device__ __forceinline__ static void solve(const Rsrc &R, int64_t wshift, const PipeArgs &a,
-                                                 int64_t g, CD<C> *lds) {
+                                                 int64_t g, unsigned char *lds_raw) {
         const C dtr = C(3.0 / 20.0);
         const int nz = int(a.nz), kl = nz - 1;
         const int low = nz - 2 - NR;            // levels 1 .. low live in LDS beside level 0
         const int part = low % PF;              // of them in the partial block
+        CD<C> *const lds = reinterpret_cast<CD<C> *>(lds_raw) + (threadIdx.x & 63);
+        T *const lpos = reinterpret_cast<T *>(lds_raw + uint32_t(low + 1) * uint32_t(64 * sizeof(CD<C>))) +
+                        (threadIdx.x & 63);
         const uint32_t skb = uint32_t(a.sk * int64_t(sizeof(T)));
         const GroupOff F = group_offsets<T>(a, g, wshift);
         auto at = [&](int k) { return F.row + uint32_t(k) * skb; };
@@ -270,6 +293,7 @@ struct RegColumn {
             cc = c / b;
             dd = d / b;
             lds[0] = CD<C>{cc, dd};
+            if constexpr (POS) lpos[0] = first.pos;
             q = Row{b, c, d, C(0), p, st_n};
         }
         // ---- partial block: levels 1 .. part ----------------------------------
@@ -279,6 +303,7 @@ struct RegColumn {
                 q = row(ring[p], q);
                 recur(q, cc, dd);
                 lds[int64_t(1 + p) * 64] = CD<C>{cc, dd};
+                if constexpr (POS) lpos[int64_t(1 + p) * 64] = ring[p].pos;
             }
         }
         if (part) {
@@ -293,10 +318,12 @@ struct RegColumn {
         uint32_t so = at(k + PF - 1);  // offset of the last level loaded
         for (; k <= low; k += PF) {
             CD<C> *out = lds + int64_t(k) * 64;
+            T *pos_out = lpos + int64_t(k) * 64;
 #pragma unroll
             for (int p = 0; p < PF; ++p) {
                 Row n;
                 recur(q, cc, dd, ring[(p + 1) % PF], n);
+                if constexpr (POS) pos_out[p * 64] = ring[p].pos;
                 step_up(so);
                 load(NR >= PF ? so : min(so, at(top)), ring[p]);
                 out[p * 64] = CD<C>{cc, dd};
@@ -307,6 +334,7 @@ struct RegColumn {
         // ---- register levels: low + 1 .. nz-2 ----------------------------------
         C rc[NR > 0 ? NR : 1], rd[NR > 0 ? NR : 1];
         T pr[PF];  // pos of the levels below, for the backward sweep
+        T rp[NR > 0 && POS ? NR : 1];
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             if (i + 1 < NR) {
@@ -323,6 +351,10 @@ struct RegColumn {
             rc[i] = cc;
             rd[i] = dd;
             if (i + PF < NR) {
+                if constexpr (POS) {
+                    rp[i] = ring[i % PF].pos;
+                    settle(rp[i]);
+                }
                 step_up(so);
                 load(so, ring[i % PF]);
             } else if (i + PF == NR) {
@@ -331,7 +363,7 @@ struct RegColumn {
         }
         // ---- level nz-1 ---------------------------------------------------------
         uint32_t sp = at(kl - 1 - PF);  // offset of the last pos level loaded, plus one
-        if constexpr (NR >= PF) {
+        if constexpr (NR >= PF && !POS) {
 #pragma unroll
             for (int p = PF - 1; p >= 0; --p) {
                 pr[p] = bload<T, 0>(R.pos, F.lane, sp);
@@ -353,6 +385,8 @@ struct RegColumn {
             T pos;
             if (i + PF >= NR) {
                 pos = ring[i % PF].pos;  // still there from the forward sweep
+            } else if constexpr (POS) {
+                pos = rp[i];
             } else {
                 pos = pr[i % PF];
                 pr[i % PF] = bload<T, 0>(R.pos, F.lane, i >= PF ? sp : at(max(low + 1 + i - PF, 0)));
@@ -365,21 +399,26 @@ struct RegColumn {
         // ---- backward: whole blocks in LDS --------------------------------------
         T pp[PF];  // pos of the partial block's levels and of level 0
 #pragma unroll
-        for (int p = 0; p < PF; ++p) pp[p] = bload<T, 0>(R.pos, F.lane, at(min(p, part)));
-        if constexpr (NR == 0) {
+        for (int p = 0; p < PF; ++p)
+            pp[p] = POS ? lpos[int64_t(min(p, part)) * 64] : bload<T, 0>(R.pos, F.lane, at(min(p, part)));
+        if constexpr (NR == 0 && !POS) {
 #pragma unroll
             for (int p = 0; p < PF; ++p)
                 pr[p] = bload<T, 0>(R.pos, F.lane, at(max(low - PF + 1 + p, 0)));
         }
         for (k = low - PF + 1; k > part; k -= PF) {
             const CD<C> *in = lds + int64_t(k) * 64;
+            const T *pos_in = lpos + int64_t(k) * 64;
             CD<C> cd[PF];
 #pragma unroll
-            for (int p = PF - 1; p >= 0; --p) cd[p] = in[p * 64];
+            for (int p = PF - 1; p >= 0; --p) {
+                cd[p] = in[p * 64];
+                if constexpr (POS) pr[p] = pos_in[p * 64];
+            }
 #pragma unroll
             for (int p = PF - 1; p >= 0; --p) {
                 const T pos = pr[p];
-                pr[p] = bload<T, 0>(R.pos, F.lane, at(max(k + p - PF, 0)));
+                if constexpr (!POS) pr[p] = bload<T, 0>(R.pos, F.lane, at(max(k + p - PF, 0)));
                 step_down(st);
                 x = cd[p].d - cd[p].c * x;
                 bstore<T>(R.ts, F.lane, st, T(dtr * (x - C(pos))));

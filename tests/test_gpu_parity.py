@@ -475,6 +475,31 @@ def test_vadv_register_builds(gpu, prec, nz):
         assert np.array_equal(g[inner(domain, halo)], e)
 
 
+# the builds that keep pos: around the fewest levels of 16, 40, 64 and 88
+# register levels, whole and partial blocks in LDS, and the tallest columns
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("nz", [17, 18, 19, 24, 33, 41, 42, 44, 49, 67, 68, 74, 89, 90, 91, 106,
+                                160, 170, 201])
+def test_vadv_register_builds_keeping_pos(gpu, prec, nz):
+    domain, halo = (37, 5, nz), (1, 1, 0)
+    fields = make_fields(domain, halo, _dtype(prec), count=16, seed=nz)
+    got = _run_vadv(gpu, fields, [3, 7, 11], domain, halo, _prec(gpu, prec), True, 0)
+    expected = _vadv_expected(fields, domain, halo, prec, ("u", "v", "w"))
+    for g, e in zip(got, expected):
+        assert np.array_equal(g[inner(domain, halo)], e)
+
+
+# more columns than a device holds at once in the builds that keep pos
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("nz", [10, 26, 42, 66, 98, 115])
+def test_vadv_register_builds_many_columns(gpu, prec, nz):
+    domain, halo = (601, 140, nz), (1, 1, 0)
+    fields = make_fields(domain, halo, _dtype(prec), count=8, seed=nz)
+    got, = _run_vadv(gpu, fields, [3], domain, halo, _prec(gpu, prec), False, 0)
+    expected = _expected(lambda *f: oracle.vadv(*f, domain, halo), fields[:5], prec)
+    assert np.array_equal(got[inner(domain, halo)], expected)
+
+
 # rows padded to whole 128- or 64-byte chunks of lanes (vadv_regs.h): the
 # lanes past a row's end repeat its last column; 64-byte aligned fields with
 # odd and even multiples of 64 bytes as row pitch, one of unaligned rows
