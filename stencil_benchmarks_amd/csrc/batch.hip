@@ -7,11 +7,15 @@
 // and the caller swaps u and u_next (parity).  The halo of u / u_next is
 // never written: it is a fixed boundary, identical in both buffers.
 //
-// A sequence of steps starts with one counter-reset kernel; each step is one
-// persistent hdiff launch and one or two persistent vadv launches (grids =
-// resident workgroups), all drawing items from device work queues.  Subdomains
-// are ordered by cost, largest first, so the tail of each queue holds the
-// small items.
+// Without launch options a step is one hdiff launch, a workgroup of the
+// LDS-DMA tile per tile and plane, and one vadv launch per register build, a
+// wave per column group, in plain grids that the dispatcher balances.
+//
+// With options a sequence of steps starts with one counter-reset kernel; each
+// step is one persistent hdiff launch and one or two persistent vadv launches
+// (grids = resident workgroups), all drawing items from device work queues.
+// Subdomains are ordered by cost, largest first, so the tail of each queue
+// holds the small items.
 //   hdiff items: (subdomain, 64 x TY tile, KC-plane chunk), the tile worker
 //     of the plain kernel (hdiff_tile.h), drawn from device counters.  The
 //     items are split into one contiguous range per XCD, each with its own

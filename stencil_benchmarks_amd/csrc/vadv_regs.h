@@ -5,8 +5,8 @@
 // or drain and needs no barrier, so a CU can hold as many groups as its
 // registers and LDS have room for: (c', d') of one level are 1 KB of a group
 // with FP64 arithmetic, a CU has 512 KB of registers beside its 160 KB of
-// LDS, and at nz = 80 with NR = 40 register levels four waves (one per SIMD)
-// share a CU.  What bounds such a wave is its own instruction stream: the
+// LDS, and at nz = 80 with NR = 64 register levels four waves (one per SIMD)
+// share a CU, pos of every level kept too.  What bounds such a wave is its own instruction stream: the
 // forward recurrence is one serial chain per column, alone on its SIMD.  So
 // the loop is arranged for few instructions and a short chain:
 //   - the register levels are the highest ones, nz-1-NR .. nz-2, so their
