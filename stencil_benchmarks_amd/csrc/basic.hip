@@ -553,16 +553,16 @@ hipError_t launch_packed_axes(int axes, bool wide, const T *inp, T *out, const B
 
 // Whether the packed kernel takes this call, its default: unit stride along
 // axis 0, rows upwards, offsets of a plane and its neighbour rows below 4 GiB,
-// indexes of lanes and workgroups below 2^31, and for the Laplacian, whose
+// indexes of lanes below 2^30 and threads of the launch below 2^32, and for the Laplacian, whose
 // terms are summed in the order i, j, k, axes in that order of strides.  The
 // other kernels were slower at every size measured, from 32x32x80 up
 // (128x128x80 FP64 average along j: 6.5 us against 5.0).
-bool packed_fits(const BasicArgs &a, int op) {
+bool packed_fits(const BasicArgs &a, int op, int vec) {
     const double rows = double(a.n[1]), row = double(a.n[0]);
     return a.s[0] == 1 && a.s[1] > 0 &&
            ((rows + 9) * double(a.s[1]) + row + 9) * 8.0 < 4294967296.0 &&
            row * (rows + 9) < 1073741824.0 &&
-           (row * (rows + 9) / BLOCK + 1) * double(a.n[2]) < 2147483648.0 &&
+           launch_fits(((row / vec + 1) * (rows + 9) / BLOCK + 1) * double(a.n[2]), BLOCK) &&
            (op == OP_COPY || op == OP_AVG1 || op == OP_AVG2 ||
             (a.lap_mask && a.perm[0] < a.perm[1] && a.perm[1] < a.perm[2]));
 }
@@ -662,9 +662,9 @@ int launch_basic_prec(const void *inp_v, void *out_v, const sb_geom *g, int axis
             });
         }
     }
-    if (variant == 0 && !row_options && packed_fits(a, OP)) {
+    const bool wide = a.n[0] >= int64_t(16 / sizeof(T));
+    if (variant == 0 && !row_options && packed_fits(a, OP, wide ? int(16 / sizeof(T)) : 1)) {
         const int axes = OP == OP_LAP ? lap_mask : OP == OP_COPY ? 0 : 1 << a.axis;
-        const bool wide = a.n[0] >= int64_t(16 / sizeof(T));
         return timed_launch(l, seconds, [&]() -> hipError_t {
             return launch_packed_axes<T, C, OP>(axes, wide, inp, out, a, ctx);
         });

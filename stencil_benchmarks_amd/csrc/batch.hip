@@ -623,7 +623,7 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
         dma_items += uint64_t((g.nx + 63) / 64) *
                      uint64_t((g.ny + dma_rows(prec) - 1) / dma_rows(prec)) * uint64_t(g.nz);
     }
-    if (dma_items >= (uint64_t(1) << 31)) p.dma_unit = 0;
+    if (!launch_fits(double(dma_items), 256.0)) p.dma_unit = 0;
     p.dma_hint = hdiff_dma_hint(points, esize);
     p.host_dma.clear();
     const int ty = p.dma_unit ? dma_rows(prec) : hdiff_ty(hl);

@@ -228,7 +228,7 @@ int launch_hdiff(const void *inp_v, const void *coeff_v, void *out_v, const sb_g
     const int unit = hdiff_dma_unit(*g, inp, sizeof(T));  // bytes that variant 2 stages at a time
     if (variant == 0) {
         // the LDS-DMA tile where it applies (figures: file comment)
-        if (!tile_options && unit && hdiff_dma_blocks(a, dma_rows) < (uint64_t(1) << 31))
+        if (!tile_options && unit && launch_fits(double(hdiff_dma_blocks(a, dma_rows)), 256.0))
             variant = 2;
         else
             variant = tile_fits ? 1 : 3;

@@ -165,7 +165,7 @@ int pack_interior(const void *src, void *dst, const sb_geom *g, Context *ctx) {
     const int64_t ti = (g->nx + 31) / 32, tk = (g->nz + 31) / 32;
     if (g->nx == 0 || g->ny == 0 || g->nz == 0) return 0;
     SB_REQUIRE(src && dst, "NULL field pointer");
-    SB_REQUIRE(double(ti) * double(tk) * double(g->ny) < 2147483648.0,
+    SB_REQUIRE(launch_fits(double(ti) * double(tk) * double(g->ny), 256.0),
                "domain too large for one launch");
     enqueue_kernel(pack_kernel<T>, dim3(unsigned(ti * tk * g->ny)), dim3(256), 0, ctx->stream,
                    static_cast<const T *>(src), static_cast<T *>(dst), g->nx, g->ny, g->nz, g->si,

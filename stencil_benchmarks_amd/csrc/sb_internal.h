@@ -161,6 +161,9 @@ __host__ __device__ inline uint32_t xcd_chunk_remap(uint32_t b, uint32_t total, 
     return first + (r % xcds) * chunk + r / xcds;
 }
 
+// The runtime refuses launches of 2^32 threads and more along one grid axis.
+inline bool launch_fits(double blocks, double threads) { return blocks * threads < 4294967296.0; }
+
 // Division of a dividend below 2^31 by a divisor fixed at launch: q =
 // (n * mul) >> shift with mul = ceil(2^shift / d), shift = 31 + ceil(log2 d).
 // The rounding error of mul stays below 1/d of the quotient's unit for every

@@ -273,11 +273,13 @@ int dispatch_vector(T *a, T *b, T *c, size_t n, double scalar, const sb_launch *
     constexpr size_t kWords = OP == SB_STREAM_COPY || OP == SB_STREAM_SCALE ? 2 : 3;
     const bool streams = n > (size_t(512) << 20) / (kWords * sizeof(T));
     const int nt = !open ? l->variant & 3 : streams ? 3 : 2;
-    const int unroll = open ? 1 : l->unroll ? l->unroll : 4;
+    constexpr int kWide = int(16 / sizeof(T));
+    // (four vectors of a thread where one would be too many threads for a launch)
+    const int unroll = open && launch_fits(double(n / kWide) + 1024.0, 1.0)
+                           ? 1 : !open && l->unroll ? l->unroll : 4;
     const int block = open ? 1024 : l->bx ? l->bx : 256;
     SB_REQUIRE(block >= 64 && block <= 1024 && block % 64 == 0,
                "STREAM block size %d must be a multiple of 64 in [64, 1024]", block);
-    constexpr int kWide = int(16 / sizeof(T));
     const int vec = (l && l->by) ? l->by : kWide;
     const int per_cu = l ? l->bz : 0;
     SB_REQUIRE(per_cu >= 0 && per_cu <= 64, "STREAM workgroups per CU %d not in 0..64", per_cu);
