@@ -31,7 +31,7 @@
 // (hdiff_dma_unit); a domain's last tiles may be partial.  When the variant is
 // asked for by number it takes whole tiles only.  Measured on MI355X against
 // variant 1, launches back to back: 512x512x160 FP64 172 / 189 us, float32
-// storage 94 / 112 us, 397x411x137 96 / 110 and 53 / 70 us, 128x128x80 6.9 /
+// storage 94 / 112 us, 397x411x137 96 / 110 and 49 / 70 us, 128x128x80 6.9 /
 // 9.5 and 5.1 / 11.6 us.
 //
 // Variant 3 (on the fly).  One thread per point reading its 13 inputs

@@ -50,6 +50,16 @@ __device__ __forceinline__ C limited(C flux, C gradient) {
     return flux * gradient > C(0) ? C(0) : flux;
 }
 
+// `v` of the lane to the left, `first` in lane 0 of the wave.
+__device__ __forceinline__ double from_left_lane(double v, double first) {
+    constexpr int kWaveShr1 = 0x138;
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), kWaveShr1,
+                                               0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), kWaveShr1,
+                                               0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
 template <bool NT, typename T>
 __device__ __forceinline__ T ld_nt(global_ptr<const T> p) {
     if constexpr (NT)
@@ -134,16 +144,34 @@ struct HdiffTile {
             lap[q] = laplacian(ic[q + 1], ((ir[q] + il[q]) + ic[q + 2]) + ic[q]);
     #pragma unroll
         for (int q = 0; q < RPT; ++q) s_lap[(ty * RPT + q) * PW + tx + 1] = lap[q + 1];
-        if (tid < 2 * TY) {
+        // Widened float32 fields: the flux at a point's left edge is the
+        // right edge of the lane before, so a wave shift of two instructions
+        // replaces its six.  Only lane 0 has no such lane; wave 0 publishes
+        // its flux, and wave 1 the Laplacian of the halo column on the right.
+        // Instructions bound these tiles (397x411x137 51.7 -> 48.8 us); FP64
+        // fields are bound by memory and lose by the longer way to the barrier
+        // (none gained, the small hdiff and vadv steps up to 4 %).
+        constexpr bool SHIFT = sizeof(S) == 4 && sizeof(C) == 8;
+        static_assert(!SHIFT || NW >= 2, "two waves share the halo columns");
+        auto column = [&](int rr, int c) {
+            return laplacian(C(sin[rr * SW + c]),
+                             ((C(sin[rr * SW + c + 1]) + C(sin[rr * SW + c - 1])) +
+                              C(sin[(rr + 1) * SW + c])) +
+                                 C(sin[(rr - 1) * SW + c]));
+        };
+        if constexpr (SHIFT) {
+            if (ty < 2 && tx < TY) {
+                const int r = tx, rr = r + 2;
+                if (ty == 0)
+                    s_lap[r * PW] = limited(column(rr, LEFT) - column(rr, LEFT - 1),
+                                            C(sin[rr * SW + LEFT]) - C(sin[rr * SW + LEFT - 1]));
+                else
+                    s_lap[r * PW + TX + 1] = column(rr, TX + LEFT);
+            }
+        } else if (tid < 2 * TY) {
             // Laplacian of the tile's halo columns -1 and TX.
             const int side = tid / TY, r = tid - side * TY;
-            const int c = side ? TX + LEFT : LEFT - 1;
-            const int rr = r + 2;
-            const C v = laplacian(C(sin[rr * SW + c]),
-                                  ((C(sin[rr * SW + c + 1]) + C(sin[rr * SW + c - 1])) +
-                                   C(sin[(rr + 1) * SW + c])) +
-                                      C(sin[(rr - 1) * SW + c]));
-            s_lap[r * PW + (side ? TX + 1 : 0)] = v;
+            s_lap[r * PW + (side ? TX + 1 : 0)] = column(r + 2, side ? TX + LEFT : LEFT - 1);
         }
         __syncthreads();
     #pragma unroll
@@ -152,7 +180,11 @@ struct HdiffTile {
             const C c0 = ic[q + 2];
             const C lc = lap[q + 1];
             const C flx = limited(s_lap[r * PW + tx + 2] - lc, ir[q + 1] - c0);
-            const C flx_m = limited(lc - s_lap[r * PW + tx], c0 - il[q + 1]);
+            C flx_m;
+            if constexpr (SHIFT)
+                flx_m = from_left_lane(flx, s_lap[r * PW]);
+            else
+                flx_m = limited(lc - s_lap[r * PW + tx], c0 - il[q + 1]);
             const C fly = limited(lap[q + 2] - lc, ic[q + 3] - c0);
             const C fly_m = limited(lc - lap[q], c0 - ic[q + 1]);
             res[q] = c0 - cf[q] * (((flx - flx_m) + fly) - fly_m);
