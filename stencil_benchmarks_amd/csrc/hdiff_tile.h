@@ -344,9 +344,10 @@ struct HdiffTile {
 // A tile that reaches past the domain's last row or column (EDGE, a uniform
 // branch) clamps its unit addresses to the last halo row and to the unit that
 // holds column nx + 1, as the register-staged tile does: what is staged there
-// only feeds outputs that are not stored.  A 16-byte unit may read up to two
-// columns more than the halo of 2 on either side; hdiff_dma_unit says where
-// the field holds them.
+// only feeds outputs that are not stored.  A 16-byte unit may read more
+// columns than the halo of 2: two on the left and up to three on the right of
+// float32 fields, one on the right of 8-byte ones; hdiff_dma_unit says where the
+// field holds them.
 template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT>
 struct HdiffDma {
     using Tile = HdiffTile<T, C, TY, RPT, 2>;
@@ -357,6 +358,13 @@ struct HdiffDma {
     static constexpr int STEPS = (UNITS + 63) / 64;  // wave instructions that stage the tile
     static constexpr int TILE_ELEMS = STEPS * 64 * UNIT / int(sizeof(T));
     static_assert(int(sizeof(T)) * LW % UNIT == 0, "a unit must not straddle two rows");
+
+    // Unit of a staged row that holds (the end of) column nx + 1, counted from
+    // the first column staged by the tile at i0.
+    __host__ __device__ static constexpr uint32_t last_unit(int32_t nx, int32_t i0) {
+        return uint32_t(nx + 1 + LEFT - i0) * uint32_t(sizeof(T)) / uint32_t(UNIT) +
+               (UNIT < int(sizeof(T)) ? 1u : 0u);
+    }
 
     // `corner` points at the tile's first staged element; wave ty of the NW
     // issues instructions ty, ty + NW, ...
@@ -415,10 +423,7 @@ struct HdiffDma {
         const global_ptr<const T> corner = scalar(inp + plane + ((j0 - 2) * sj + (i0 - LEFT)));
         if (edge) {
             const uint32_t last_row = uint32_t(ny + 3 - j0);
-            const uint32_t last_unit =
-                uint32_t(nx + 1 + LEFT - i0) * uint32_t(sizeof(T)) / uint32_t(UNIT) +
-                (UNIT < int(sizeof(T)) ? 1u : 0u);
-            stage<true>(corner, s_tile, last_row, last_unit, pitch, tx, ty);
+            stage<true>(corner, s_tile, last_row, last_unit(nx, i0), pitch, tx, ty);
         } else {
             stage<false>(corner, s_tile, 0, 0, pitch, tx, ty);
         }
@@ -456,8 +461,10 @@ inline bool hdiff_dma_hint(double points, size_t itemsize) {
 // where the tile corners are 16-byte aligned (row and plane strides of whole
 // chunks and an aligned interior origin) and the field holds the columns
 // beyond the halo of 2 that come with the chunks: column nx + 2 with odd nx
-// (8-byte fields, a halo of 3), or columns -4 .. nx + 3 (4-byte fields; past
-// a row's own halo they are in the neighbouring rows or planes).
+// (8-byte fields, a halo of 3), or columns from -4 on up to the end of the
+// chunk of column nx + 1, which is nx + 4 where that column opens a chunk and
+// nx + 3 at most elsewhere (4-byte fields; past a row's own halo they are in
+// the neighbouring rows or planes).
 inline int hdiff_dma_unit(const sb_geom &g, const void *inp, size_t itemsize) {
     if (g.si != 1 || g.sj <= 0 || g.sj * int64_t(itemsize) >= (int64_t(1) << 24)) return 0;
     if (!hdiff_tile_fits(g.nx, g.ny, g.si, g.sj, itemsize) ||
@@ -467,7 +474,7 @@ inline int hdiff_dma_unit(const sb_geom &g, const void *inp, size_t itemsize) {
     const bool aligned = g.sj % chunk == 0 && g.sk % chunk == 0 &&
                          reinterpret_cast<uintptr_t>(inp) % 16 == 0;
     const bool holds = itemsize == 8 ? g.nx % 2 == 0 || g.hi >= 3
-                                     : g.hi >= 4 || g.hj >= 3 || g.hk >= 1;
+                                     : g.hi >= (g.nx % 4 == 3 ? 5 : 4) || g.hj >= 3 || g.hk >= 1;
     return aligned && holds ? 16 : 4;
 }
 
