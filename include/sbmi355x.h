@@ -170,8 +170,7 @@ int sb_laplacian(int prec, int along_x, int along_y, int along_z,
  * templates/horizontal_diffusion_*.j2); semantics of base.py:276-311.
  * Requires hi, hj >= 2.  Variants: 0 default (the kernel of 2, also on
  * partial tiles and any alignment, where si = 1, 0 < sj with a row pitch
- * below 16 MiB, a k-plane is below 4 GiB and no tile option is given; else 1
- * where positive i and j strides and a k-plane below 4 GiB let the tile use
+ * below 16 MiB and no tile option is given; else 1 where positive i and j strides and a k-plane below 4 GiB let the tile use
  * 32-bit plane offsets, else 3), 1 LDS-staged tile
  * (launch->by = tile rows 8/16/32, ->bz = k-planes per workgroup 1..16, 0
  * measured default; ->unroll 0 = default (non-temporal coeff loads), else
@@ -180,7 +179,8 @@ int sb_laplacian(int prec, int along_x, int along_y, int along_z,
  * workgroup (every precision; launch->by = tile rows 8 or 16, 0 = 8 for
  * SB_F64 and 16 for float32 fields; needs nx a multiple of 64, ny of the
  * tile rows, si = 1, 0 < sj with a row pitch below 16 MiB, and for SB_F64 even sj and
- * sk and a 16-byte aligned inp), 3 per-point recomputation through the caches
+ * sk and a 16-byte aligned inp; planes of 4 GiB and more take several
+ * launches), 3 per-point recomputation through the caches
  * (the reference's OnTheFly schedule). */
 int sb_hdiff(int prec, const void *inp, const void *coeff, void *out,
              const sb_geom *g, const sb_launch *l, double *seconds);

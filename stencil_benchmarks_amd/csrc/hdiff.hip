@@ -28,7 +28,8 @@
 // arithmetic was bound by its instructions (a scalar unit serves the four
 // SIMDs of a CU, and a wave issued 177 scalar beside 210 vector
 // instructions; 111 and 165 now).  Unit i stride and a row pitch below 16 MiB
-// (hdiff_dma_unit); a domain's last tiles may be partial.  When the variant is
+// (hdiff_dma_unit); a domain's last tiles may be partial, and planes of 4 GiB
+// and more take several launches.  When the variant is
 // asked for by number it takes whole tiles only.  Measured on MI355X against
 // variant 1, launches back to back: 512x512x160 FP64 172 / 189 us, float32
 // storage 94 / 112 us, 397x411x137 96 / 110 and 49 / 70 us, 128x128x80 6.9 /
@@ -39,6 +40,7 @@
 // (stencils/cuda_hip/horizontal_diffusion.py:50-96) with the oracle's
 // arithmetic order.  Kept as an independent implementation to cross-check
 // variant 1.
+#include <algorithm>
 #include <type_traits>
 
 #include "hdiff_tile.h"
@@ -117,19 +119,25 @@ uint64_t hdiff_dma_blocks(const HdiffArgs &a, int ty) {
 
 template <typename T, typename C, int TY, int RPT, int UNIT>
 hipError_t launch_dma(const T *inp, const T *coeff, T *out, HdiffArgs a, Context *ctx) {
+    const int64_t rows = a.ny, band = hdiff_dma_band(a.nx, rows, a.sj, sizeof(T));
+    const bool hint = hdiff_dma_hint(double(a.nx) * double(rows) * double(a.nz), sizeof(T));
     a.tiles_i = int32_t((a.nx + 63) / 64);
-    a.tiles_j = int32_t((a.ny + TY - 1) / TY);
-    const uint64_t blocks = hdiff_dma_blocks(a, TY);
-    if (blocks >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
-    const TileGrid tg = make_tile_grid(uint32_t(blocks), uint32_t(a.tiles_i), uint32_t(a.tiles_j),
-                                       ctx->xcds);
-    const dim3 grid{unsigned(blocks)}, threads{64u, unsigned(TY / RPT)};
-    if (hdiff_dma_hint(double(a.nx) * double(a.ny) * double(a.nz), sizeof(T)))
-        enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, true>), grid, threads, 0, ctx->stream,
-                       inp, coeff, out, a, tg);
-    else
-        enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, false>), grid, threads, 0,
-                       ctx->stream, inp, coeff, out, a, tg);
+    for (int64_t j = 0; j < rows; j += band) {
+        a.ny = std::min(band, rows - j);
+        a.tiles_j = int32_t((a.ny + TY - 1) / TY);
+        const uint64_t blocks = hdiff_dma_blocks(a, TY);
+        if (blocks >= (uint64_t(1) << 31)) return hipErrorInvalidValue;
+        const TileGrid tg = make_tile_grid(uint32_t(blocks), uint32_t(a.tiles_i),
+                                           uint32_t(a.tiles_j), ctx->xcds);
+        const dim3 grid{unsigned(blocks)}, threads{64u, unsigned(TY / RPT)};
+        const int64_t at = j * a.sj;
+        if (hint)
+            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, true>), grid, threads, 0,
+                           ctx->stream, inp + at, coeff + at, out + at, a, tg);
+        else
+            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, false>), grid, threads, 0,
+                           ctx->stream, inp + at, coeff + at, out + at, a, tg);
+    }
     return hipGetLastError();
 }
 

@@ -406,7 +406,7 @@ struct HdiffDma {
         return (P)v;
     }
 
-    // Offsets within a plane are 32-bit (hdiff_dma_unit), on a plane's uniform
+    // Offsets within a plane are 32-bit (hdiff_dma_band), on a plane's uniform
     // base.
     __device__ static void run(global_ptr<const T> inp, global_ptr<const T> coeff,
                                global_ptr<T> out, int32_t nx, int32_t ny, int32_t sj, int64_t sk,
@@ -455,9 +455,16 @@ inline bool hdiff_dma_hint(double points, size_t itemsize) {
     return 3 * points * double(itemsize) > 96.0 * (1 << 20);
 }
 
+// Rows that one launch of the LDS-DMA tile takes: the tile addresses a plane by
+// 32-bit byte offsets, so planes of 4 GiB and more go in bands of whole tiles.
+// A row pitch below 16 MiB leaves bands of 240 rows and more.
+inline int64_t hdiff_dma_band(int64_t nx, int64_t ny, int64_t sj, size_t itemsize) {
+    if (hdiff_tile_fits(nx, ny, 1, sj, itemsize)) return ny;
+    return (((int64_t(1) << 32) / int64_t(itemsize) - (nx + 4)) / sj - 4) / 16 * 16;
+}
+
 // Bytes of the unit that the LDS-DMA tile stages this field by, or 0 where it
-// does not take it: unit i stride, a positive row pitch below 16 MiB and a
-// plane below 4 GiB (2^31 elements); 16
+// does not take it: unit i stride and a positive row pitch below 16 MiB; 16
 // where the tile corners are 16-byte aligned (row and plane strides of whole
 // chunks and an aligned interior origin) and the field holds the columns
 // beyond the halo of 2 that come with the chunks: column nx + 2 with odd nx
@@ -467,9 +474,7 @@ inline bool hdiff_dma_hint(double points, size_t itemsize) {
 // the neighbouring rows or planes).
 inline int hdiff_dma_unit(const sb_geom &g, const void *inp, size_t itemsize) {
     if (g.si != 1 || g.sj <= 0 || g.sj * int64_t(itemsize) >= (int64_t(1) << 24)) return 0;
-    if (!hdiff_tile_fits(g.nx, g.ny, g.si, g.sj, itemsize) ||
-        (g.ny + 3) * g.sj + g.nx + 4 >= (int64_t(1) << 31))
-        return 0;
+    if (hdiff_dma_band(g.nx, g.ny, g.sj, itemsize) <= 0) return 0;  // rows far beyond the pitch
     const int64_t chunk = 16 / int64_t(itemsize);
     const bool aligned = g.sj % chunk == 0 && g.sk % chunk == 0 &&
                          reinterpret_cast<uintptr_t>(inp) % 16 == 0;

@@ -1,8 +1,9 @@
 // Host-side check of what the LDS-DMA hdiff tile reads
 // (stencil_benchmarks_amd/csrc/hdiff_tile.h): over halos, extents and strides,
 // every byte of every unit that hdiff_dma_unit lets the tile stage lies in the
-// field, from its lowest to its highest halo point.  Exits non-zero on the
-// first unit that does not.
+// field, from its lowest to its highest halo point, and every launch's rows
+// are whole tiles that 32-bit byte offsets cover.  Exits non-zero on the first
+// unit or band that does not hold this.
 #include <algorithm>
 #include <cstdio>
 
@@ -53,7 +54,30 @@ static int check_field(const sb_geom &g, uintptr_t origin) {
     return unit == 16 ? check_units<T, TY, 16>(g) : check_units<T, TY, 4>(g);
 }
 
+// Bands of planes around and beyond 4 GiB.
+static int check_bands() {
+    for (int64_t size : {4, 8})
+        for (int64_t pitch : {int64_t(1) << 10, int64_t(123456), int64_t(1) << 20, (int64_t(1) << 24) - 8})
+            for (int64_t rows : {int64_t(1), int64_t(240), int64_t(256), int64_t(272), (int64_t(1) << 32) / pitch - 4,
+                                 (int64_t(1) << 32) / pitch - 3, (int64_t(1) << 32) / pitch, int64_t(9000000)}) {
+                const int64_t sj = pitch / size;
+                for (int64_t nx : {int64_t(1), int64_t(64), sj - 4}) {
+                    const int64_t band = sb::hdiff_dma_band(nx, rows, sj, size_t(size));
+                    const int64_t in_band = std::min(band, rows);
+                    const int64_t last = (in_band + 1) * sj + nx + 4;  // row in_band + 1: the halo
+                    if (band < 1 || (band < rows && band % 16 != 0) || last * size >= (int64_t(1) << 32)) {
+                        std::printf("%lld-byte field, nx %lld, %lld rows of pitch %lld: bands of %lld rows\n",
+                                    (long long)size, (long long)nx, (long long)rows, (long long)sj,
+                                    (long long)band);
+                        return 1;
+                    }
+                }
+            }
+    return 0;
+}
+
 int main() {
+    if (check_bands()) return 1;
     const int64_t widths[] = {1, 2, 3, 4, 5, 6, 7, 8, 61, 62, 63, 64, 65, 66, 67, 125, 126, 127, 128, 129, 131};
     const int64_t heights[] = {1, 7, 8, 9, 15, 16, 17, 33};
     for (int64_t nx : widths)

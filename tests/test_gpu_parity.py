@@ -330,6 +330,46 @@ def test_hdiff_partial_tiles(gpu, prec, domain, halo, alignment):
     _check_halo(got, domain, halo)
 
 
+# a k-plane beyond 4 GiB, rows at the widest pitch: several launches of the
+# LDS-DMA tile, the last one of whole and of partial tiles
+@pytest.mark.parametrize("prec", ["f64", "f32_f64"])
+@pytest.mark.parametrize("variant,domain", [(2, (64, 272, 1)), (0, (64, 272, 1)), (0, (61, 267, 1))])
+def test_hdiff_planes_beyond_4_gib(gpu, prec, variant, domain):
+    from stencil_benchmarks_amd.device import DeviceBuffer
+
+    halo, dtype = (2, 2, 0), np.dtype(_dtype(prec))
+    pitch = (1 << 24) - 16
+    inp, coeff = make_fields(domain, halo, dtype, count=2, seed=sum(domain))
+    out = _with_sentinel(make_fields(domain, halo, dtype)[0])
+    width, rows = out.shape[0], out.shape[1]
+    bufs = [DeviceBuffer(rows * pitch) for _ in range(3)]
+    try:
+        lead = 16 - 2 * dtype.itemsize  # bytes before a row: the origin is 16-byte aligned
+        for buf, host in zip(bufs, (inp, coeff, out)):
+            for j in range(rows):
+                line = np.ascontiguousarray(host[:, j, 0])
+                gpu.call("sb_memcpy_h2d", ctypes.c_void_p(buf.ptr + j * pitch + lead),
+                         ctypes.c_void_p(line.ctypes.data), line.nbytes)
+        origin = [ctypes.c_void_p(b.ptr + 2 * pitch + lead + 2 * dtype.itemsize) for b in bufs]
+        sj = pitch // dtype.itemsize
+        geom = gpu.Geom(*domain, 1, sj, sj * rows, *halo)
+        gpu.call("sb_hdiff", _prec(gpu, prec), *origin, geom, gpu.launch_options(variant=variant),
+                 None)
+        gpu.call("sb_synchronize")
+        got = np.empty((width, rows, 1), dtype)
+        for j in range(rows):
+            line = np.empty(width, dtype)
+            gpu.call("sb_memcpy_d2h", ctypes.c_void_p(line.ctypes.data),
+                     ctypes.c_void_p(bufs[2].ptr + j * pitch + lead), line.nbytes)
+            got[:, j, 0] = line
+    finally:
+        for b in bufs:
+            b.free()
+    expected = _expected(lambda a, b: oracle.hdiff(a, b, domain, halo), [inp, coeff], prec)
+    assert np.array_equal(got[inner(domain, halo)], expected)
+    _check_halo(got, domain, halo)
+
+
 @pytest.mark.parametrize("domain,prec,tile,match", [((70, 16, 2), "f64", 0, "multiple of 64"),
                                                     ((64, 12, 2), "f64", 0, "multiple of 8"),
                                                     ((70, 16, 2), "f32_f64", 0, "multiple of 64"),
