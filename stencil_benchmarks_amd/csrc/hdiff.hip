@@ -90,11 +90,11 @@ __global__ __launch_bounds__(64 * (TY / RPT)) void hdiff_lds_kernel(
 
 // Variant 2 kernel: one 64 x TY tile of one k-plane per workgroup
 // (HdiffDma, hdiff_tile.h).
-template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT>
+template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT, bool STREAM>
 __global__ __launch_bounds__(64 * (TY / RPT)) void hdiff_dma_kernel(
     const T *__restrict__ inp, const T *__restrict__ coeff, T *__restrict__ out, HdiffArgs a,
     TileGrid tg) {
-    using Dma = HdiffDma<T, C, TY, RPT, UNIT, HINT>;
+    using Dma = HdiffDma<T, C, TY, RPT, UNIT, HINT, STREAM>;
     __shared__ __attribute__((aligned(16))) T s_tile[Dma::TILE_ELEMS];
     __shared__ C s_lap[Dma::Tile::LAP_ELEMS];
     uint32_t ti, tj, k;
@@ -120,7 +120,10 @@ uint64_t hdiff_dma_blocks(const HdiffArgs &a, int ty) {
 template <typename T, typename C, int TY, int RPT, int UNIT>
 hipError_t launch_dma(const T *inp, const T *coeff, T *out, HdiffArgs a, Context *ctx) {
     const int64_t rows = a.ny, band = hdiff_dma_band(a.nx, rows, a.sj, sizeof(T));
-    const bool hint = hdiff_dma_hint(double(a.nx) * double(rows) * double(a.nz), sizeof(T));
+    const double points = double(a.nx) * double(rows) * double(a.nz);
+    const bool hint = hdiff_dma_hint(points, sizeof(T));
+    // plain stores only in fields that take the hint on coeff
+    const bool stream = hdiff_dma_stream(out, a.sj, points, sizeof(T));
     a.tiles_i = int32_t((a.nx + 63) / 64);
     for (int64_t j = 0; j < rows; j += band) {
         a.ny = std::min(band, rows - j);
@@ -131,11 +134,14 @@ hipError_t launch_dma(const T *inp, const T *coeff, T *out, HdiffArgs a, Context
                                            uint32_t(a.tiles_j), ctx->xcds);
         const dim3 grid{unsigned(blocks)}, threads{64u, unsigned(TY / RPT)};
         const int64_t at = j * a.sj;
-        if (hint)
-            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, true>), grid, threads, 0,
+        if (!stream)
+            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, true, false>), grid, threads, 0,
+                           ctx->stream, inp + at, coeff + at, out + at, a, tg);
+        else if (hint)
+            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, true, true>), grid, threads, 0,
                            ctx->stream, inp + at, coeff + at, out + at, a, tg);
         else
-            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, false>), grid, threads, 0,
+            enqueue_kernel((hdiff_dma_kernel<T, C, TY, RPT, UNIT, false, true>), grid, threads, 0,
                            ctx->stream, inp + at, coeff + at, out + at, a, tg);
     }
     return hipGetLastError();

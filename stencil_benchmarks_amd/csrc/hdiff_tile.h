@@ -337,9 +337,8 @@ struct HdiffTile {
 // 4-byte word, which needs no alignment beyond the element's.  Float32 fields
 // gain most from the wide units: FP64 arithmetic bounds the kernel by its
 // instructions, and 64x16 tiles take 6 staging instructions instead of 22.
-// The stores are non-temporal (512x512x160 FP64 179 -> 172 us, float32
-// storage 95 -> 91 us; a vadv launch that reads the result next loses nothing
-// by it), and with HINT the coeff loads (dma_hint below).
+// With HINT the coeff loads are non-temporal (hdiff_dma_hint below), with
+// STREAM the stores (hdiff_dma_stream below).
 //
 // A tile that reaches past the domain's last row or column (EDGE, a uniform
 // branch) clamps its unit addresses to the last halo row and to the unit that
@@ -348,7 +347,7 @@ struct HdiffTile {
 // columns than the halo of 2: two on the left and up to three on the right of
 // float32 fields, one on the right of 8-byte ones; hdiff_dma_unit says where the
 // field holds them.
-template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT>
+template <typename T, typename C, int TY, int RPT, int UNIT, bool HINT, bool STREAM = true>
 struct HdiffDma {
     using Tile = HdiffTile<T, C, TY, RPT, 2>;
     static constexpr int LEFT = UNIT == 16 ? 16 / int(sizeof(T)) : 2;
@@ -442,7 +441,8 @@ struct HdiffDma {
         if (tx < nx - i0) {
     #pragma unroll
             for (int q = 0; q < RPT; ++q)
-                if (row0 + q < ny) st_nt<true>(at(out_k, uint32_t(row0 + q) * pitch + lane), T(res[q]));
+                if (row0 + q < ny)
+                    st_nt<STREAM>(at(out_k, uint32_t(row0 + q) * pitch + lane), T(res[q]));
         }
     }
 };
@@ -453,6 +453,23 @@ struct HdiffDma {
 // 400x400x100 float32 storage, 192 MB: 36.8 / 41.1 us).
 inline bool hdiff_dma_hint(double points, size_t itemsize) {
     return 3 * points * double(itemsize) > 96.0 * (1 << 20);
+}
+
+// Whether the results are stored non-temporally, which keeps the inputs in the
+// Infinity Cache for the next launch that reads them: 512x512x160 FP64 174 -> 168
+// us over three sets of fields in turn, 397x411x137 float32 storage 57 -> 49 us;
+// a vadv launch that reads the result next loses nothing by it.  The price is
+// paid by a launch on cold caches, which without the hint ends with up to
+// 256 MB of its results still in them: 512x512x160 FP64 155 -> 166 us.
+// Rows that start inside a 64-byte line are the exception in fields of more than
+// 128 MB: tiles beside each other then share lines that the hint writes in two
+// parts, 512x512x160 without padding FP64 173.6 us plain, 177.1 with the hint
+// (float32 94.2 / 96.9), 1024x1024x80 333 / 345 and 175 / 186, 1000x700x40 117.5
+// / 121.6; smaller ones still gain (397x411x137 float32 storage 55.7 -> 53.1,
+// 300x300x120 FP64 51.0 -> 43.8).
+inline bool hdiff_dma_stream(const void *out, int64_t sj, double points, size_t itemsize) {
+    const bool lines = reinterpret_cast<uintptr_t>(out) % 64 == 0 && sj * int64_t(itemsize) % 64 == 0;
+    return lines || points * double(itemsize) <= 128.0 * (1 << 20);
 }
 
 // Rows that one launch of the LDS-DMA tile takes: the tile addresses a plane by

@@ -76,8 +76,28 @@ static int check_bands() {
     return 0;
 }
 
+// Non-temporal stores: rows of whole 64-byte lines, or up to 128 MB of results.
+static int check_stores() {
+    const struct { uintptr_t out; int64_t sj; double points; size_t size; bool stream; } cases[] = {
+        {256, 520, 512.0 * 512 * 160, 8, true},     // padded rows
+        {256, 518, 512.0 * 512 * 160, 8, false},    // rows end inside a line
+        {264, 520, 512.0 * 512 * 160, 8, false},    // and start inside one
+        {256, 528, 512.0 * 512 * 160, 4, true},     {256, 520, 512.0 * 512 * 160, 4, false},
+        {256, 403, 397.0 * 411 * 137, 4, true},     {256, 403, 397.0 * 411 * 137, 8, false},
+        {256, 134, 128.0 * 128 * 80, 8, true},      {4, 1, 1 << 25, 4, true},
+        {4, 1, (1 << 25) + 1, 4, false},
+    };
+    for (const auto &c : cases)
+        if (sb::hdiff_dma_stream(reinterpret_cast<const void *>(c.out), c.sj, c.points, c.size) != c.stream) {
+            std::printf("stores of %g points of %zu bytes, pitch %lld, origin %zu: expected %d\n", c.points,
+                        c.size, (long long)c.sj, size_t(c.out), int(c.stream));
+            return 1;
+        }
+    return 0;
+}
+
 int main() {
-    if (check_bands()) return 1;
+    if (check_bands() || check_stores()) return 1;
     const int64_t widths[] = {1, 2, 3, 4, 5, 6, 7, 8, 61, 62, 63, 64, 65, 66, 67, 125, 126, 127, 128, 129, 131};
     const int64_t heights[] = {1, 7, 8, 9, 15, 16, 17, 33};
     for (int64_t nx : widths)

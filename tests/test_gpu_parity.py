@@ -330,6 +330,22 @@ def test_hdiff_partial_tiles(gpu, prec, domain, halo, alignment):
     _check_halo(got, domain, halo)
 
 
+# results of more than 128 MB in rows that start inside a line are stored
+# plainly: whole and partial tiles, by 16-byte units and by words
+@pytest.mark.parametrize("prec,domain,alignment", [("f64", (512, 512, 65), 16), ("f64", (397, 411, 103), 0),
+                                                   ("f32_f64", (512, 512, 129), 0),
+                                                   ("f32", (1021, 700, 48), 16)])
+def test_hdiff_large_unaligned_rows(gpu, prec, domain, alignment):
+    halo, dtype = (3, 3, 3), _dtype(prec)
+    inp, coeff = make_fields(domain, halo, dtype, (2, 1, 0), alignment, count=2, seed=sum(domain))
+    out = _with_sentinel(make_fields(domain, halo, dtype, (2, 1, 0), alignment)[0])
+    assert np.prod(domain) * out.itemsize > 128 << 20 and out.strides[1] % 64
+    got, = _run(gpu, "sb_hdiff", [inp, coeff, out], [2], domain, halo, _prec(gpu, prec))
+    expected = _expected(lambda a, b: oracle.hdiff(a, b, domain, halo), [inp, coeff], prec)
+    assert np.array_equal(got[inner(domain, halo)], expected)
+    _check_halo(got, domain, halo)
+
+
 # a k-plane beyond 4 GiB, rows at the widest pitch: several launches of the
 # LDS-DMA tile, the last one of whole and of partial tiles
 @pytest.mark.parametrize("prec", ["f64", "f32_f64"])
