@@ -382,18 +382,22 @@ __global__ __launch_bounds__(64 * kWsWaves) void vadv_ws_kernel(Components comps
 // highest NR levels in registers and of the rest in LDS (vadv_regs.h).  An
 // item is one component of a group, components innermost: the solves that
 // read the same wcon run side by side, and all of a small domain's at once.
-// A grid of every resident wave walks the items in rounds of consecutive
-// ones, or (SPREAD) every item is a workgroup of its own; either way
-// neighbouring items run on one XCD, whose L2 fetches the cache lines at
-// their edges once.
-template <typename T, typename C, int BUILD, bool NT, bool SPREAD>
+// Every item is a workgroup: the dispatcher starts one wherever another ends,
+// while a grid of the resident waves that walks the items in rounds leaves its
+// last round part empty (FP64 400x400x40, 2500 items on 2048 waves, 73 -> 60 us;
+// 512x512x160 393 -> 379).  Neighbouring items run on one XCD, whose L2 fetches
+// the cache lines at their edges once: runs of `chunk` items, all of an XCD's
+// share in one run where every item is in flight at once (128x128x80 three
+// components float32 storage 3-7 % faster than runs of 16).
+// The loop takes one turn; the kernel written without it is scheduled worse
+// (128x128x80 FP64 15.4 us, 14.8 with it).
+template <typename T, typename C, int BUILD, bool NT>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(RegBuilds<T, C>::of[BUILD].waves_per_simd)))
-void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
+void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a, uint32_t chunk) {
     extern __shared__ unsigned char lds_raw[];
     const uint32_t ncomp = uint32_t(a.ncomp), items = uint32_t(a.ngroups) * ncomp;
-    const uint32_t slot = SPREAD ? xcd_chunk_remap(blockIdx.x, gridDim.x, a.xcds, kRegItemsPerXcd)
-                                 : xcd_remap(blockIdx.x, gridDim.x, a.xcds);
+    const uint32_t slot = xcd_chunk_remap(blockIdx.x, gridDim.x, a.xcds, chunk);
     for (uint32_t n = slot; n < items; n += gridDim.x) {
         const uint32_t g = n / ncomp;
         const Component &cp = comps.c[n - g * ncomp];
@@ -408,20 +412,14 @@ void vadv_reg_kernel(Components comps, const T *__restrict__ wcon, PipeArgs a) {
 template <typename T, typename C, int BUILD, bool NT>
 hipError_t launch_reg_k(const RegShape &shape, uint64_t items, const Components &comps,
                         const T *wcon, const PipeArgs &pa, Context *ctx) {
-    // float32 fields: one workgroup per item.  The last of a few rounds of
-    // resident waves would be part empty, which costs a wave bound by its own
-    // instructions (512x512x160: 230 -> 216 us, 512x512x80: 113 -> 109 us);
-    // FP64 fields are bound by memory and read it more evenly in rounds
-    // (512x512x80: 202 -> 189 us, 400x400x137: 212 -> 198 us).
-    constexpr bool SPREAD = sizeof(T) == 4;
-    const uint64_t resident = uint64_t(shape.per_cu) * uint64_t(ctx->compute_units);
-    const uint64_t grid = SPREAD ? items : std::min(items, resident);
     PipeArgs args = pa;
-    args.xcds = grid >= uint64_t(ctx->xcds) ? uint32_t(ctx->xcds) : 1u;
-    const void *fn = reinterpret_cast<const void *>(&vadv_reg_kernel<T, C, BUILD, NT, SPREAD>);
+    args.xcds = items >= uint64_t(ctx->xcds) ? uint32_t(ctx->xcds) : 1u;
+    const bool at_once = items <= uint64_t(shape.per_cu) * uint64_t(ctx->compute_units);
+    const uint32_t chunk = at_once ? uint32_t(items) / args.xcds : kRegItemsPerXcd;
+    const void *fn = reinterpret_cast<const void *>(&vadv_reg_kernel<T, C, BUILD, NT>);
     (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(shape.lds_bytes));
-    enqueue_kernel((vadv_reg_kernel<T, C, BUILD, NT, SPREAD>), dim3(unsigned(grid)), dim3(64),
-                   shape.lds_bytes, ctx->stream, comps, wcon, args);
+    enqueue_kernel((vadv_reg_kernel<T, C, BUILD, NT>), dim3(unsigned(items)), dim3(64),
+                   shape.lds_bytes, ctx->stream, comps, wcon, args, chunk);
     return hipGetLastError();
 }
 
