@@ -569,21 +569,6 @@ hipError_t launch_ws(int block, bool nt, bool fast, int per_cu_limit, uint64_t b
                                        ctx);
 }
 
-// Whether variant 5 loads stage, tens and tensstage (each read once) with the
-// non-temporal hint, which leaves L2 and the Infinity Cache to pos, read a
-// second time by the backward sweep, and to wcon, shared with the neighbour
-// columns (hints on those two as well measured up to 20 % slower than none).
-// FP64 fields: always (512x512x160 437 -> 400 us, 256x256x80 54 -> 47 us).
-// Float32 fields: where groups are whole chunks of aligned rows, or one
-// component is larger than the Infinity Cache (512x512x160 239 -> 217 us,
-// 313x327x100 59 -> 49 us): elsewhere neighbouring groups share a line that
-// the hint drops too early (301x283x60 without row padding 30.6 -> 32.5 us,
-// 500x500x40 all components 150 -> 171 us).
-inline bool stream_hint(size_t itemsize, bool aligned, int ncomp, uint64_t field_bytes) {
-    if (itemsize == 8 || aligned) return true;
-    return ncomp == 1 && 5 * field_bytes > (uint64_t(256) << 20);
-}
-
 // The fields that a call reads and writes, in argument order.
 struct FieldList {
     void *const *f;
@@ -662,17 +647,22 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
                            uint64_t(last_elem + 1) * sizeof(T) < (uint64_t(1) << 32);
     // default: one wave per group with register levels (variant 5) wherever
     // its columns fit (measured on MI355X against the fastest of the others,
-    // in us: 32x32x80 FP64 14.7 / 16.4, 128x128x80 16.6 / 18.4, 512x512x160
-    // 387 / 421, 512x512x12 36 / 36; float32 storage 512x512x160 216 / 262,
-    // 200x200x137 29 / 55, 301x283x60 all components 68 / 115); fields of
-    // 4 GiB and up or with negative strides take variant 1, taller columns
-    // the global scratch
+    // in us: 32x32x80 FP64 14.7 / 16.4, 128x128x80 14.8 / 18.4, 512x512x160
+    // 379 / 421; float32 storage 512x512x160 216 / 262, 200x200x137 29 / 55,
+    // 301x283x60 all components 61 / 115) except short columns (reg_default);
+    // fields of 4 GiB and up or with negative strides take variant 1, taller
+    // columns the global scratch
     const ColumnRow row = padded_row(g->nx, g->si, g->sj, sizeof(T), fields_of(f, a.ncomp));
     const int64_t reg_groups = vadv_groups(row.lanes, g->ny);
     const uint64_t items = uint64_t(reg_groups) * uint64_t(a.ncomp);
     const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block,
                                          reg_waves_needed(items, uint64_t(ctx->compute_units)));
-    if (variant == 0) variant = buffer_ok && reg.per_cu > 0 ? 5 : lds_fits ? 1 : 2;
+    if (variant == 0) {
+        if (!buffer_ok || reg.per_cu == 0)
+            variant = lds_fits ? 1 : 2;
+        else
+            variant = reg_default<T, C>(reg, items, uint64_t(ctx->compute_units)) ? 5 : 3;
+    }
     SB_REQUIRE(variant >= 1 && variant <= 5, "vadv variant %d not available", variant);
     if (variant == 5) {
         SB_REQUIRE(reg.per_cu > 0, "vadv variant 5 keeps at most %lld levels in registers and LDS, got nz = %lld",
@@ -683,7 +673,9 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
                     uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds), row.lanes};
         const int hint = l ? l->bz : 0;
         const bool nt = hint ? hint > 0 && (hint & 1)
-                             : stream_hint(sizeof(T), row.aligned, a.ncomp, uint64_t(last_elem) * sizeof(T));
+                             : stream_hint<T, C>(reg, row.aligned, a.ncomp,
+                                                 double(a.nx) * double(a.ny) * double(a.nz),
+                                                 uint64_t(last_elem) * sizeof(T));
         return timed_launch(l, seconds, [&]() -> hipError_t {
             return launch_reg<T, C>(reg, nt, items, comps, wcon, pa, ctx);
         });

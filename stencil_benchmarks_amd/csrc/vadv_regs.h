@@ -179,6 +179,45 @@ RegShape reg_shape(int64_t nz, size_t lds, uint64_t need) {
     return uint64_t(keeps.per_cu) >= std::min(uint64_t(most.per_cu), need) ? keeps : most;
 }
 
+// Whether variant 5 loads stage, tens and tensstage (each read once) with the
+// non-temporal hint, which leaves L2 and the Infinity Cache to pos, read a
+// second time by the backward sweep, and to wcon, shared with the neighbour
+// columns (hints on those two as well measured up to 20 % slower than none).
+// FP64 fields: always (512x512x160 437 -> 400 us, 256x256x80 54 -> 47 us).
+// Float32 fields: where groups are whole chunks of aligned rows, or one
+// component is larger than the Infinity Cache (512x512x160 239 -> 217 us,
+// 313x327x100 59 -> 49 us): elsewhere neighbouring groups share a line that
+// the hint drops too early (301x283x60 without row padding 30.6 -> 32.5 us,
+// 500x500x40 all components 150 -> 171 us).
+// Short columns, those without register levels, read pos again before it has
+// left the caches, so the hint gains only where a call's fields are about as
+// large as the Infinity Cache (600x600x12 FP64, 173 MB: 49 us plain, 45 with
+// it); smaller fields lose what the cache holds of them from the call before
+// (512x512x4 14.2 / 17.4, 600x600x8 float32 storage 14.6 / 18.1), larger ones
+// 1 to 14 % (1024x1024x8 three components FP64 264 / 288, float32 123 / 140).
+// `points` are the domain's, `field_bytes` include the halo.
+template <typename T, typename C>
+bool stream_hint(const RegShape &shape, bool aligned, int ncomp, double points,
+                 uint64_t field_bytes) {
+    if (RegBuilds<T, C>::of[shape.build].nr == 0) {
+        const double mb = (4 * ncomp + 1) * points * double(sizeof(T)) / (1 << 20);
+        return (sizeof(T) == 8 || aligned) && mb > 128.0 && mb <= 320.0;
+    }
+    if (sizeof(T) == 8 || aligned) return true;
+    return ncomp == 1 && 5 * field_bytes > (uint64_t(256) << 20);
+}
+
+// Whether variant 5 is the default for the columns it takes: not for short FP64
+// columns, those without register levels, beyond what a device holds at once.
+// The single-wave pipeline (variant 3), which loads the next group while the
+// last one finishes, is up to 9 % faster there (450x450x12 26.4 us, 28.4 here;
+// 1024x1024x4 three components 155 / 168) and never much slower.
+template <typename T, typename C>
+bool reg_default(const RegShape &shape, uint64_t items, uint64_t cus) {
+    return !(sizeof(T) == 8 && RegBuilds<T, C>::of[shape.build].nr == 0 &&
+             items > uint64_t(shape.per_cu) * cus);
+}
+
 template <typename T, typename C, int NR, int PF, int AUX, bool POS>
 struct RegColumn {
     static_assert(NR == 0 || (NR % PF == 0 && NR >= 2 * PF), "register levels: whole prefetch blocks");

@@ -556,6 +556,20 @@ def test_vadv_register_builds_many_columns(gpu, prec, nz):
     assert np.array_equal(got[inner(domain, halo)], expected)
 
 
+# short columns beyond what a device holds at once, with every cache hint
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("domain", [(641, 340, 2), (640, 340, 9), (641, 340, 17), (1024, 520, 6)])
+def test_vadv_short_columns_default(gpu, prec, domain):
+    halo = (1, 1, 0)
+    fields = make_fields(domain, halo, _dtype(prec), count=8, seed=sum(domain), alignment=64)
+    expected = _expected(lambda *f: oracle.vadv(*f, domain, halo), fields[:5], prec)
+    for variant, hint in ((0, 0), (5, -1), (5, 1)):
+        got, = _run_vadv(gpu, fields, [3], domain, halo, _prec(gpu, prec), False, variant,
+                         extra=dict(bz=hint))
+        # one float32 pivot is exactly zero: its column is NaN in both
+        assert np.array_equal(got[inner(domain, halo)], expected, equal_nan=True), (variant, hint)
+
+
 # rows padded to whole 128- or 64-byte chunks of lanes (vadv_regs.h): the
 # lanes past a row's end repeat its last column; 64-byte aligned fields with
 # odd and even multiples of 64 bytes as row pitch, one of unaligned rows

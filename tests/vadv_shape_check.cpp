@@ -26,8 +26,52 @@ static int check_remap() {
     return 0;
 }
 
+constexpr size_t kLds = 160 << 10;  // of a CU
+constexpr uint64_t kCus = 256;
+
+template <typename T, typename C>
+static sb::RegShape shape_of(int64_t nz, uint64_t items) {
+    return sb::reg_shape<T, C>(nz, kLds, sb::reg_waves_needed(items, kCus));
+}
+
+// Short columns: the default solver and the cache hint.
+static int check_short_columns() {
+    const struct { int64_t nz, nx, ny; int ncomp; bool own, hint; } fp64[] = {
+        {4, 128, 128, 1, true, false},    {17, 313, 327, 1, true, false},  // all in flight
+        {4, 512, 512, 1, false, false},   {17, 512, 512, 1, false, true},  // beyond it
+        {4, 1024, 1024, 3, false, false}, {12, 1024, 1024, 3, false, false},
+        {40, 512, 512, 1, true, true},    {80, 128, 128, 3, true, true},   // register levels
+    };
+    for (const auto &c : fp64) {
+        const uint64_t items = uint64_t(c.nx * c.ny / 64 * c.ncomp);
+        const sb::RegShape s = shape_of<double, double>(c.nz, items);
+        const double points = double(c.nx * c.ny * c.nz);
+        const uint64_t bytes = uint64_t(points) * 8;
+        if (sb::reg_default<double, double>(s, items, kCus) != c.own ||
+            sb::stream_hint<double, double>(s, true, c.ncomp, points, bytes) != c.hint) {
+            std::printf("FP64 %lldx%lldx%lld x%d: default %d, hint %d\n", (long long)c.nx, (long long)c.ny,
+                        (long long)c.nz, c.ncomp, int(sb::reg_default<double, double>(s, items, kCus)),
+                        int(sb::stream_hint<double, double>(s, true, c.ncomp, points, bytes)));
+            return 1;
+        }
+    }
+    // float32 storage keeps the solver; the hint goes by the bytes and the rows
+    for (int64_t nz : {8, 12, 60})
+        for (bool aligned : {false, true}) {
+            const sb::RegShape s = shape_of<float, double>(nz, 1024 * 1024 / 64);
+            const double points = 1024.0 * 1024 * double(nz);
+            const bool hint = sb::stream_hint<float, double>(s, aligned, 1, points, uint64_t(points) * 4);
+            const bool expected = nz == 60 ? true : nz == 8 ? aligned : aligned && 5 * nz * 4 <= 320;
+            if (!sb::reg_default<float, double>(s, 1024 * 1024 / 64, kCus) || hint != expected) {
+                std::printf("float32 storage nz %lld aligned %d: hint %d\n", (long long)nz, int(aligned), int(hint));
+                return 1;
+            }
+        }
+    return 0;
+}
+
 int main() {
-    if (check_remap()) return 1;
+    if (check_remap() || check_short_columns()) return 1;
     std::printf("ok\n");
     return 0;
 }
