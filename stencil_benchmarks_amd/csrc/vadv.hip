@@ -649,19 +649,33 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
     // its columns fit (measured on MI355X against the fastest of the others,
     // in us: 32x32x80 FP64 14.7 / 16.4, 128x128x80 14.8 / 18.4, 512x512x160
     // 379 / 421; float32 storage 512x512x160 216 / 262, 200x200x137 29 / 55,
-    // 301x283x60 all components 61 / 115) except short columns (reg_default);
-    // fields of 4 GiB and up or with negative strides take variant 1, taller
-    // columns the global scratch
+    // 301x283x60 all components 61 / 115) except some short and tall columns
+    // (reg_default); fields of 4 GiB and up or with negative strides take
+    // variant 1, taller columns the global scratch
     const ColumnRow row = padded_row(g->nx, g->si, g->sj, sizeof(T), fields_of(f, a.ncomp));
     const int64_t reg_groups = vadv_groups(row.lanes, g->ny);
     const uint64_t items = uint64_t(reg_groups) * uint64_t(a.ncomp);
     const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block,
                                          reg_waves_needed(items, uint64_t(ctx->compute_units)));
+    const bool reg_fits = buffer_ok && reg.per_cu > 0;
+    // the best of variants 1 to 4: the warp-specialised solver where every
+    // workgroup gets at least two groups of tall enough columns (float32
+    // storage, against the pipeline: 512x512x64 1.24x, 512x512x48 1.07x,
+    // 512x512x40 0.84x; FP64 512x512x160 1.18x, 256x256x80 0.96x), the pipeline
+    // where LDS holds the column
+    auto other_solver = [&] {
+        const bool ws = ws_lds_bytes<C>(g->nz) <= ctx->lds_per_block && buffer_ok &&
+                        uint64_t(last_elem + 1 + g->sk) * sizeof(T) < kWsDropOffset &&
+                        g->nz >= (sizeof(T) == 8 ? 96 : 48) &&
+                        groups >= 2 * int64_t(ctx->compute_units);
+        return ws ? 4 : lds_fits ? (buffer_ok ? 3 : 1) : reg_fits ? 5 : 2;
+    };
     if (variant == 0) {
-        if (!buffer_ok || reg.per_cu == 0)
+        if (!reg_fits)
             variant = lds_fits ? 1 : 2;
         else
-            variant = reg_default<T, C>(reg, items, uint64_t(ctx->compute_units)) ? 5 : 3;
+            variant = reg_default<T, C>(reg, a.ncomp, items, uint64_t(ctx->compute_units))
+                          ? 5 : other_solver();
     }
     SB_REQUIRE(variant >= 1 && variant <= 5, "vadv variant %d not available", variant);
     if (variant == 5) {

@@ -207,15 +207,26 @@ bool stream_hint(const RegShape &shape, bool aligned, int ncomp, double points,
     return ncomp == 1 && 5 * field_bytes > (uint64_t(256) << 20);
 }
 
-// Whether variant 5 is the default for the columns it takes: not for short FP64
-// columns, those without register levels, beyond what a device holds at once.
-// The single-wave pipeline (variant 3), which loads the next group while the
-// last one finishes, is up to 9 % faster there (450x450x12 26.4 us, 28.4 here;
-// 1024x1024x4 three components 155 / 168) and never much slower.
+// Whether variant 5 is the default for the columns it takes.  Not for
+//   - short FP64 columns, those without register levels, beyond what a device
+//     holds at once: the single-wave pipeline (variant 3), which loads the next
+//     group while the last one finishes, is up to 9 % faster there (450x450x12
+//     26.4 us, 28.4 here; 1024x1024x4 three components 155 / 168) and never
+//     much slower;
+//   - tall columns of float32 arithmetic, whose levels beyond the 80 in
+//     registers leave LDS for two waves or one a CU: variants 4 and 3 take nz
+//     <= 320 with four waves a CU, or one with two groups in its pipeline.  One
+//     wave a CU (us, here / they): 512x512x300 1071 / 529, 128x128x300 64 / 52,
+//     but three components of few columns 100x90x300 121 / 149.  Two waves:
+//     181x181x201 79 / 58, 512x512x201 396 / 368, 64x64x201 39 / 35, but
+//     160x150x201 46 / 57 and three components of 301x283x201 402 / 428.
 template <typename T, typename C>
-bool reg_default(const RegShape &shape, uint64_t items, uint64_t cus) {
-    return !(sizeof(T) == 8 && RegBuilds<T, C>::of[shape.build].nr == 0 &&
-             items > uint64_t(shape.per_cu) * cus);
+bool reg_default(const RegShape &shape, int ncomp, uint64_t items, uint64_t cus) {
+    const uint64_t at_once = uint64_t(shape.per_cu) * cus;
+    if (sizeof(T) == 8 && RegBuilds<T, C>::of[shape.build].nr == 0) return items <= at_once;
+    if (sizeof(C) == 8 || shape.per_cu > 2) return true;
+    if (ncomp == 1) return shape.per_cu == 2 && items > cus && items <= at_once;
+    return items <= (shape.per_cu == 2 ? 20 : 2) * cus;
 }
 
 template <typename T, typename C, int NR, int PF, int AUX, bool POS>

@@ -570,6 +570,21 @@ def test_vadv_short_columns_default(gpu, prec, domain):
         assert np.array_equal(got[inner(domain, halo)], expected, equal_nan=True), (variant, hint)
 
 
+# tall columns of float32 arithmetic, three, two and one wave a CU: the default
+# is variant 3, 4 or 5 by the number of column groups
+@pytest.mark.parametrize("domain,components", [((70, 9, 186), 1), ((70, 9, 201), 1), ((300, 80, 201), 1),
+                                               ((330, 101, 201), 1), ((70, 9, 300), 1), ((300, 80, 300), 3),
+                                               ((330, 101, 267), 1), ((70, 9, 320), 3), ((70, 9, 321), 1)])
+def test_vadv_tall_float32_columns(gpu, domain, components):
+    halo = (1, 1, 0)
+    names = ("u", "v", "w")[:components]
+    fields = make_fields(domain, halo, np.float32, count=16 if components == 3 else 8, seed=sum(domain))
+    got = _run_vadv(gpu, fields, [4 * q + 3 for q in range(components)], domain, halo, gpu.SB_F32,
+                    components == 3, 0)
+    for g, e in zip(got, _vadv_expected(fields, domain, halo, "f32", names)):
+        assert np.array_equal(g[inner(domain, halo)], e, equal_nan=True)
+
+
 # rows padded to whole 128- or 64-byte chunks of lanes (vadv_regs.h): the
 # lanes past a row's end repeat its last column; 64-byte aligned fields with
 # odd and even multiples of 64 bytes as row pitch, one of unaligned rows

@@ -47,10 +47,10 @@ static int check_short_columns() {
         const sb::RegShape s = shape_of<double, double>(c.nz, items);
         const double points = double(c.nx * c.ny * c.nz);
         const uint64_t bytes = uint64_t(points) * 8;
-        if (sb::reg_default<double, double>(s, items, kCus) != c.own ||
+        if (sb::reg_default<double, double>(s, c.ncomp, items, kCus) != c.own ||
             sb::stream_hint<double, double>(s, true, c.ncomp, points, bytes) != c.hint) {
             std::printf("FP64 %lldx%lldx%lld x%d: default %d, hint %d\n", (long long)c.nx, (long long)c.ny,
-                        (long long)c.nz, c.ncomp, int(sb::reg_default<double, double>(s, items, kCus)),
+                        (long long)c.nz, c.ncomp, int(sb::reg_default<double, double>(s, c.ncomp, items, kCus)),
                         int(sb::stream_hint<double, double>(s, true, c.ncomp, points, bytes)));
             return 1;
         }
@@ -62,7 +62,7 @@ static int check_short_columns() {
             const double points = 1024.0 * 1024 * double(nz);
             const bool hint = sb::stream_hint<float, double>(s, aligned, 1, points, uint64_t(points) * 4);
             const bool expected = nz == 60 ? true : nz == 8 ? aligned : aligned && 5 * nz * 4 <= 320;
-            if (!sb::reg_default<float, double>(s, 1024 * 1024 / 64, kCus) || hint != expected) {
+            if (!sb::reg_default<float, double>(s, 1, 1024 * 1024 / 64, kCus) || hint != expected) {
                 std::printf("float32 storage nz %lld aligned %d: hint %d\n", (long long)nz, int(aligned), int(hint));
                 return 1;
             }
@@ -70,8 +70,37 @@ static int check_short_columns() {
     return 0;
 }
 
+// Tall columns: the default solver of float32 arithmetic; FP64 arithmetic has
+// no other one beyond the LDS and keeps this one up to there.
+static int check_tall_columns() {
+    const struct { int64_t nz, groups; int ncomp; bool own; } cases[] = {
+        {160, 4096, 1, true},  {186, 4096, 3, true},                         // three waves a CU
+        {201, 64, 1, false},   {201, 375, 1, true},   {201, 625, 1, false},  // two
+        {201, 625, 3, true},   {201, 4096, 3, false},
+        {300, 64, 1, false},   {300, 375, 1, false},  {300, 141, 3, true},   // one
+        {300, 4096, 3, false},
+    };
+    for (const auto &c : cases) {
+        const uint64_t items = uint64_t(c.groups * c.ncomp);
+        const sb::RegShape s = shape_of<float, float>(c.nz, items);
+        if (s.per_cu == 0 || sb::reg_default<float, float>(s, c.ncomp, items, kCus) != c.own) {
+            std::printf("float32 nz %lld, %lld groups x%d: %d waves a CU, default %d\n", (long long)c.nz,
+                        (long long)c.groups, c.ncomp, s.per_cu, int(!c.own));
+            return 1;
+        }
+        const sb::RegShape d = shape_of<double, double>(std::min<int64_t>(c.nz, 201), items);
+        const sb::RegShape m = shape_of<float, double>(std::min<int64_t>(c.nz, 201), items);
+        if (!sb::reg_default<double, double>(d, c.ncomp, items, kCus) ||
+            !sb::reg_default<float, double>(m, c.ncomp, items, kCus)) {
+            std::printf("FP64 arithmetic, %lld groups x%d: not the default\n", (long long)c.groups, c.ncomp);
+            return 1;
+        }
+    }
+    return 0;
+}
+
 int main() {
-    if (check_remap() || check_short_columns()) return 1;
+    if (check_remap() || check_short_columns() || check_tall_columns()) return 1;
     std::printf("ok\n");
     return 0;
 }
