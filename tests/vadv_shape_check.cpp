@@ -99,7 +99,29 @@ static int check_tall_columns() {
     return 0;
 }
 
+// The waves counted on a CU fit its LDS, which is allocated in granules of
+// 1280 bytes, and its registers.
+template <typename T, typename C>
+static int check_waves(const char *name) {
+    for (int64_t nz = 2; nz <= sb::reg_max_levels<C>(); ++nz)
+        for (uint64_t need = 1; need <= 20; ++need) {
+            const sb::RegShape s = sb::reg_shape<T, C>(nz, kLds, need);
+            const sb::RegLevels &levels = sb::RegBuilds<T, C>::of[s.build];
+            const size_t taken = (s.lds_bytes + 1279) / 1280 * 1280;
+            if (s.per_cu < 1 || s.per_cu > 4 * levels.waves_per_simd ||
+                size_t(s.per_cu) * taken > kLds || nz < levels.nr + 2) {
+                std::printf("%s nz %lld: build %d, %d waves of %zu bytes\n", name, (long long)nz, s.build,
+                            s.per_cu, s.lds_bytes);
+                return 1;
+            }
+        }
+    return 0;
+}
+
 int main() {
+    if (check_waves<double, double>("FP64") || check_waves<float, double>("float32 storage") ||
+        check_waves<float, float>("float32"))
+        return 1;
     if (check_remap() || check_short_columns() || check_tall_columns()) return 1;
     std::printf("ok\n");
     return 0;
