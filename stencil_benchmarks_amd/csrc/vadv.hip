@@ -670,9 +670,19 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
                         groups >= 2 * int64_t(ctx->compute_units);
         return ws ? 4 : lds_fits ? (buffer_ok ? 3 : 1) : reg_fits ? 5 : 2;
     };
+    // options that only the other solvers have (workgroups per CU, prefetch
+    // depth, fast reciprocal) choose among those without a variant too, which
+    // check their values; calls of few columns, whose groups four waves a CU
+    // hold at once (three from 82 levels of FP64 arithmetic on, two from 90),
+    // have register columns whatever the options
+    const bool options = l && (l->bx || l->unroll || (l->bz > 0 && (l->bz & ~1)));
+    const int few_per_cu = sizeof(C) == 4 || g->nz <= 81 ? 4 : g->nz <= 89 ? 3 : 2;
+    const bool few = g->nz <= 96 && groups <= few_per_cu * int64_t(ctx->compute_units);
     if (variant == 0) {
         if (!reg_fits)
             variant = lds_fits ? 1 : 2;
+        else if (options && !few)
+            variant = other_solver();
         else
             variant = reg_default<T, C>(reg, a.ncomp, items, uint64_t(ctx->compute_units))
                           ? 5 : other_solver();

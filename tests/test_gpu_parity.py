@@ -669,6 +669,39 @@ def test_vadv_fast_reciprocal_needs_float32_storage(gpu):
         _run_vadv(gpu, fields, [3], domain, halo, gpu.SB_F64, False, 4, extra=dict(bz=4))
 
 
+# options without a variant are checked by the solver that has them
+@pytest.mark.parametrize("prec,domain,options,match", [
+    ("f64", (700, 101, 9), dict(bz=4), "fast reciprocal"),
+    ("f32", (700, 101, 60), dict(bz=5), "fast reciprocal"),
+    ("f32_f64", (700, 101, 9), dict(bz=4), "fast reciprocal"),  # the pipeline has none
+    ("f64", (700, 101, 9), dict(unroll=5), "prefetch depth 5"),
+    ("f32_f64", (700, 101, 50), dict(unroll=2), "prefetch depth 2")])
+def test_vadv_default_rejects_options(gpu, prec, domain, options, match):
+    from stencil_benchmarks_amd.benchmark import ExecutionError
+
+    fields = make_fields(domain, (1, 0, 0), _dtype(prec), count=8, seed=1)
+    with pytest.raises(ExecutionError, match=match):
+        _run_vadv(gpu, fields, [3], domain, (1, 0, 0), _prec(gpu, prec), False, 0, extra=options)
+
+
+# and honoured: the fast reciprocal gives the bits it gives variant 4; a call of
+# few columns keeps the register columns
+def test_vadv_default_takes_options(gpu):
+    domain, halo = (700, 101, 50), (1, 0, 0)
+    fields = make_fields(domain, halo, np.float32, count=8, seed=5)
+    run = lambda d, f, variant, **extra: _run_vadv(  # noqa: E731
+        gpu, f, [3], d, halo, gpu.SB_F32_F64, False, variant, extra=extra)[0][inner(d, halo)]
+    exact = run(domain, fields, 0)
+    fast = run(domain, fields, 0, bz=5)
+    assert np.array_equal(fast, run(domain, fields, 4, bz=5))
+    assert not np.array_equal(fast, exact)
+    for extra in (dict(unroll=8), dict(bx=1), dict(unroll=16, bz=1)):
+        assert np.array_equal(run(domain, fields, 0, **extra), exact), extra
+    small = (64, 4, 20)
+    fields = make_fields(small, halo, np.float32, count=8, seed=6)
+    assert np.array_equal(run(small, fields, 0, bz=5, unroll=5, bx=3), run(small, fields, 5))
+
+
 @pytest.mark.parametrize("flags", [1, 2, 3])
 @pytest.mark.parametrize("variant,depth", [(1, 4), (1, 16), (2, 8)])
 def test_vadv_streaming_options(gpu, flags, variant, depth):
