@@ -5,7 +5,6 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -122,8 +121,8 @@ bool staged_download(Context *ctx, void *dst, const void *src, size_t bytes, int
             workers[w] = std::thread(copy_pieces, ctx->device, ctx->stream, s.piece[w], s.done[w],
                                      static_cast<char *>(dst), static_cast<const char *>(src),
                                      bytes, &next, &error);
-        } catch (const std::system_error &) {
-            break;  // no more threads: the others take its pieces
+        } catch (...) {
+            break;  // no more threads or memory: the others take its pieces
         }
     }
     copy_pieces(ctx->device, ctx->stream, s.piece[0], s.done[0], static_cast<char *>(dst),
