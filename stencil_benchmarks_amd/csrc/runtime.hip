@@ -70,7 +70,10 @@ int usable_cpus() {
 void copy_pieces(int device, hipStream_t stream, char *piece, hipEvent_t done, char *dst,
                  const char *src, size_t bytes, std::atomic<size_t> *next,
                  std::atomic<int> *error) {
-    if (const hipError_t e = hipSetDevice(device); e != hipSuccess) error->store(int(e));
+    if (const hipError_t e = hipSetDevice(device); e != hipSuccess) {
+        (void)hipGetLastError();
+        error->store(int(e));
+    }
     for (;;) {
         const size_t at = next->fetch_add(kPieceBytes);
         if (at >= bytes || error->load() != hipSuccess) return;
@@ -79,6 +82,7 @@ void copy_pieces(int device, hipStream_t stream, char *piece, hipEvent_t done, c
         if (e == hipSuccess) e = hipEventRecord(done, stream);
         if (e == hipSuccess) e = hipEventSynchronize(done);
         if (e != hipSuccess) {
+            (void)hipGetLastError();  // reported by the copy, not by the thread's next call
             error->store(int(e));
             return;
         }

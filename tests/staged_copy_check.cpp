@@ -1,7 +1,8 @@
 // Host-side check of the staged device-to-host copy
 // (stencil_benchmarks_amd/csrc/runtime.hip), with the HIP calls it makes
-// replaced by host ones: a copy is whole where a worker cannot be started.
-// Exits non-zero on the first that is not.
+// replaced by host ones: a copy is whole where a worker cannot be started, and
+// one that fails says so and leaves no error for the next call to report.
+// Exits non-zero on the first that does not.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -15,6 +16,7 @@ void vadv_noalloc_setup(Context &) {}
 
 // ---- the host in place of the device ------------------------------------
 static thread_local hipError_t t_last = hipSuccess;
+static thread_local bool t_fail_copies = false;
 static thread_local long t_allocations_left = -1;  // -1: no limit
 
 void *operator new(size_t n) {
@@ -59,6 +61,7 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
+    if (t_fail_copies) return t_last = hipErrorUnknown;
     std::memcpy(dst, src, n);
     return hipSuccess;
 }
@@ -79,6 +82,17 @@ int main() {
             std::printf("copy with %ld allocations: status %d\n", left, status);
             return 1;
         }
+    }
+    t_fail_copies = true;
+    const int status = sb_memcpy_d2h(dst, src, kBytes);
+    t_fail_copies = false;
+    if (status == 0 || std::strlen(sb_last_error()) == 0) {
+        std::printf("a failed copy reported status %d\n", status);
+        return 1;
+    }
+    if (const hipError_t left = hipGetLastError(); left != hipSuccess) {
+        std::printf("a failed copy left error %d behind\n", int(left));
+        return 1;
     }
     std::printf("ok\n");
     return 0;
