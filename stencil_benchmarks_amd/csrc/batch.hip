@@ -105,6 +105,9 @@ constexpr int kWsGroupsPerItem = 16;
 // launch names it by giving none)
 constexpr int kRegVariant = 5;
 
+// Class of the subdomains that the register-column solver takes
+constexpr int8_t kRegClass = -1;
+
 // One scheduled item of the warp-specialised vadv: subdomain rank, residue.
 struct VItem {
     int32_t rank, residue;
@@ -404,7 +407,9 @@ struct Plan {
         std::vector<int32_t> host_off;
         std::vector<VItem> host_list;
     } ws[2];
-    std::vector<int8_t> host_vclass;  // LDS class of each subdomain (by rank)
+    // LDS class of each subdomain (by rank), or kRegClass
+    std::vector<int8_t> host_vclass;
+    bool ws_items() const { return ws[0].max_nz || ws[1].max_nz; }
     // LDS-DMA hdiff (the default): bytes of its staging unit (0: the queues
     // of register-staged tiles), first item of each subdomain and the total,
     // then the subdomain of every 2^kStartShift-th item
@@ -572,14 +577,33 @@ RegShape batch_reg_shape(int prec, int64_t nz, const Context *ctx) {
     return reg_shape<float, double>(nz, ctx->lds_per_block, 4);
 }
 
+// Subdomains that the warp-specialised solver takes where the caller leaves the
+// choice open: the ones whose columns leave LDS for few register-column waves
+// a CU, if they are many columns (batch_reg_default, vadv_regs.h).
+std::vector<char> tall_subdomains(int prec, const sb_subdomain *subs, const std::vector<int> &order,
+                                  const Context *ctx) {
+    std::vector<char> tall(order.size(), 0);
+    if (prec != SB_F32) return tall;
+    uint64_t groups[3] = {0, 0, 0};  // by the waves that a CU holds
+    auto waves = [&](int i) { return batch_reg_shape(prec, subs[i].geom.nz, ctx).per_cu; };
+    for (int i : order)
+        if (const int w = waves(i); w <= 2) groups[w] += uint64_t(vadv_groups(subs[i].geom.nx, subs[i].geom.ny));
+    for (size_t r = 0; r < order.size(); ++r) {
+        const int w = waves(order[r]);
+        tall[r] = w <= 2 && !batch_reg_default(w, groups[w], uint64_t(ctx->compute_units));
+    }
+    return tall;
+}
+
 // Classes of the register-column vadv, tallest columns first, the subdomains
 // of each in order of decreasing height (the last workgroups to start are the
 // short ones).
 void build_reg_classes(Plan &p, const Context *ctx) {
     p.reg.clear();
     const std::vector<SubDev> &subs = p.host_subs[0];
-    std::vector<int32_t> ranks(subs.size());
-    std::iota(ranks.begin(), ranks.end(), 0);
+    std::vector<int32_t> ranks;
+    for (int32_t r = 0; r < int32_t(subs.size()); ++r)
+        if (p.host_vclass[size_t(r)] == kRegClass) ranks.push_back(r);
     std::stable_sort(ranks.begin(), ranks.end(),
                      [&](int32_t a, int32_t b) { return subs[a].nz > subs[b].nz; });
     std::vector<int32_t> prefix;
@@ -638,19 +662,21 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
     p.max_nz = 2;
     for (int i = 0; i < count; ++i) p.max_nz = std::max<int>(p.max_nz, int(subs[i].geom.nz));
     const int64_t workers = vadv_workers(p, ctx);
-    const bool ws = vadv_variant(&p.vl) == 4;
+    const int variant = vadv_variant(&p.vl);
     p.reg.clear();
-    const int64_t per_item = ws ? vadv_ws_per_item(&p.vl) : kMinGroupsPerItem;
     // warp-specialised solver: columns whose slot buffer fits twice in a
     // CU's LDS (class 0) run in their own launch at two workgroups per CU,
     // the taller ones (class 1) at one
-    p.host_vclass.assign(size_t(count), 0);
+    p.host_vclass.assign(size_t(count), kRegClass);
     for (int c = 0; c < 2; ++c) {
         p.ws[c] = Plan::WsClass{};
     }
-    if (ws) {
+    if (variant == 4 || variant == kRegVariant) {
         const int block = vadv_ws_block(&p.vl);
+        std::vector<char> tall(size_t(count), 1);
+        if (variant == kRegVariant) tall = tall_subdomains(prec, subs, order, ctx);
         for (int r = 0; r < count; ++r) {
+            if (!tall[size_t(r)]) continue;
             const int nz = int(subs[order[r]].geom.nz);
             const int c = 2 * plan_vadv_lds(prec, nz, 4, block) <= ctx->lds_per_block ? 0 : 1;
             p.host_vclass[size_t(r)] = int8_t(c);
@@ -672,8 +698,11 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
                              (g.nz - 1 + g.hk) * g.sk;
         const int64_t tiles_i = (g.nx + 63) / 64;
         const int64_t groups = vadv_groups(g.nx, g.ny);
+        const int cls = p.host_vclass[size_t(r)];
+        const bool ws = cls != kRegClass;
+        const int64_t per_item = ws ? vadv_ws_per_item(&p.vl) : kMinGroupsPerItem;
         const int64_t class_workers =
-            ws ? int64_t(p.ws[p.host_vclass[size_t(r)]].per_cu) * ctx->compute_units : workers;
+            ws ? int64_t(p.ws[cls].per_cu) * ctx->compute_units : workers;
         const int64_t vitems = std::max<int64_t>(1, std::min(class_workers, groups / per_item));
         for (int flip = 0; flip < 2; ++flip) {
             const int cur = (s.parity + flip) & 1;
@@ -709,11 +738,10 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
         p.host_hprefix[r + 1] = p.host_hprefix[r] + hitems;
         p.host_vprefix[r + 1] = p.host_vprefix[r] + vitems;
     }
-    if (ws)
-        for (int c = 0; c < 2; ++c)
-            if (p.ws[c].max_nz)
-                schedule_ws(p, c, p.ws[c].per_cu * ctx->compute_units, vadv_queues(ctx));
-    if (vadv_variant(&p.vl) == kRegVariant) build_reg_classes(p, ctx);
+    for (int c = 0; c < 2; ++c)
+        if (p.ws[c].max_nz)
+            schedule_ws(p, c, p.ws[c].per_cu * ctx->compute_units, vadv_queues(ctx));
+    if (variant == kRegVariant) build_reg_classes(p, ctx);
     if (p.dma_unit) {
         p.host_dma.assign(p.host_hprefix.begin(), p.host_hprefix.end());
         int32_t s = 0;
@@ -792,16 +820,9 @@ hipError_t enqueue_step(const Plan &p, int flip, unsigned long long *counters, C
 #undef SB_HB
     if (return_h != hipSuccess) return return_h;
     // vadv
-    if (vadv_variant(&p.vl) == kRegVariant) {
-        for (const Plan::RegClass &c : p.reg) {
-            const hipError_t e = enqueue_reg_class<T, C>(c, subs, ctx);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
     const unsigned vgrid = vadv_workers(p, ctx);
-    if (vadv_variant(&p.vl) == 4) {
-        // one launch per LDS class, taller columns first
+    if (vadv_variant(&p.vl) != 3) {
+        // one launch per LDS class, taller columns first, then one per register build
         for (int cls = 1; cls >= 0; --cls) {
             const Plan::WsClass &c = p.ws[cls];
             if (!c.max_nz) continue;
@@ -837,6 +858,10 @@ hipError_t enqueue_step(const Plan &p, int flip, unsigned long long *counters, C
             }
             if (e != hipSuccess) return e;
         }
+        for (const Plan::RegClass &c : p.reg) {
+            const hipError_t e = enqueue_reg_class<T, C>(c, subs, ctx);
+            if (e != hipSuccess) return e;
+        }
         return hipSuccess;
     }
     const size_t lds = vadv_lds_bytes<C>(p.max_nz);
@@ -854,7 +879,7 @@ hipError_t enqueue_step(const Plan &p, int flip, unsigned long long *counters, C
 template <typename T, typename C>
 hipError_t enqueue_sequence(const Plan &p, Context *ctx) {
     hipError_t e = hipSuccess;
-    if (!p.dma_unit || vadv_variant(&p.vl) != kRegVariant) {  // there are queues
+    if (!p.dma_unit || p.ws_items() || vadv_variant(&p.vl) == 3) {  // there are queues
         const int ncounters = kCountersPerStep * p.steps;
         hipLaunchKernelGGL(reset_counters, dim3((ncounters + 255) / 256), dim3(256), 0, ctx->stream,
                            p.counters, ncounters);

@@ -236,6 +236,17 @@ bool reg_default(const RegShape &shape, int ncomp, uint64_t items, uint64_t cus)
     return items <= (shape.per_cu == 2 ? 20 : 2) * cus;
 }
 
+// The same for the subdomains of a batch (float32 arithmetic) whose columns leave
+// LDS for `per_cu` waves a CU and that have `groups` together, against the
+// warp-specialised solver, whose workgroups take several groups one after the
+// other.  One step of n times 128x128 columns, in us, register columns / that one:
+//   one wave a CU, 268 levels    n = 6 411 / 498, 8 549 / 526, 10 686 / 550, 14 962 / 600
+//   two, 230 levels              n = 24 883 / 1000, 32 1169 / 1084, 40 1450 / 1545, 64 2332 / 2180
+//   two, 190 levels              n = 32 963 / 897, 48 1434 / 1345, 64 1914 / 1780
+inline bool batch_reg_default(int per_cu, uint64_t groups, uint64_t cus) {
+    return per_cu > 2 || groups <= (per_cu == 2 ? 48 : 7) * cus;
+}
+
 template <typename T, typename C, int NR, int PF, int AUX, bool POS>
 struct RegColumn {
     static_assert(NR == 0 || (NR % PF == 0 && NR >= 2 * PF), "register levels: whole prefetch blocks");

@@ -123,6 +123,33 @@ def test_batch_register_classes(gpu, prec):
     _check(subs, hosts, dtype)
 
 
+def test_batch_tall_float32_columns_take_both_solvers(gpu):
+    """Many tall columns of float32 arithmetic go to the warp-specialised solver,
+    the rest of the batch to register columns, eager and in a replayed graph."""
+    from stencil_benchmarks_amd import batch, native
+
+    # 2601 column groups of 268 levels; the others stay (7 groups a CU at most)
+    domains = [(408, 408, 268), (70, 37, 9), (33, 66, 200), (40, 9, 100)]
+
+    def make():
+        return [batch.Subdomain(d, (3, 3, 3), np.float32, seed=i) for i, d in enumerate(domains)]
+
+    subs, twins = make(), make()
+    plan = batch.Plan(subs, steps=2, compute=np.float32)
+    options = native.launch_options(variant=4)
+    for replay in range(3):
+        plan.run(use_graph=replay != 1)
+        for _ in range(2):
+            batch.step(twins, compute=np.float32, vadv_options=options)
+        for sub, twin in zip(subs, twins):
+            sl = inner(sub.domain, sub.halo)
+            assert np.array_equal(sub.state()[sl], twin.state()[sl]), sub.domain
+            assert np.array_equal(sub.download("utensstage")[sl], twin.download("utensstage")[sl])
+    plan.close()
+    for sub in subs + twins:
+        sub.free()
+
+
 def test_batch_plan_graph_replays_match_eager(gpu):
     from stencil_benchmarks_amd import batch
 

@@ -99,6 +99,25 @@ static int check_tall_columns() {
     return 0;
 }
 
+// The same in a batch, whose subdomains count together.
+static int check_batched_columns() {
+    const struct { int64_t nz, groups; bool own; } cases[] = {
+        {160, 100000, true}, {186, 100000, true},                                  // three waves a CU
+        {201, 48 * 256, true}, {230, 20 * 256, true}, {230, 48 * 256 + 1, false},  // two
+        {250, 7 * 256, true},  {250, 7 * 256 + 1, false},                          // one
+        {300, 64, true},       {320, 4 * 4096, false},
+    };
+    for (const auto &c : cases) {
+        const int per_cu = sb::reg_shape<float, float>(c.nz, kLds, 4).per_cu;
+        if (per_cu == 0 || sb::batch_reg_default(per_cu, uint64_t(c.groups), kCus) != c.own) {
+            std::printf("batch of float32 nz %lld, %lld groups: %d waves a CU\n", (long long)c.nz,
+                        (long long)c.groups, per_cu);
+            return 1;
+        }
+    }
+    return 0;
+}
+
 // The waves counted on a CU fit its LDS, which is allocated in granules of
 // 1280 bytes, and its registers.
 template <typename T, typename C>
@@ -122,7 +141,8 @@ int main() {
     if (check_waves<double, double>("FP64") || check_waves<float, double>("float32 storage") ||
         check_waves<float, float>("float32"))
         return 1;
-    if (check_remap() || check_short_columns() || check_tall_columns()) return 1;
+    if (check_remap() || check_short_columns() || check_tall_columns() || check_batched_columns())
+        return 1;
     std::printf("ok\n");
     return 0;
 }
