@@ -421,7 +421,7 @@ struct Plan {
     struct RegClass {
         int build = 0;
         size_t lds_bytes = 0;           // of its tallest column
-        int64_t aligned_groups = 0;     // of subdomains whose groups are aligned chunks
+        int64_t stream_groups = 0;      // of subdomains that gain by the non-temporal hint
         std::vector<int32_t> host;      // ranks, then prefix sums of their groups
         int32_t *dev = nullptr;
         int count() const { return int(host.size() / 2); }
@@ -578,21 +578,22 @@ RegShape batch_reg_shape(int prec, int64_t nz, const Context *ctx) {
 }
 
 // Subdomains that the warp-specialised solver takes where the caller leaves the
-// choice open: the ones whose columns leave LDS for few register-column waves
-// a CU, if they are many columns (batch_reg_default, vadv_regs.h).
-std::vector<char> tall_subdomains(int prec, const sb_subdomain *subs, const std::vector<int> &order,
-                                  const Context *ctx) {
-    std::vector<char> tall(order.size(), 0);
-    if (prec != SB_F32) return tall;
-    uint64_t groups[3] = {0, 0, 0};  // by the waves that a CU holds
-    auto waves = [&](int i) { return batch_reg_shape(prec, subs[i].geom.nz, ctx).per_cu; };
-    for (int i : order)
-        if (const int w = waves(i); w <= 2) groups[w] += uint64_t(vadv_groups(subs[i].geom.nx, subs[i].geom.ny));
+// choice open: the kinds of columns that register columns are slower for, if
+// they are many (BatchColumns, vadv_regs.h).
+std::vector<char> ws_subdomains(int prec, const sb_subdomain *subs, const std::vector<int> &order,
+                                const Context *ctx) {
+    std::vector<char> ws(order.size(), 0);
+    auto kind = [&](int i) {
+        const sb_geom &g = subs[i].geom;
+        return batch_columns(g.si, g.sj, g.sk, prec == SB_F32, batch_reg_shape(prec, g.nz, ctx).per_cu);
+    };
+    uint64_t groups[kBatchColumnKinds] = {};
+    for (int i : order) groups[kind(i)] += uint64_t(vadv_groups(subs[i].geom.nx, subs[i].geom.ny));
     for (size_t r = 0; r < order.size(); ++r) {
-        const int w = waves(order[r]);
-        tall[r] = w <= 2 && !batch_reg_default(w, groups[w], uint64_t(ctx->compute_units));
+        const BatchColumns k = kind(order[r]);
+        ws[r] = !batch_reg_default(k, groups[k], uint64_t(ctx->compute_units));
     }
-    return tall;
+    return ws;
 }
 
 // Classes of the register-column vadv, tallest columns first, the subdomains
@@ -626,7 +627,9 @@ void build_reg_classes(Plan &p, const Context *ctx) {
         c.host.push_back(r);
         const int32_t groups = int32_t(vadv_groups(subs[r].row, subs[r].ny));
         prefix.push_back((prefix.empty() ? 0 : prefix.back()) + groups);
-        if (subs[r].aligned) c.aligned_groups += groups;
+        // as in the plain kernel (stream_hint, vadv_regs.h): unit i stride, and
+        // for float32 fields groups that are aligned chunks
+        if (subs[r].si == 1 && (p.prec == SB_F64 || subs[r].aligned)) c.stream_groups += groups;
     }
     close();
 }
@@ -673,10 +676,10 @@ void build_tables(int prec, const sb_subdomain *subs, int count, const sb_launch
     }
     if (variant == 4 || variant == kRegVariant) {
         const int block = vadv_ws_block(&p.vl);
-        std::vector<char> tall(size_t(count), 1);
-        if (variant == kRegVariant) tall = tall_subdomains(prec, subs, order, ctx);
+        std::vector<char> ws(size_t(count), 1);
+        if (variant == kRegVariant) ws = ws_subdomains(prec, subs, order, ctx);
         for (int r = 0; r < count; ++r) {
-            if (!tall[size_t(r)]) continue;
+            if (!ws[size_t(r)]) continue;
             const int nz = int(subs[order[r]].geom.nz);
             const int c = 2 * plan_vadv_lds(prec, nz, 4, block) <= ctx->lds_per_block ? 0 : 1;
             p.host_vclass[size_t(r)] = int8_t(c);
@@ -777,9 +780,8 @@ template <typename T, typename C, int BUILD = 0>
 hipError_t enqueue_reg_class(const Plan::RegClass &c, const SubDev *subs, Context *ctx) {
     if constexpr (BUILD + 1 < int(std::size(RegBuilds<T, C>::of)))
         if (c.build != BUILD) return enqueue_reg_class<T, C, BUILD + 1>(c, subs, ctx);
-    // non-temporal loads as in the plain kernel (stream_hint in vadv.hip), for
-    // float32 fields where most groups are aligned chunks
-    const bool stream = sizeof(T) == 8 || 2 * c.aligned_groups > int64_t(c.items());
+    // non-temporal loads where most groups gain by them
+    const bool stream = 2 * c.stream_groups > int64_t(c.items());
     const auto kernel = stream ? vadv_reg_batch_kernel<T, C, BUILD, true>
                                : vadv_reg_batch_kernel<T, C, BUILD, false>;
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),

@@ -415,7 +415,11 @@ hipError_t launch_reg_k(const RegShape &shape, uint64_t items, const Components 
     PipeArgs args = pa;
     args.xcds = items >= uint64_t(ctx->xcds) ? uint32_t(ctx->xcds) : 1u;
     const bool at_once = items <= uint64_t(shape.per_cu) * uint64_t(ctx->compute_units);
-    const uint32_t chunk = at_once ? uint32_t(items) / args.xcds : kRegItemsPerXcd;
+    // rows beside each other share every line where i has no unit stride: an
+    // XCD's share of what is in flight in one run (650x125x184 FP64 1351 -> 1103 us)
+    const uint32_t resident = uint32_t(shape.per_cu) * uint32_t(ctx->compute_units) / args.xcds;
+    const uint32_t chunk = at_once ? uint32_t(items) / args.xcds
+                           : pa.si == 1 ? kRegItemsPerXcd : resident;
     const void *fn = reinterpret_cast<const void *>(&vadv_reg_kernel<T, C, BUILD, NT>);
     (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(shape.lds_bytes));
     enqueue_kernel((vadv_reg_kernel<T, C, BUILD, NT>), dim3(unsigned(items)), dim3(64),
@@ -655,8 +659,19 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
     const ColumnRow row = padded_row(g->nx, g->si, g->sj, sizeof(T), fields_of(f, a.ncomp));
     const int64_t reg_groups = vadv_groups(row.lanes, g->ny);
     const uint64_t items = uint64_t(reg_groups) * uint64_t(a.ncomp);
-    const RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block,
-                                         reg_waves_needed(items, uint64_t(ctx->compute_units)));
+    // Without unit i stride (reg_default_strided): the components of many FP64
+    // columns, or of columns that no other solver but the scratch takes, in
+    // launches of their own, so that three times the rows share their lines at a
+    // time (FP64, rows beside: 640x640x175 24754 us, one after the other
+    // 14459); the latter one wave a CU, with contiguous levels or many items
+    // (456x256x172 1368 us, 990 with one).
+    const uint64_t cus = uint64_t(ctx->compute_units);
+    const bool strided = g->si != 1, levels_inner = g->sk < g->si && g->sk < g->sj;
+    const bool apart = strided && a.ncomp > 1 && (!lds_fits || sizeof(T) == 8) && items > 4 * cus;
+    const uint64_t launched = apart ? uint64_t(reg_groups) : items;
+    RegShape reg = reg_shape<T, C>(g->nz, ctx->lds_per_block, reg_waves_needed(launched, cus));
+    if (strided && !lds_fits && (levels_inner || launched > 4 * cus))
+        reg = reg_limit(reg, 1, ctx->lds_per_block);
     const bool reg_fits = buffer_ok && reg.per_cu > 0;
     // the best of variants 1 to 4: the warp-specialised solver where every
     // workgroup gets at least two groups of tall enough columns (float32
@@ -679,13 +694,11 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
     const int few_per_cu = sizeof(C) == 4 || g->nz <= 81 ? 4 : g->nz <= 89 ? 3 : 2;
     const bool few = g->nz <= 96 && groups <= few_per_cu * int64_t(ctx->compute_units);
     if (variant == 0) {
-        if (!reg_fits)
-            variant = lds_fits ? 1 : 2;
-        else if (options && !few)
-            variant = other_solver();
-        else
-            variant = reg_default<T, C>(reg, a.ncomp, items, uint64_t(ctx->compute_units))
-                          ? 5 : other_solver();
+        const bool own = options    ? few
+                         : !strided ? reg_default<T, C>(reg, a.ncomp, items, cus)
+                                    : reg_default_strided(g->nz, sizeof(C) == 4 && a.ncomp == 1, few,
+                                                          levels_inner, items, cus);
+        variant = !reg_fits ? (lds_fits ? 1 : 2) : own ? 5 : other_solver();
     }
     SB_REQUIRE(variant >= 1 && variant <= 5, "vadv variant %d not available", variant);
     if (variant == 5) {
@@ -697,11 +710,18 @@ int launch_vadv(int all_components, void *const *f, const sb_geom *g, const sb_l
                     uint32_t(uint64_t(last_elem + 1) * sizeof(T)), uint32_t(ctx->xcds), row.lanes};
         const int hint = l ? l->bz : 0;
         const bool nt = hint ? hint > 0 && (hint & 1)
-                             : stream_hint<T, C>(reg, row.aligned, a.ncomp,
-                                                 double(a.nx) * double(a.ny) * double(a.nz),
-                                                 uint64_t(last_elem) * sizeof(T));
+                             : !strided &&
+                                   stream_hint<T, C>(reg, row.aligned, a.ncomp,
+                                                     double(a.nx) * double(a.ny) * double(a.nz),
+                                                     uint64_t(last_elem) * sizeof(T));
         return timed_launch(l, seconds, [&]() -> hipError_t {
-            return launch_reg<T, C>(reg, nt, items, comps, wcon, pa, ctx);
+            if (!apart) return launch_reg<T, C>(reg, nt, items, comps, wcon, pa, ctx);
+            PipeArgs one = pa;
+            one.ncomp = 1;
+            hipError_t e = hipSuccess;
+            for (int c = 0; c < a.ncomp && e == hipSuccess; ++c)
+                e = launch_reg<T, C>(reg, nt, launched, Components{{comps.c[c]}}, wcon, one, ctx);
+            return e;
         });
     }
     SB_REQUIRE(variant == 2 || variant == 4 || lds_fits,

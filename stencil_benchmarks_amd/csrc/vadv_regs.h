@@ -236,15 +236,57 @@ bool reg_default(const RegShape &shape, int ncomp, uint64_t items, uint64_t cus)
     return items <= (shape.per_cu == 2 ? 20 : 2) * cus;
 }
 
-// The same for the subdomains of a batch (float32 arithmetic) whose columns leave
-// LDS for `per_cu` waves a CU and that have `groups` together, against the
+// The same where i has no unit stride, so a lane's accesses are lines of their
+// own: the lines of all waves in flight have to stay in L2 until their other
+// points are used, by the next levels where those are contiguous
+// (`levels_inner`), else by the rows beside.  Register columns hold several
+// times the waves of the other solvers, so beyond some number of items the lines
+// are fetched again and again.  They are the default
+//   - up to 96 levels for the `few` column groups that four waves a CU hold, with
+//     contiguous levels one item a CU (us, here / the others: 32x33x40 float32
+//     15.1 / 15.2, 224x320x43 FP64 283 / 147, 333x293x16 float32 storage 145 / 66;
+//     rows beside 301x336x94 float32 467 / 688, 448x717x89 float32 storage 3056 /
+//     1435);
+//   - above for two items a CU, with contiguous levels half of one (67x22x167
+//     three components float32 51 / 131, 78x159x156 FP64 396 / 216; rows beside
+//     64x274x134 float32 storage 155 / 216, 391x160x172 float32 992 / 614), but not
+//     for one component of float32 arithmetic (`single_float`: 64x128x197 93 / 50).
+inline bool reg_default_strided(int64_t nz, bool single_float, bool few, bool levels_inner,
+                                uint64_t items, uint64_t cus) {
+    if (nz > 96) return !single_float && items <= (levels_inner ? cus / 2 : 2 * cus);
+    return few && (!levels_inner || items <= cus);
+}
+
+// `shape` with at most `waves` of them on a CU.
+inline RegShape reg_limit(RegShape shape, int waves, size_t lds) {
+    if (waves < shape.per_cu) {
+        shape.per_cu = waves;
+        shape.lds_bytes = std::max(shape.lds_bytes, lds / size_t(waves) / kLdsGranule * kLdsGranule);
+    }
+    return shape;
+}
+
+// The kinds of columns in a batch, and whether the subdomains with columns of one
+// kind, `groups` together, go to the register columns rather than to the
 // warp-specialised solver, whose workgroups take several groups one after the
-// other.  One step of n times 128x128 columns, in us, register columns / that one:
-//   one wave a CU, 268 levels    n = 6 411 / 498, 8 549 / 526, 10 686 / 550, 14 962 / 600
-//   two, 230 levels              n = 24 883 / 1000, 32 1169 / 1084, 40 1450 / 1545, 64 2332 / 2180
-//   two, 190 levels              n = 32 963 / 897, 48 1434 / 1345, 64 1914 / 1780
-inline bool batch_reg_default(int per_cu, uint64_t groups, uint64_t cus) {
-    return per_cu > 2 || groups <= (per_cu == 2 ? 48 : 7) * cus;
+// other.  One step of n subdomains, in us, register columns / that one:
+//   float32 arithmetic, one wave a CU, 128x128x268: n = 6 411 / 498, 8 549 / 526, 10 686 / 550,
+//   14 962 / 600
+//   two, 128x128x230: n = 24 883 / 1000, 32 1169 / 1084, 40 1450 / 1545, 64 2332 / 2180; x190:
+//   32 963 / 897, 48 1434 / 1345, 64 1914 / 1780
+//   contiguous levels, FP64: 16 64x64x80 771 / 1125, 8 128x100x140 2440 / 1673, 8 200x200x12 772 / 514
+//   rows beside, FP64: 8 200x180x40 1381 / 1557, 8 200x200x12 563 / 505, 6 300x300x80 5291 / 5031
+enum BatchColumns { kBatchColumns, kBatchTall1, kBatchTall2, kBatchLevels, kBatchRows, kBatchColumnKinds };
+
+inline BatchColumns batch_columns(int64_t si, int64_t sj, int64_t sk, bool float_arithmetic, int per_cu) {
+    if (si != 1) return sk < si && sk < sj ? kBatchLevels : kBatchRows;
+    if (!float_arithmetic || per_cu > 2) return kBatchColumns;
+    return per_cu == 2 ? kBatchTall2 : kBatchTall1;
+}
+
+inline bool batch_reg_default(BatchColumns kind, uint64_t groups, uint64_t cus) {
+    constexpr uint64_t kMost[kBatchColumnKinds] = {0, 7, 48, 4, 18};  // groups a CU
+    return kind == kBatchColumns || groups <= kMost[kind] * cus;
 }
 
 template <typename T, typename C, int NR, int PF, int AUX, bool POS>

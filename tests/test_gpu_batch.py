@@ -150,6 +150,29 @@ def test_batch_tall_float32_columns_take_both_solvers(gpu):
         sub.free()
 
 
+@pytest.mark.parametrize("storage", [np.float64, np.float32])
+def test_batch_strided_layouts_take_both_solvers(gpu, storage):
+    """Subdomains without unit i stride beside others: many columns of contiguous
+    levels on the warp-specialised solver, the rest on register columns."""
+    from stencil_benchmarks_amd import batch
+
+    # 1093 column groups with contiguous levels
+    shapes = [((280, 230, 12), (0, 1, 2)), ((60, 66, 20), (0, 1, 2)), ((70, 37, 9), (2, 1, 0)),
+              ((33, 66, 17), (0, 2, 1))]
+    rng = np.random.default_rng(3)
+    subs, hosts = [], []
+    for domain, layout in shapes:
+        sub = batch.Subdomain(domain, (3, 3, 3), storage, fill=False, layout=layout)
+        hosts.append(_host_fields(sub, rng))
+        sub.upload(hosts[-1])
+        subs.append(sub)
+    for _ in range(2):
+        batch.step(subs, compute=np.float64)
+        for sub, hf in zip(subs, hosts):
+            oracle_step(hf, sub.domain, sub.halo, np.dtype(storage))
+    _check(subs, hosts, storage)
+
+
 def test_batch_plan_graph_replays_match_eager(gpu):
     from stencil_benchmarks_amd import batch
 

@@ -605,6 +605,24 @@ def test_vadv_padded_rows(gpu, prec, domain, alignment):
         assert np.array_equal(g[outside], fields[w][outside])
 
 
+# layouts without unit i stride, contiguous levels or rows: few and many columns,
+# columns that only register columns hold, and components in launches of their own
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("layout", [(0, 1, 2), (1, 2, 0), (0, 2, 1)])
+@pytest.mark.parametrize("domain,components", [((70, 9, 40), 3), ((330, 101, 33), 1), ((235, 128, 21), 3),
+                                               ((100, 90, 170), 1), ((300, 230, 165), 1),
+                                               ((200, 120, 163), 3)])
+def test_vadv_strided_layouts(gpu, prec, layout, domain, components):
+    halo = (1, 1, 0)
+    names = ("u", "v", "w")[:components]
+    fields = make_fields(domain, halo, _dtype(prec), layout, 0, count=16 if components == 3 else 8,
+                         seed=sum(domain))
+    got = _run_vadv(gpu, fields, [4 * q + 3 for q in range(components)], domain, halo, _prec(gpu, prec),
+                    components == 3, 0)
+    for g, e in zip(got, _vadv_expected(fields, domain, halo, prec, names)):
+        assert np.array_equal(g[inner(domain, halo)], e, equal_nan=True)
+
+
 # pivots at zero and past both ends of the exponent range that the recurrence's
 # reciprocal covers without a division: the register solver gives what the
 # solver that divides at every level gives, infinities and NaN included

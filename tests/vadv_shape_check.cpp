@@ -99,6 +99,36 @@ static int check_tall_columns() {
     return 0;
 }
 
+// Fields without unit i stride.
+static int check_strided() {
+    const struct { int64_t nz; bool single, few, levels; uint64_t items; bool own; } cases[] = {
+        {96, true, true, true, 256, true},     {96, true, true, true, 257, false},
+        {96, true, true, false, 3072, true},   {40, false, false, false, 513, false},
+        {97, false, false, true, 128, true},   {97, false, false, true, 129, false},
+        {97, false, false, false, 512, true},  {97, false, false, false, 513, false},
+        {97, true, false, true, 1, false},     {200, true, false, false, 1, false},
+    };
+    for (const auto &c : cases)
+        if (sb::reg_default_strided(c.nz, c.single, c.few, c.levels, c.items, kCus) != c.own) {
+            std::printf("strided nz %lld: few %d, levels %d, %llu items\n", (long long)c.nz, int(c.few),
+                        int(c.levels), (unsigned long long)c.items);
+            return 1;
+        }
+    for (int64_t nz : {30, 90, 201})
+        for (int waves : {1, 2, 3, 4}) {
+            const sb::RegShape s = sb::reg_shape<double, double>(nz, kLds, 1);
+            const sb::RegShape l = sb::reg_limit(s, waves, kLds);
+            const size_t taken = (l.lds_bytes + 1279) / 1280 * 1280;
+            if (l.build != s.build || l.lds_bytes < s.lds_bytes || l.per_cu > waves || l.per_cu < 1 ||
+                size_t(l.per_cu) * taken > kLds || (waves < s.per_cu && size_t(waves + 1) * taken <= kLds)) {
+                std::printf("limit of %d waves, nz %lld: %d of %zu bytes\n", waves, (long long)nz, l.per_cu,
+                            l.lds_bytes);
+                return 1;
+            }
+        }
+    return 0;
+}
+
 // The same in a batch, whose subdomains count together.
 static int check_batched_columns() {
     const struct { int64_t nz, groups; bool own; } cases[] = {
@@ -109,9 +139,25 @@ static int check_batched_columns() {
     };
     for (const auto &c : cases) {
         const int per_cu = sb::reg_shape<float, float>(c.nz, kLds, 4).per_cu;
-        if (per_cu == 0 || sb::batch_reg_default(per_cu, uint64_t(c.groups), kCus) != c.own) {
+        const sb::BatchColumns kind = sb::batch_columns(1, 100, 10000, true, per_cu);
+        if (per_cu == 0 || sb::batch_reg_default(kind, uint64_t(c.groups), kCus) != c.own) {
             std::printf("batch of float32 nz %lld, %lld groups: %d waves a CU\n", (long long)c.nz,
                         (long long)c.groups, per_cu);
+            return 1;
+        }
+    }
+    // i, j and k stride: unit i stride, contiguous levels, contiguous rows
+    const struct { int64_t si, sj, sk; sb::BatchColumns kind; uint64_t most; } kinds[] = {
+        {1, 100, 10000, sb::kBatchColumns, 1000000}, {10000, 100, 1, sb::kBatchLevels, 4 * 256},
+        {100, 10000, 1, sb::kBatchLevels, 4 * 256},  {10000, 1, 100, sb::kBatchRows, 18 * 256},
+        {100, 1, 10000, sb::kBatchRows, 18 * 256},
+    };
+    for (const auto &c : kinds) {
+        const sb::BatchColumns kind = sb::batch_columns(c.si, c.sj, c.sk, false, 2);
+        if (kind != c.kind || !sb::batch_reg_default(kind, c.most, kCus) ||
+            (kind != sb::kBatchColumns && sb::batch_reg_default(kind, c.most + 1, kCus))) {
+            std::printf("batch of strides %lld %lld %lld: kind %d\n", (long long)c.si, (long long)c.sj,
+                        (long long)c.sk, int(kind));
             return 1;
         }
     }
@@ -141,7 +187,8 @@ int main() {
     if (check_waves<double, double>("FP64") || check_waves<float, double>("float32 storage") ||
         check_waves<float, float>("float32"))
         return 1;
-    if (check_remap() || check_short_columns() || check_tall_columns() || check_batched_columns())
+    if (check_remap() || check_short_columns() || check_tall_columns() || check_strided() ||
+        check_batched_columns())
         return 1;
     std::printf("ok\n");
     return 0;
