@@ -249,7 +249,7 @@ def bench_batched(compute_dtype, storage_dtype, repeats=2):
     return {"seconds": seconds, "gbs": nbytes / seconds / 1e9,
             "gridpoint_steps_per_s": points / seconds, "subdomains": len(subs),
             "steps": 10, "points_per_step": points // 10,
-            "autotuned": {"hdiff": tuned.hdiff, "vadv": tuned.vadv,
+            "autotuned": {"hdiff": tuned.hdiff, "vadv": tuned.vadv, "defaults": tuned.defaults,
                           "from_cache": tuned.from_cache, "candidates": len(tuned.trials)}}
 
 
@@ -338,7 +338,8 @@ def bench_serving(count=160, load=0.8):
         "speedup_vs_plain_f64": capacity / (count / plain_s),
         # continuous batching alone: the same precision served one request at a time
         "speedup_vs_plain_same_precision": capacity / (count / plain32_s),
-        "autotuned": {"hdiff": tuned.hdiff, "vadv": tuned.vadv, "from_cache": tuned.from_cache},
+        "autotuned": {"hdiff": tuned.hdiff, "vadv": tuned.vadv, "defaults": tuned.defaults,
+                      "from_cache": tuned.from_cache},
     })
     return out
 

@@ -10,15 +10,17 @@ options on the device and keeps the fastest per device and workload:
   groups per item, 4 or 8 levels per barrier step and 4 or 5 waves, or the
   single-wave pipeline at prefetch depth 4/8),
   chosen by coordinate descent (hdiff with the first vadv, then vadv with
-  the chosen hdiff), then compared with no options at all, each candidate
-  timed over whole steps on scratch subdomains of the workload's geometry
-  (user fields are never advanced);
+  the chosen hdiff), each candidate timed over whole steps on scratch
+  subdomains of the workload's geometry (user fields are never advanced);
 * plain horizontal diffusion (`tune_hdiff`): tile height x k-planes x cache
   hints over one domain;
 * plain vertical advection (`tune_vadv`): the warp-specialised solver at 4 or
   8 levels per barrier step, the single-wave pipeline at prefetch depth
   4/8/16 or register columns, each with plain or non-temporal streamed loads,
   over one domain.
+
+What is found is compared with no options at all, whose kernels (the LDS-DMA
+tile and the register columns) the spaces do not hold for every workload.
 
 Every candidate computes the same arithmetic (the tests check that results
 are bit-identical across launch options), so tuning changes speed only.
@@ -231,7 +233,8 @@ def tune_hdiff(domain, storage, compute=None, halo=(3, 3, 3), cache=None, repeat
     cache = cache if cache is not None else TuneCache()
     hit = None if force else cache.get(key)
     if hit:
-        return TuneResult(key, hit["hdiff"], {}, hit["seconds"], True)
+        return TuneResult(key, hit["hdiff"], {}, hit["seconds"], True,
+                          defaults=hit.get("defaults", False))
     shape = tuple(d + 2 * h for d, h in zip(domain, halo))
     template = array.alloc_array(shape, storage, (2, 1, 0), 64, halo)
     strides = [s // storage.itemsize for s in template.strides]
@@ -267,10 +270,13 @@ def tune_hdiff(domain, storage, compute=None, halo=(3, 3, 3), cache=None, repeat
             # (the tuning fields have 64-byte aligned rows, as FP64 needs)
             space = space + tuple({"variant": 2, "by": by} for by in (8, 16) if domain[1] % by == 0)
         h, _, seconds, trials = descend(space, (), measure, {})
+        default = measure({}, {})
+        defaults, seconds = default <= seconds, min(seconds, default)
     finally:
         fields[0].free()
-    cache.put(key, {"hdiff": h, "vadv": {}, "seconds": seconds, "trials": len(trials)})
-    return TuneResult(key, h, {}, seconds, False, trials)
+    cache.put(key, {"hdiff": h, "vadv": {}, "seconds": seconds, "trials": len(trials),
+                    "defaults": defaults})
+    return TuneResult(key, h, {}, seconds, False, trials, defaults)
 
 
 def tune_vadv(domain, storage, compute=None, halo=(3, 3, 3), cache=None, repeats=3,
@@ -290,7 +296,8 @@ def tune_vadv(domain, storage, compute=None, halo=(3, 3, 3), cache=None, repeats
     cache = cache if cache is not None else TuneCache()
     hit = None if force else cache.get(key)
     if hit:
-        return TuneResult(key, {}, hit["vadv"], hit["seconds"], True)
+        return TuneResult(key, {}, hit["vadv"], hit["seconds"], True,
+                          defaults=hit.get("defaults", False))
     shape = tuple(d + 2 * h for d, h in zip(domain, halo))
     template = array.alloc_array(shape, storage, (2, 1, 0), 64, halo)
     strides = [s // storage.itemsize for s in template.strides]
@@ -323,9 +330,12 @@ def tune_vadv(domain, storage, compute=None, halo=(3, 3, 3), cache=None, repeats
         for _ in range(warmup):
             native.call("sb_vadv", code, 0, pointers, geom, native.launch_options(), None)
         _, v, seconds, trials = descend(({},), PLAIN_VADV_SPACE, measure, PLAIN_VADV_SPACE[0])
+        default = measure({}, {})
+        defaults, seconds = default <= seconds, min(seconds, default)
     finally:
         fields[0].free()
     if seconds == float("inf"):
         raise ExecutionError(f"no vadv solver takes the domain {tuple(domain)}")
-    cache.put(key, {"hdiff": {}, "vadv": v, "seconds": seconds, "trials": len(trials)})
-    return TuneResult(key, {}, v, seconds, False, trials)
+    cache.put(key, {"hdiff": {}, "vadv": v, "seconds": seconds, "trials": len(trials),
+                    "defaults": defaults})
+    return TuneResult(key, {}, v, seconds, False, trials, defaults)

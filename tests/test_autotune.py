@@ -9,6 +9,7 @@ files tolerated); workload keys depend on the shapes, not their order.
 import json
 
 import numpy as np
+import pytest
 
 from stencil_benchmarks_amd import autotune
 
@@ -65,3 +66,53 @@ def test_spaces_hold_only_built_combinations():
 def test_launch_from_sets_fields():
     launch = autotune.launch_from({"variant": 4, "by": 16})
     assert (launch.variant, launch.by, launch.bz) == (4, 16, 0)
+
+
+class _NoDevice:
+    base = span = 8
+
+    def pointer(self):
+        return self.base
+
+    def free(self):
+        pass
+
+
+def _tune_without_device(monkeypatch, tmp_path, name, fastest):
+    """The tuner over calls that take 1 s with the options `fastest` accepts, else 2 s."""
+    from stencil_benchmarks_amd import device, native
+
+    def call(function, *arguments):
+        if function == "sb_" + name and arguments[-1] is not None:
+            arguments[-1]._obj.value = 1.0 if fastest(arguments[-2]) else 2.0
+
+    monkeypatch.setattr(autotune, "device_key", lambda: "device")
+    monkeypatch.setattr(native, "call", call)
+    monkeypatch.setattr(device.DeviceField, "group",
+                        lambda shape, dtype, strides, count, halo: [_NoDevice()] * count)
+    tune = {"hdiff": autotune.tune_hdiff, "vadv": autotune.tune_vadv}[name]
+    return lambda: tune((20, 10, 8), "float32", repeats=1,
+                        cache=autotune.TuneCache(tmp_path / "tune.json"))
+
+
+@pytest.mark.parametrize("name", ["hdiff", "vadv"])
+def test_plain_tuners_return_no_options_where_those_are_fastest(monkeypatch, tmp_path, name):
+    def fields(options):
+        return [getattr(options, f) for f in ("variant", "bx", "by", "bz", "unroll")]
+
+    tune = _tune_without_device(monkeypatch, tmp_path, name,
+                                lambda options: not any(fields(options)))
+    for from_cache in (False, True):
+        tuned = tune()
+        assert tuned.defaults and tuned.seconds == 1.0 and tuned.from_cache == from_cache
+        assert not any(fields(getattr(tuned, name + "_options")))
+
+
+@pytest.mark.parametrize("name", ["hdiff", "vadv"])
+def test_plain_tuners_return_the_fastest_options(monkeypatch, tmp_path, name):
+    tune = _tune_without_device(monkeypatch, tmp_path, name,
+                                lambda options: options.variant > 0 and options.unroll == 4)
+    for from_cache in (False, True):
+        tuned = tune()
+        assert not tuned.defaults and tuned.seconds == 1.0 and tuned.from_cache == from_cache
+        assert getattr(tuned, name + "_options").unroll == 4
