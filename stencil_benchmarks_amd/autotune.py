@@ -119,6 +119,11 @@ def launch_from(options):
     return launch
 
 
+# Of the kernels and the spaces searched, part of every cache key: raised when
+# either changes, so that choices made between other kernels are made anew.
+REVISION = 2
+
+
 def device_key():
     info = native.device_info()
     return f"{info['name']}|{info['arch']}|{info['compute_units']}"
@@ -127,7 +132,7 @@ def device_key():
 def workload_key(kind, domains, storage, compute, halo=(3, 3, 3)):
     shapes = json.dumps(sorted(tuple(int(d) for d in dom) for dom in domains))
     digest = hashlib.sha1(shapes.encode()).hexdigest()[:16]
-    return (f"{kind}|{np.dtype(storage).name}|{np.dtype(compute).name}|halo={tuple(halo)}|"
+    return (f"r{REVISION}|{kind}|{np.dtype(storage).name}|{np.dtype(compute).name}|halo={tuple(halo)}|"
             f"n={len(domains)}|{digest}")
 
 

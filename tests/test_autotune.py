@@ -116,3 +116,16 @@ def test_plain_tuners_return_the_fastest_options(monkeypatch, tmp_path, name):
         tuned = tune()
         assert not tuned.defaults and tuned.seconds == 1.0 and tuned.from_cache == from_cache
         assert getattr(tuned, name + "_options").unroll == 4
+
+
+@pytest.mark.parametrize("name", ["hdiff", "vadv"])
+def test_choices_between_older_kernels_are_made_anew(monkeypatch, tmp_path, name):
+    tune = _tune_without_device(monkeypatch, tmp_path, name, lambda options: options.variant == 1)
+    # the key of an entry written before keys named a revision
+    key = autotune.workload_key(name, [(20, 10, 8)], "float32", "float32", (3, 3, 3))
+    old = "device|" + key[key.index(name):]
+    autotune.TuneCache(tmp_path / "tune.json").put(
+        old, {"hdiff": {"variant": 3}, "vadv": {"variant": 3}, "seconds": 0.1, "trials": 60})
+    assert not tune().from_cache and tune().from_cache
+    monkeypatch.setattr(autotune, "REVISION", autotune.REVISION + 1)
+    assert not tune().from_cache
