@@ -130,7 +130,7 @@ struct RegBuilds<double, double> {
 };
 template <>
 struct RegBuilds<float, double> {
-    static constexpr RegLevels of[] = {{0, 4, false}, {24, 3, false}, {48, 2, false}, {80, 1, false}, {112, 1, false}, {16, 3, true}, {40, 2, true}, {88, 1, true}};
+    static constexpr RegLevels of[] = {{0, 4, false}, {24, 3, false}, {48, 2, false}, {112, 1, false}, {16, 3, true}, {40, 2, true}, {88, 1, true}};
 };
 template <>
 struct RegBuilds<float, float> {

@@ -220,6 +220,20 @@ def test_laplacian_default_tile_rows(gpu, domain):
     _check_halo(got, domain, halo)
 
 
+# the tile rows that the LDS-DMA tile chooses itself (16 where ny allows, else
+# 8): asked for by number, and as the default of fields beyond 256 MB
+@pytest.mark.parametrize("domain,variant", [((64, 16, 3), 3), ((64, 24, 3), 3), ((128, 8, 2), 3),
+                                            ((1024, 528, 33), 0), ((1024, 520, 33), 0)])
+def test_laplacian_lds_dma_tile_rows(gpu, domain, variant):
+    halo = (1, 1, 1)
+    inp, = make_fields(domain, halo, np.float64, (2, 1, 0), 0, seed=sum(domain))
+    out = _with_sentinel(make_fields(domain, halo, np.float64, (2, 1, 0), 0)[0])
+    got, = _run(gpu, "sb_laplacian", [inp, out], [1], domain, halo, gpu.SB_F64, 1, 1, 0,
+                launch=gpu.launch_options(variant=variant))
+    assert np.array_equal(got[inner(domain, halo)], oracle.laplacian(inp, (1, 1, 0), domain, halo))
+    _check_halo(got, domain, halo)
+
+
 @pytest.mark.parametrize("domain,prec,mask,tile,match", [
     ((70, 16, 2), "f64", (1, 1, 0), 0, "multiple of 64"),
     ((64, 12, 2), "f64", (1, 1, 0), 0, "multiple of 8"),
@@ -554,6 +568,19 @@ def test_vadv_register_builds_many_columns(gpu, prec, nz):
     got, = _run_vadv(gpu, fields, [3], domain, halo, _prec(gpu, prec), False, 0)
     expected = _expected(lambda *f: oracle.vadv(*f, domain, halo), fields[:5], prec)
     assert np.array_equal(got[inner(domain, halo)], expected)
+
+
+# the builds that keep no pos: 24 and 112 register levels of float32 storage at
+# the edges of their ranges, 24 of FP64
+@pytest.mark.parametrize("prec", PRECISIONS)
+@pytest.mark.parametrize("domain", [(601, 320, 28), (601, 320, 31), (601, 320, 42), (601, 140, 122),
+                                    (601, 140, 193)])
+def test_vadv_register_builds_without_pos(gpu, prec, domain):
+    halo = (1, 1, 0)
+    fields = make_fields(domain, halo, _dtype(prec), count=8, seed=sum(domain))
+    got, = _run_vadv(gpu, fields, [3], domain, halo, _prec(gpu, prec), False, 0)
+    expected = _expected(lambda *f: oracle.vadv(*f, domain, halo), fields[:5], prec)
+    assert np.array_equal(got[inner(domain, halo)], expected, equal_nan=True)
 
 
 # short columns beyond what a device holds at once, with every cache hint

@@ -1,6 +1,7 @@
 // Host-side check of the launch rules of the register-column vadv
 // (stencil_benchmarks_amd/csrc/vadv_regs.h, sb_internal.h).  Exits non-zero on
 // the first rule that does not hold.
+#include <array>
 #include <cstdio>
 #include <vector>
 
@@ -164,6 +165,29 @@ static int check_batched_columns() {
     return 0;
 }
 
+// Every build is the choice for some columns, and the choices that the device
+// tests name (tests/test_gpu_parity.py).
+template <typename T, typename C>
+static int check_builds(const char *name, std::initializer_list<std::array<int, 4>> named) {
+    std::vector<char> seen(std::size(sb::RegBuilds<T, C>::of), 0);
+    for (int64_t nz = 2; nz <= sb::reg_max_levels<C>(); ++nz)
+        for (uint64_t need = 1; need <= 20; ++need) seen[size_t(sb::reg_shape<T, C>(nz, kLds, need).build)] = 1;
+    for (size_t b = 0; b < seen.size(); ++b)
+        if (!seen[b]) {
+            std::printf("%s: the build of %d register levels is never chosen\n", name,
+                        sb::RegBuilds<T, C>::of[b].nr);
+            return 1;
+        }
+    for (const auto &[nz, items, nr, pos] : named) {
+        const sb::RegLevels &of = sb::RegBuilds<T, C>::of[shape_of<T, C>(nz, uint64_t(items)).build];
+        if (of.nr != nr || of.pos != bool(pos)) {
+            std::printf("%s nz %d, %d items: build of %d register levels\n", name, nz, items, of.nr);
+            return 1;
+        }
+    }
+    return 0;
+}
+
 // The waves counted on a CU fit its LDS, which is allocated in granules of
 // 1280 bytes, and its registers.
 template <typename T, typename C>
@@ -186,6 +210,16 @@ static int check_waves(const char *name) {
 int main() {
     if (check_waves<double, double>("FP64") || check_waves<float, double>("float32 storage") ||
         check_waves<float, float>("float32"))
+        return 1;
+    // 601 x 140 columns (1315 items) and 601 x 320 (3005)
+    if (check_builds<double, double>("FP64", {{26, 1315, 16, 1}, {42, 1315, 24, 0}, {66, 1315, 40, 0},
+                                              {98, 1315, 64, 0}, {115, 1315, 96, 0}, {30, 3005, 16, 1},
+                                              {31, 3005, 24, 0}, {42, 3005, 24, 0}}) ||
+        check_builds<float, double>("float32 storage", {{26, 1315, 16, 1}, {42, 1315, 40, 1},
+                                                        {66, 1315, 48, 0}, {98, 1315, 88, 1},
+                                                        {122, 1315, 112, 0}, {193, 1315, 112, 0},
+                                                        {30, 3005, 24, 0}, {42, 3005, 24, 0}}) ||
+        check_builds<float, float>("float32", {{42, 1315, 40, 0}, {98, 1315, 80, 0}}))
         return 1;
     if (check_remap() || check_short_columns() || check_tall_columns() || check_strided() ||
         check_batched_columns())
