@@ -170,8 +170,9 @@ int sb_laplacian(int prec, int along_x, int along_y, int along_z,
  * templates/horizontal_diffusion_*.j2); semantics of base.py:276-311.
  * Requires hi, hj >= 2.  Variants: 0 default (the kernel of 2, also on
  * partial tiles and any alignment, where si = 1, 0 < sj with a row pitch
- * below 16 MiB and no tile option is given; else 1 where positive i and j strides and a k-plane below 4 GiB let the tile use
- * 32-bit plane offsets, else 3), 1 LDS-staged tile
+ * below 16 MiB and no tile option is given; else 1 where positive i and j
+ * strides and a k-plane below 4 GiB let the tile use 32-bit plane offsets,
+ * else 3), 1 LDS-staged tile
  * (launch->by = tile rows 8/16/32, ->bz = k-planes per workgroup 1..16, 0
  * measured default; ->unroll 0 = default (non-temporal coeff loads), else
  * 4 | flags with bit 0 non-temporal out stores, bit 1 non-temporal coeff
@@ -194,9 +195,11 @@ int sb_hdiff(int prec, const void *inp, const void *coeff, void *out,
  * *tensstage fields are written; ccol, dcol and datacol are never touched
  * (the Thomas coefficients stay on chip, or in a library-owned scratch for
  * variant 2).  Requires hi >= 1 (all components: hj >= 1 too).  Variants:
- * 0 default (5 up to nz = 201 with FP64 arithmetic, 401 with float32; above
- * that, or with fields of 4 GiB and more or negative strides, 1 where the
- * LDS holds the column, else 2),
+ * 0 default (5 up to nz = 201 with FP64 arithmetic, 401 with float32, but 3 or
+ * 4 for many short FP64 columns, for tall columns of float32 arithmetic, for
+ * many columns without unit i stride, and for options that only those have;
+ * above that, or with fields of 4 GiB and more or negative strides, 1 where
+ * the LDS holds the column, else 2),
  * 1 one wave per
  * group with the coefficients in LDS, 2 coefficients in a global FP64
  * scratch, 3 single-wave pipeline fusing the forward sweep of one group with
@@ -206,9 +209,9 @@ int sb_hdiff(int prec, const void *inp, const void *coeff, void *out,
  * component with the coefficients of the highest levels (up to 112) in
  * registers and the rest in LDS (nz <= 201 with FP64 arithmetic).
  * launch->bz: bit 0
- * non-temporal streamed loads (variant 5: 0 the library's choice), bit 2 (variant 4, SB_F32_F64 only) reciprocal
- * estimate plus Newton steps instead of the correctly rounded division; 0
- * and -1 plain loads. */
+ * non-temporal streamed loads (variant 5: 0 the library's choice), bit 2
+ * (variant 4, SB_F32_F64 only) reciprocal estimate plus Newton steps instead
+ * of the correctly rounded division; 0 and -1 plain loads. */
 int sb_vadv(int prec, int all_components, void *const *fields,
             const sb_geom *g, const sb_launch *l, double *seconds);
 
@@ -276,7 +279,9 @@ int sb_stream_check(int prec, const void *x, size_t n, double expected,
  * ->unroll = tile height / planes per item / non-temporal flags of the
  * register-staged tile, drawn from work queues; vadv_launch all zero = the
  * register-column solver of sb_vadv's variant 5, one launch per register
- * build the columns need; ->variant = 4 (also 0 with any option of it:
+ * build the columns need, beside it the one of variant 4 for many tall columns
+ * of float32 arithmetic or without unit i stride; ->variant = 4 (also 0 with
+ * any option of it:
  * warp-specialised solver, items of ->by column groups, 0 = 16,
  * drawn from per-XCD device work queues in order of decreasing cost, ->unroll
  * = levels per barrier step 4 or 8, 0 = 4, ->bx = waves per workgroup 4 or
@@ -296,9 +301,10 @@ typedef struct sb_subdomain {
 /* One timestep for `count` subdomains: one hdiff launch (with hdiff options a
  * persistent one, tiles from per-XCD device work queues; a counter reset
  * precedes launches that use queues) and the vadv launches (by
- * default one to five, a workgroup per column group; warp-specialised: one or
+ * default one to four, a workgroup per column group; warp-specialised: one or
  * two persistent ones, column-group items from per-XCD device work queues,
- * one launch per LDS class; variant 3: items from one device counter).  Does not flip the parities; the caller does. */
+ * one launch per LDS class; variant 3: items from one device counter).  Does
+ * not flip the parities; the caller does. */
 int sb_batch_step(int prec, const sb_subdomain *subs, int count, const sb_launch *hdiff_launch,
                   const sb_launch *vadv_launch, double *seconds);
 /* A fixed set of subdomains advanced `steps` steps per run: device tables

@@ -4,7 +4,9 @@ One lane per (i, j) column with contiguous i, forward sweep and fused
 backward substitution in one kernel (csrc/vadv.hip).  ``Fused`` picks the
 solver: one wave per 64-column group and component, with the highest
 levels' Thomas coefficients in registers and the rest in LDS (nz <= 201 in
-FP64 arithmetic), and a global FP64 scratch beyond.  ``LdsColumn``,
+FP64 arithmetic), one of the others for many short FP64 columns, tall columns
+of float32 arithmetic and many columns without unit i stride, and a global
+FP64 scratch beyond.  ``LdsColumn``,
 ``GlobalScratch``, ``Pipelined``, ``WarpSpecialised`` (four waves per group)
 and ``RegisterColumns`` pin one solver (``WarpSpecialised`` with
 ``levels_per_step`` 4 or 8 per workgroup barrier).  Arithmetic follows

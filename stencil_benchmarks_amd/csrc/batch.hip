@@ -9,7 +9,9 @@
 //
 // Without launch options a step is one hdiff launch, a workgroup of the
 // LDS-DMA tile per tile and plane, and one vadv launch per register build, a
-// wave per column group, in plain grids that the dispatcher balances.
+// wave per column group, in plain grids that the dispatcher balances; kinds of
+// columns that this is slower for go the way of variant 4 below instead, if they
+// are many (ws_subdomains).
 //
 // With options a sequence of steps starts with one counter-reset kernel; each
 // step is one persistent hdiff launch and one or two persistent vadv launches
@@ -417,7 +419,7 @@ struct Plan {
     bool dma_hint = false;
     std::vector<int32_t> host_dma;
     int32_t *dma = nullptr;
-    // register-column vadv (the default): one launch per class
+    // register-column vadv (the default, but see ws_subdomains): one launch per class
     struct RegClass {
         int build = 0;
         size_t lds_bytes = 0;           // of its tallest column

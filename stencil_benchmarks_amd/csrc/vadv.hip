@@ -24,7 +24,8 @@
 // runs the backward substitution from that storage in the same kernel.
 //
 // The default is variant 5 (vadv_regs.h): one wave per group, the highest
-// levels' (c', d') in registers, the rest in LDS.
+// levels' (c', d') in registers, the rest in LDS; 3 or 4 where reg_default and
+// reg_default_strided there say so.
 //
 // Storage of (c', d'): variant 1 keeps it in LDS ((nz-1) x 64 x 16 bytes
 // for FP64 arithmetic, so nz <= 160 fits one workgroup); variant 2 keeps it
